@@ -394,6 +394,25 @@ int fl_attention_fwd(const fl_attn_params* p, fl_stream_t stream) {
   a.scale = static_cast<float>(p->softmax_scale);
   a.scale_log2 = static_cast<float>(p->softmax_scale * 1.4426950408889634);
   a.q_blocks = static_cast<int>(q_blocks);
+  // The query heads of a KV head share its K and V tiles, so their rows are packed (launch.hpp): a
+  // block then covers 1 / group of the positions, which leaves less of it past a causal diagonal and
+  // past the last row. (B, H, H_kv, S, D) causal, one box, before / after: (16, 32, 8, 700, 128) 128 /
+  // 104 us, (4, 16, 2, 1078, 64) 41 / 23, (8, 24, 8, 28, 64) 5.7 / 4.4, (1, 32, 8, 8192, 128) 439 / 437.
+  // Not where the packed grid is smaller than half the CUs: there the time is that of one
+  // workgroup's rows, and separate heads spread them over more CUs ((1, 64, 8), 18 new rows after
+  // 1,194 keys, D = 128: 23.0 us separate, 25.0 packed). Nor past pack_position's range.
+  const int64_t packed_rows = static_cast<int64_t>(p->seqlen_q) * a.group;
+  const int64_t packed_grid = (packed_rows + fl::kPrefillBlockM - 1) / fl::kPrefillBlockM *
+                              p->batch * p->heads_kv;
+  a.pack = packed_rows < (int64_t{1} << 30) && packed_grid >= 128 ? a.group : 1;
+  a.work_heads = p->heads / a.pack;
+  a.rows = p->seqlen_q * a.pack;
+  // Division by a constant d < 2^31 of any n < 2^31 as a multiplication: with 2^l >= d,
+  // m = floor(2^(31 + l) / d) + 1 exceeds 2^(31 + l) / d by at most 1, so n m / 2^(31 + l) exceeds
+  // n / d by less than 2^31 / 2^(31 + l) <= 1 / d.
+  a.pack_shift = 31;
+  while ((int64_t{1} << (a.pack_shift - 31)) < a.pack) ++a.pack_shift;
+  a.pack_mul = static_cast<uint32_t>((uint64_t{1} << a.pack_shift) / static_cast<uint32_t>(a.pack) + 1);
 
   const fl::DType dt = p->dtype == FL_DTYPE_BF16 ? fl::DType::bf16 : fl::DType::f16;
   const hipError_t err = fl::launch_prefill(a, dt, p->head_dim, static_cast<hipStream_t>(stream));

@@ -25,8 +25,21 @@ struct PrefillArgs {
   int batch, seqlen_q, seqlen_k, heads, heads_kv, group, causal_offset, causal;
   float scale;       // softmax scale, natural-log domain (used for the LSE)
   float scale_log2;  // scale * log2(e): probabilities are 2^(s * scale_log2 - ref)
-  int q_blocks;      // ceil(S_q / rows per workgroup)
+  int q_blocks;      // ceil(rows / rows per workgroup)
+  // Packed query rows: one work head is `pack` adjacent query heads of one KV head (its whole group,
+  // or 1), and its rows run position by position, row r being position r / pack of head r % pack, so
+  // that a block of rows covers 1 / pack of the positions. rows = S_q pack, work_heads = H / pack;
+  // r / pack is (r pack_mul) >> pack_shift for every r in [0, 2^31).
+  int pack, work_heads, rows;
+  uint32_t pack_mul;
+  int pack_shift;
+  // Causal ping-pong calls: 1 = a workgroup runs a heavy and a light block of rows, 0 = one block per
+  // workgroup, the heaviest of every work head first.
+  int paired;
 };
+__host__ __device__ __forceinline__ int pack_position(const PrefillArgs& a, int row) {
+  return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(row)) * a.pack_mul) >> a.pack_shift);
+}
 
 // Decode problem. q [B, H, D], caches [B, S_max, H_kv, D], o [B, H, D], lse [B, H].
 struct DecodeArgs {

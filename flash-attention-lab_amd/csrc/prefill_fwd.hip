@@ -76,26 +76,29 @@ __global__ void __launch_bounds__(kThreads)
   const int bh = work / a.q_blocks;
   int qb = work - bh * a.q_blocks;
   if (a.causal) qb = a.q_blocks - 1 - qb;
-  const int b = bh / a.heads;
-  const int h = bh - b * a.heads;
+  const int b = bh / a.work_heads;
+  const int h = (bh - b * a.work_heads) * a.pack;  // first query head
   const int hkv = h / a.group;
   const int q0 = qb * kBlockM;
   const int row0 = q0 + wave * kRowsPerWave;  // first query row of this wave
   const int my_row = row0 + (lane & 31);      // the query row this lane owns
+  const int my_pos = pack_position(a, my_row);
+  const int my_head = my_row - my_pos * a.pack;  // of the packed heads
 
   const uint16_t* qp = a.q + b * a.q_bs + h * a.q_hs;
   const uint16_t* kp = a.k + b * a.k_bs + hkv * a.k_hs;
   const uint16_t* vp = a.v + b * a.v_bs + hkv * a.v_hs;
 
   int kv_end = a.seqlen_k;
-  if (a.causal) kv_end = min(kv_end, min(q0 + kBlockM, a.seqlen_q) + a.causal_offset);
+  if (a.causal)
+    kv_end = min(kv_end, pack_position(a, min(q0 + kBlockM, a.rows) - 1) + 1 + a.causal_offset);
   const int num_tiles = kv_end > 0 ? (kv_end + kBlockN - 1) / kBlockN : 0;
 
   // Q^T fragments, the B operand of every S^T step: row my_row, dims 16 ks + 8 half .. + 7.
   u32x4 qf[D / 16];
   {
-    const bool ok = my_row < a.seqlen_q;
-    const uint16_t* src = qp + static_cast<int64_t>(ok ? my_row : 0) * a.q_ss + 8 * half;
+    const bool ok = my_row < a.rows;
+    const uint16_t* src = qp + (ok ? my_pos : 0) * a.q_ss + (ok ? my_head : 0) * a.q_hs + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) qf[ks] = ok ? load16(src + 16 * ks) : u32x4{0, 0, 0, 0};
   }
@@ -146,7 +149,10 @@ __global__ void __launch_bounds__(kThreads)
   float l = 0.f;          // this lane's share of the running sum
   const float sl2 = a.scale_log2;
   // Last key my_row may see in the whole problem.
-  const int last_key = a.causal ? min(a.seqlen_k - 1, my_row + a.causal_offset) : a.seqlen_k - 1;
+  const int last_key = a.causal ? min(a.seqlen_k - 1, my_pos + a.causal_offset) : a.seqlen_k - 1;
+  // Keys that the wave's first row, and any of its rows, sees under the causal mask.
+  const int first_limit = pack_position(a, row0) + a.causal_offset;
+  const int wave_limit = pack_position(a, row0 + kRowsPerWave - 1) + a.causal_offset;
 
   // One tile: loads of the next tile into the other slots, then (for a wave that sees any of its
   // keys) scores, softmax and P V from slot kSlot, and a barrier after which the next tile's data
@@ -161,7 +167,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     const int k0 = t * kBlockN;
     // A wave that sees no key of this tile sees none of the later ones either (causal).
-    const bool active = !(a.causal && k0 > row0 + kRowsPerWave - 1 + a.causal_offset);
+    const bool active = !(a.causal && k0 > wave_limit);
     if (active) {
       // S^T = K Q^T, K fragments read kAhead steps ahead of their MFMAs.
       constexpr int kSteps = D / 16;
@@ -200,7 +206,7 @@ __global__ void __launch_bounds__(kThreads)
       // Keys past the end or above the diagonal: only edge and diagonal tiles (wave-uniform
       // branch; the empty asm keeps the compiler from turning it into selects on every tile).
       if ((k0 + kBlockN > a.seqlen_k) ||
-          (a.causal && k0 + kBlockN - 1 > row0 + a.causal_offset)) {
+          (a.causal && k0 + kBlockN - 1 > first_limit)) {
         asm volatile("" ::: "memory");
         // acc_key(j, half) = acc_key(j, 0) + 4 half: fold the lane's part into the limit so every
         // comparison is against a compile-time constant (no per-key registers live in the loop).
@@ -270,8 +276,8 @@ __global__ void __launch_bounds__(kThreads)
   // Epilogue: l over both halves, 1/l (0 for rows that saw no key, which then store zeros).
   const float lt = l + xor_lane(l, 32);
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
-  if (my_row < a.seqlen_q) {
-    uint16_t* orow = a.o + b * a.o_bs + static_cast<int64_t>(my_row) * a.o_ss + h * a.o_hs;
+  if (my_row < a.rows) {
+    uint16_t* orow = a.o + b * a.o_bs + my_pos * a.o_ss + (h + my_head) * a.o_hs;
 #pragma unroll
     for (int nb = 0; nb < D / 32; ++nb) {
 #pragma unroll
@@ -284,7 +290,7 @@ __global__ void __launch_bounds__(kThreads)
     }
     if (half == 0) {
       // l = sum 2^(s scale_log2 - ref), so ln(sum e^(s scale)) = ref ln 2 + ln l.
-      a.lse[(static_cast<int64_t>(b) * a.heads + h) * a.seqlen_q + my_row] =
+      a.lse[(static_cast<int64_t>(b) * a.heads + h + my_head) * a.seqlen_q + my_pos] =
           lt > 0.f ? ref * kLn2 + logf(lt) : -INFINITY;
     }
   }
@@ -347,8 +353,9 @@ __global__ void __launch_bounds__(64) mfma_tile_test_kernel(const uint16_t* a, c
 }
 
 template <typename Tag, int D>
-hipError_t launch_typed(const PrefillArgs& args, hipStream_t stream) {
-  const int blocks = args.q_blocks * args.batch * args.heads;
+hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
+  args.q_blocks = (args.rows + kBlockM - 1) / kBlockM;
+  const int blocks = args.q_blocks * args.batch * args.work_heads;
   hipLaunchKernelGGL((prefill_fwd_kernel<Tag, D>), dim3(blocks), dim3(kThreads), 0, stream, args);
   return hipGetLastError();
 }
@@ -378,13 +385,13 @@ static_assert(kPrefillBlockN == prefill::kBlockN, "host and kernel tile widths d
 // this with its own workgroup threshold (so tests can route one shape to either kernel).
 bool prefill_on_pingpong(const PrefillArgs& args, int head_dim) {
   const int rows = prefill_pp_block_rows(head_dim);
-  const int64_t pp_blocks = (args.seqlen_q + rows - 1) / rows;
+  const int64_t pp_blocks = (args.rows + rows - 1) / rows;
   const int64_t pp_items = args.causal ? (pp_blocks + 1) / 2 : pp_blocks;
-  const int64_t workgroups = pp_items * args.batch * args.heads;
+  const int64_t workgroups = pp_items * args.batch * args.work_heads;
   const int v = knob(FL_KNOB_PREFILL_PP_MIN_WG);
   if (v >= 0) return workgroups >= v;
   if (args.causal) return workgroups >= 128;
-  const int64_t padding = pp_blocks * rows - args.seqlen_q;
+  const int64_t padding = pp_blocks * rows - args.rows;
   if (4 * padding > pp_blocks * rows && workgroups > 256) return false;
   return workgroups >= 256;
 }

@@ -40,7 +40,10 @@
 //    issues the same number of loads and the vmcnt accounting is
 //    uniform.
 //  * Work order: XCD-contiguous (batch, head) ranges (workgroups are dealt round-robin over the 8
-//    XCDs, each with its own L2); causal query blocks in heavy/light pairs per workgroup.
+//    XCDs, each with its own L2); causal query blocks in heavy/light pairs per workgroup, or singly,
+//    heaviest first, where pairs would leave much of the last round empty (launch_typed).
+//  * With grouped-query heads the rows of a KV head's query heads are packed position by position
+//    (PrefillArgs::pack), so "row" below is a packed row.
 #include <type_traits>
 
 #include "prefill_pp.hpp"
@@ -90,16 +93,24 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   const uint32_t sel_word = ((lane >> 4) & 1) == ((lane >> 2) & 1) ? E::kOnePair : 0u;
   const u32x4 sum_sel{sel_word, sel_word, sel_word, sel_word};
 
-  // Work item: (batch, head) and query blocks. Non-causal: one block per workgroup. Causal: the
-  // blocks of a (batch, head) go in pairs (q_blocks - 1 - i, i), heavy first, so every workgroup
-  // runs about the same number of tiles (a plain heaviest-first order still leaves a tail of heavy
-  // blocks dealt late) and the light block's K and V are a prefix of the heavy one's.
-  const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const int items_per_bh = a.causal ? (a.q_blocks + 1) / 2 : a.q_blocks;
-  const int bh = work / items_per_bh;
-  const int item = work - bh * items_per_bh;
-  const int b = bh / a.heads;
-  const int h = bh - b * a.heads;
+  // Work item: (batch, head) and query blocks. Non-causal: one block per workgroup. Causal, paired:
+  // the blocks of a (batch, head) go in pairs (q_blocks - 1 - i, i), heavy first, so every workgroup
+  // runs about the same number of tiles and the light block's K and V are a prefix of the heavy
+  // one's. Causal, not paired: block q_blocks - 1 of every (batch, head), then block q_blocks - 2 of
+  // every one, and so on, for grids whose pairs would leave the last round mostly empty.
+  int bh, item;
+  if (a.causal && !a.paired) {
+    const int bhs = a.batch * a.work_heads;
+    item = blockIdx.x / bhs;
+    bh = xcd_remap(blockIdx.x - item * bhs, bhs);
+  } else {
+    const int work = xcd_remap(blockIdx.x, gridDim.x);
+    const int items_per_bh = a.causal ? (a.q_blocks + 1) / 2 : a.q_blocks;
+    bh = work / items_per_bh;
+    item = work - bh * items_per_bh;
+  }
+  const int b = bh / a.work_heads;
+  const int h = (bh - b * a.work_heads) * a.pack;  // first query head
   const int hkv = h / a.group;
   const uint16_t* qp = a.q + b * a.q_bs + h * a.q_hs;
   const uint16_t* kp = a.k + b * a.k_bs + hkv * a.k_hs;
@@ -145,8 +156,10 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   u32x4 qf[D / 16];
   auto load_q = [&](int qb) {
     const int r = qb * kBlockM + wave * kRowsPerWave + (lane & 31);
-    const bool ok = r < a.seqlen_q;
-    const uint16_t* src = qp + static_cast<int64_t>(ok ? r : 0) * a.q_ss + 8 * half;
+    const bool ok = r < a.rows;
+    const int pos = ok ? pack_position(a, r) : 0;
+    const int g = ok ? r - pos * a.pack : 0;
+    const uint16_t* src = qp + pos * a.q_ss + g * a.q_hs + 8 * half;
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) qf[ks] = ok ? load16(src + 16 * ks) : u32x4{0, 0, 0, 0};
   };
@@ -167,10 +180,11 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   auto process = [&](const int qb, const int next_qb) {
     const int q0 = qb * kBlockM;
     const int row0 = q0 + wave * kRowsPerWave;
-    const int my_row = row0 + (lane & 31);
+    const int my_pos = pack_position(a, row0 + (lane & 31));
 
     int kv_end = a.seqlen_k;
-    if (a.causal) kv_end = min(kv_end, min(q0 + kBlockM, a.seqlen_q) + a.causal_offset);
+    if (a.causal)
+      kv_end = min(kv_end, pack_position(a, min(q0 + kBlockM, a.rows) - 1) + 1 + a.causal_offset);
     const int num_tiles = kv_end > 0 ? (kv_end + kBlockN - 1) / kBlockN : 0;
     // Tiles this wave sees any key of (a prefix of the workgroup's tiles), and the first tile whose
     // scores need masking (it reaches past the sequence end or, causal, past the diagonal of the
@@ -178,14 +192,16 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     int my_tiles = num_tiles;
     int mask_from = a.seqlen_k / kBlockN;
     if (a.causal) {
-      const int last = row0 + kRowsPerWave - 1 + a.causal_offset;  // last key any of its rows sees
+      // last key any of its rows sees
+      const int last = pack_position(a, row0 + kRowsPerWave - 1) + a.causal_offset;
       my_tiles = last < 0 ? 0 : min(num_tiles, last / kBlockN + 1);
-      const int x = row0 + a.causal_offset - (kBlockN - 1);  // tile t needs masking iff 64 t > x
+      // tile t needs masking iff 64 t > x
+      const int x = pack_position(a, row0) + a.causal_offset - (kBlockN - 1);
       mask_from = min(mask_from, x < 0 ? 0 : x / kBlockN + 1);
     }
     // A wave whose rows all lie past the sequence (the last block of a ragged S_q) only keeps its
     // turn in the loads and barriers.
-    if (row0 >= a.seqlen_q) my_tiles = 0;
+    if (row0 >= a.rows) my_tiles = 0;
 
     if (!q_loaded) {
       load_q(qb);
@@ -230,7 +246,7 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     float l = 0.f;  // the lane's part of its row's sum; with kMfmaSums, the whole row's
     f32x4 ls = {};  // kMfmaSums: P's row sums from the last MFMA phase, added by the next softmax
     const float sl2 = a.scale_log2;
-    const int last_key = a.causal ? min(a.seqlen_k - 1, my_row + a.causal_offset) : a.seqlen_k - 1;
+    const int last_key = a.causal ? min(a.seqlen_k - 1, my_pos + a.causal_offset) : a.seqlen_k - 1;
 
     // MFMA phase of a period with slots kS = m % kStages: O += V(m-1) P(m-1) (16 MFMAs) and
     // S = K(m) Q^T (16 MFMAs). No branches: in period 0 the previous P and V are zeros (P starts at
@@ -653,18 +669,22 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
       for (int j = 0; j < kRowsPerWave / kRowsPerStore; ++j) {
         const int r = row0 + j * kRowsPerStore + e_lane / kChunks;
         const u32x4 v = *reinterpret_cast<const u32x4*>(rbase + j * kRowsPerStore * kStageRow);
-        if (r < a.seqlen_q) *reinterpret_cast<u32x4*>(obase + static_cast<int64_t>(r) * a.o_ss) = v;
+        const int pos = pack_position(a, r);
+        const int g = r - pos * a.pack;
+        if (r < a.rows) *reinterpret_cast<u32x4*>(obase + pos * a.o_ss + g * a.o_hs) = v;
       }
     }
-    if (e_row < a.seqlen_q && e_half == 0) {
-      a.lse[(static_cast<int64_t>(b) * a.heads + h) * a.seqlen_q + e_row] =
+    if (e_row < a.rows && e_half == 0) {
+      const int pos = pack_position(a, e_row);
+      const int g = e_row - pos * a.pack;
+      a.lse[(static_cast<int64_t>(b) * a.heads + h + g) * a.seqlen_q + pos] =
           lt > 0.f ? ref * kLn2 + logf(lt) : -INFINITY;
     }
   };
 
   // One call site (a loop), so the block body is inlined once.
   const int heavy = a.q_blocks - 1 - item;
-  const int blocks_here = a.causal && item < heavy ? 2 : 1;
+  const int blocks_here = a.causal && a.paired && item < heavy ? 2 : 1;
   for (int i = 0; i < blocks_here; ++i) {
     // The next block's prologue refills the ring, which the epilogue's staging reads just used (no
     // memory fence: the output stores need not complete first).
@@ -675,9 +695,18 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
 
 template <typename Tag, int D>
 hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
-  args.q_blocks = (args.seqlen_q + kPpBlockMOf<D> - 1) / kPpBlockMOf<D>;
-  const int items_per_bh = args.causal ? (args.q_blocks + 1) / 2 : args.q_blocks;
-  const int blocks = items_per_bh * args.batch * args.heads;
+  args.q_blocks = (args.rows + kPpBlockMOf<D> - 1) / kPpBlockMOf<D>;
+  const int pairs = (args.q_blocks + 1) / 2 * args.batch * args.work_heads;
+  // Pairs all take about the same time, so a last round that is partly empty costs a whole one; single
+  // blocks, heaviest first, fill it, but start more blocks without the pair's early query rows. The
+  // line is where the two measured the same (us, singles / pairs; (B, H, H_kv, S, D), share of the
+  // rounds' workgroups that pairs fill): (1, 32, 8, 5000, 128) 63% 188 / 233, (8, 16, 16, 2048, 64)
+  // 75% 95 / 116, (5, 32, 8, 2048, 128) 83% 181 / 184, (14, 32, 8, 512, 128) 88% 63 / 58, (16, 32, 8,
+  // 700, 128) 100% 114 / 104; with many blocks per head a start weighs less: (1, 32, 8, 7000, 128)
+  // 86% 340 / 347, (3, 24, 8, 4627, 64) 89% 218 / 230.
+  const int64_t slots = static_cast<int64_t>((pairs + kCus - 1) / kCus) * kCus;
+  args.paired = int64_t{100} * pairs >= (args.q_blocks >= 32 ? 90 : 85) * slots;
+  const int blocks = args.causal && args.paired ? pairs : args.q_blocks * args.batch * args.work_heads;
   hipLaunchKernelGGL((prefill_pp_kernel<Tag, D>), dim3(blocks), dim3(64 * kPpWavesOf<D>), 0, stream, args);
   return hipGetLastError();
 }

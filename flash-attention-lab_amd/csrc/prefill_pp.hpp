@@ -28,6 +28,7 @@ constexpr int kPpWavesOf = 4 * kPpGroups<D>;
 template <int D>
 constexpr int kPpBlockMOf = kRowsPerWave * kPpWavesOf<D>;  // 256 rows at D = 128, 384 at 64
 constexpr int kXcds = 8;
+constexpr int kCus = 256;
 constexpr float kLn2 = 0.693147180559945309f;
 // Reference point of a row that has not seen a key yet: finite, so a masked score (-inf) still
 // gives p = 2^(s scale_log2 - ref) = 0 and the first visible key always moves it, with no separate
