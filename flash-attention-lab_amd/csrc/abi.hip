@@ -273,6 +273,132 @@ int decode_call(const fl_decode_params* p, float* workspace, size_t workspace_by
   return FL_OK;
 }
 
+int check_attention_shape(const fl_attn_params* p) {
+  if (p == nullptr) return fail(FL_ERR_INVALID, "null attention parameters");
+  if (p->dtype != FL_DTYPE_BF16 && p->dtype != FL_DTYPE_F16)
+    return fail(FL_ERR_UNSUPPORTED, "attention_mma_pipelined takes bf16 or fp16");
+  if (p->head_dim != 64 && p->head_dim != 128)
+    return fail(FL_ERR_UNSUPPORTED, fmt("unsupported head_dim %lld", p->head_dim));
+  if (p->batch <= 0 || p->seqlen_q <= 0 || p->seqlen_k <= 0 || p->heads <= 0 || p->heads_kv <= 0)
+    return fail(FL_ERR_INVALID, "empty input");
+  if (p->heads % p->heads_kv != 0)
+    return fail(FL_ERR_INVALID, "query heads must be a multiple of KV heads");
+  const int64_t q_blocks = (static_cast<int64_t>(p->seqlen_q) + fl::kPrefillBlockM - 1) /
+                           fl::kPrefillBlockM;
+  const int64_t blocks = q_blocks * p->batch * p->heads;
+  if (blocks > (int64_t{1} << 24))
+    return fail(FL_ERR_INVALID, "batch * heads * query blocks exceeds the grid limit");
+  return FL_OK;
+}
+
+// The sizes of a checked attention call, and how its rows are packed; `split`: its keys are (or may
+// be) split.
+void attention_sizes(const fl_attn_params* p, bool split, fl::PrefillArgs& a) {
+  a.batch = p->batch;
+  a.seqlen_q = p->seqlen_q;
+  a.seqlen_k = p->seqlen_k;
+  a.heads = p->heads;
+  a.heads_kv = p->heads_kv;
+  a.group = p->heads / p->heads_kv;
+  a.causal_offset = p->seqlen_k - p->seqlen_q;
+  a.causal = p->causal != 0;
+  // The query heads of a KV head share its K and V tiles, so their rows are packed (launch.hpp): a
+  // block then covers 1 / group of the positions, which leaves less of it past a causal diagonal and
+  // past the last row. (B, H, H_kv, S, D) causal, one box, before / after: (16, 32, 8, 700, 128) 128 /
+  // 104 us, (4, 16, 2, 1078, 64) 41 / 23, (8, 24, 8, 28, 64) 5.7 / 4.4, (1, 32, 8, 8192, 128) 439 / 437.
+  // Not, unless the keys are split, where the packed grid is smaller than half the CUs: there the
+  // time is that of one workgroup's rows, and separate heads spread them over more CUs ((1, 64, 8),
+  // 18 new rows after 1,194 keys, D = 128: 23.0 us separate, 25.0 packed). Nor past pack_position's
+  // range.
+  const int64_t packed_rows = static_cast<int64_t>(p->seqlen_q) * a.group;
+  const int64_t packed_grid = (packed_rows + fl::kPrefillBlockM - 1) / fl::kPrefillBlockM *
+                              p->batch * p->heads_kv;
+  a.pack = packed_rows < (int64_t{1} << 30) && (split || packed_grid >= 128) ? a.group : 1;
+  a.work_heads = p->heads / a.pack;
+  a.rows = p->seqlen_q * a.pack;
+  // Division by a constant d < 2^31 of any n < 2^31 as a multiplication: with 2^l >= d,
+  // m = floor(2^(31 + l) / d) + 1 exceeds 2^(31 + l) / d by at most 1, so n m / 2^(31 + l) exceeds
+  // n / d by less than 2^31 / 2^(31 + l) <= 1 / d.
+  a.pack_shift = 31;
+  while ((int64_t{1} << (a.pack_shift - 31)) < a.pack) ++a.pack_shift;
+  a.pack_mul = static_cast<uint32_t>((uint64_t{1} << a.pack_shift) / static_cast<uint32_t>(a.pack) + 1);
+}
+
+size_t prefill_workspace_bytes(const fl::PrefillArgs& a, int head_dim, int num_splits) {
+  int64_t ml_offset = 0;
+  return num_splits > 1 ? fl::prefill_partial_floats(a, head_dim, num_splits, &ml_offset) * sizeof(float) : 0;
+}
+
+int attention_call(const fl_attn_params* p, int num_splits, float* workspace, size_t workspace_bytes,
+                   fl_stream_t stream) {
+  if (int rc = check_attention_shape(p)) return rc;
+  if (!valid_scale(p->softmax_scale)) return fail(FL_ERR_INVALID, "softmax_scale must be positive");
+  if (!p->q || !p->k || !p->v || !p->o || !p->lse)
+    return fail(FL_ERR_INVALID, "null tensor pointer");
+  const int eb = elem_bytes(p->dtype);
+  if (!rows_16_byte(p->q, eb, p->batch, p->q_batch_stride, p->seqlen_q, p->q_seq_stride, p->heads,
+                    p->q_head_stride))
+    return fail(FL_ERR_INVALID, "q must have 16-byte aligned rows (data pointer and strides)");
+  if (!rows_16_byte(p->k, eb, p->batch, p->k_batch_stride, p->seqlen_k, p->k_seq_stride,
+                    p->heads_kv, p->k_head_stride))
+    return fail(FL_ERR_INVALID, "k must have 16-byte aligned rows (data pointer and strides)");
+  if (!rows_16_byte(p->v, eb, p->batch, p->v_batch_stride, p->seqlen_k, p->v_seq_stride,
+                    p->heads_kv, p->v_head_stride))
+    return fail(FL_ERR_INVALID, "v must have 16-byte aligned rows (data pointer and strides)");
+  if (!rows_16_byte(p->o, eb, p->batch, p->o_batch_stride, p->seqlen_q, p->o_seq_stride, p->heads,
+                    p->o_head_stride))
+    return fail(FL_ERR_INVALID, "o must have 16-byte aligned rows (data pointer and strides)");
+  if (!aligned(p->lse, 4)) return fail(FL_ERR_INVALID, "lse must be 4-byte aligned");
+  // Tile loads address K and V rows through 32-bit byte offsets from a per-tile base, and rely on
+  // rows not overlapping (sequence stride >= head_dim) to zero-fill past the end.
+  const int64_t max_seq_stride = ((int64_t{1} << 31) / 2 - p->head_dim) / fl::kPrefillBlockN;
+  if (p->seqlen_k > 1 && (p->k_seq_stride < p->head_dim || p->v_seq_stride < p->head_dim))
+    return fail(FL_ERR_INVALID, "k and v rows must not overlap (sequence stride >= head_dim)");
+  if (p->k_seq_stride > max_seq_stride || p->v_seq_stride > max_seq_stride)
+    return fail(FL_ERR_INVALID, "k or v sequence stride too large");
+
+  fl::PrefillArgs a{};
+  a.q = static_cast<const uint16_t*>(p->q);
+  a.k = static_cast<const uint16_t*>(p->k);
+  a.v = static_cast<const uint16_t*>(p->v);
+  a.o = static_cast<uint16_t*>(p->o);
+  a.lse = p->lse;
+  a.q_bs = p->q_batch_stride;
+  a.q_ss = p->q_seq_stride;
+  a.q_hs = p->q_head_stride;
+  a.k_bs = p->k_batch_stride;
+  a.k_ss = p->k_seq_stride;
+  a.k_hs = p->k_head_stride;
+  a.v_bs = p->v_batch_stride;
+  a.v_ss = p->v_seq_stride;
+  a.v_hs = p->v_head_stride;
+  a.o_bs = p->o_batch_stride;
+  a.o_ss = p->o_seq_stride;
+  a.o_hs = p->o_head_stride;
+  attention_sizes(p, num_splits > 1, a);
+  a.scale = static_cast<float>(p->softmax_scale);
+  a.scale_log2 = static_cast<float>(p->softmax_scale * 1.4426950408889634);
+  a.num_splits = num_splits;
+  const fl::DType dt = p->dtype == FL_DTYPE_BF16 ? fl::DType::bf16 : fl::DType::f16;
+  hipError_t err = hipSuccess;
+  if (num_splits > 1) {
+    int64_t ml_offset = 0;
+    const int64_t floats = fl::prefill_partial_floats(a, p->head_dim, num_splits, &ml_offset);
+    if (floats / (p->head_dim + 2) / fl::kPrefillBlockN > (int64_t{1} << 24))
+      return fail(FL_ERR_INVALID, "batch * heads * query blocks * num_splits exceeds the grid limit");
+    if (workspace == nullptr || workspace_bytes < floats * sizeof(float))
+      return fail(FL_ERR_INVALID, "attention workspace is missing or smaller than fl_attention_plan reports");
+    if (!aligned(workspace, 16)) return fail(FL_ERR_INVALID, "attention workspace must be 16-byte aligned");
+    a.partial_o = workspace;
+    a.partial_ml = reinterpret_cast<fl::f32pair*>(workspace + ml_offset);
+    err = fl::launch_prefill_split(a, dt, p->head_dim, static_cast<hipStream_t>(stream));
+  } else {
+    err = fl::launch_prefill(a, dt, p->head_dim, static_cast<hipStream_t>(stream));
+  }
+  if (err != hipSuccess) return fail(FL_ERR_LAUNCH, std::string("prefill launch: ") + hipGetErrorString(err));
+  return FL_OK;
+}
+
 // The split workspace of fl_decode_noalloc: a file-scope device array, one copy per GPU (each GPU
 // the library runs on holds it until the process ends). In host code `scratch` is a host-side
 // stand-in for the array, not its device address: the address comes from hipGetSymbolAddress,
@@ -325,99 +451,34 @@ const char* fl_last_error(void) { return g_last_error.c_str(); }
 const char* fl_version(void) { return "flash_lab_hip 0.1.0 gfx950"; }
 
 int fl_attention_fwd(const fl_attn_params* p, fl_stream_t stream) {
-  if (p == nullptr) return fail(FL_ERR_INVALID, "null attention parameters");
-  if (p->dtype != FL_DTYPE_BF16 && p->dtype != FL_DTYPE_F16)
-    return fail(FL_ERR_UNSUPPORTED, "attention_mma_pipelined takes bf16 or fp16");
-  if (p->head_dim != 64 && p->head_dim != 128)
-    return fail(FL_ERR_UNSUPPORTED, fmt("unsupported head_dim %lld", p->head_dim));
-  if (p->batch <= 0 || p->seqlen_q <= 0 || p->seqlen_k <= 0 || p->heads <= 0 || p->heads_kv <= 0)
-    return fail(FL_ERR_INVALID, "empty input");
-  if (p->heads % p->heads_kv != 0)
-    return fail(FL_ERR_INVALID, "query heads must be a multiple of KV heads");
-  if (!valid_scale(p->softmax_scale)) return fail(FL_ERR_INVALID, "softmax_scale must be positive");
-  if (!p->q || !p->k || !p->v || !p->o || !p->lse)
-    return fail(FL_ERR_INVALID, "null tensor pointer");
-  const int eb = elem_bytes(p->dtype);
-  if (!rows_16_byte(p->q, eb, p->batch, p->q_batch_stride, p->seqlen_q, p->q_seq_stride, p->heads,
-                    p->q_head_stride))
-    return fail(FL_ERR_INVALID, "q must have 16-byte aligned rows (data pointer and strides)");
-  if (!rows_16_byte(p->k, eb, p->batch, p->k_batch_stride, p->seqlen_k, p->k_seq_stride,
-                    p->heads_kv, p->k_head_stride))
-    return fail(FL_ERR_INVALID, "k must have 16-byte aligned rows (data pointer and strides)");
-  if (!rows_16_byte(p->v, eb, p->batch, p->v_batch_stride, p->seqlen_k, p->v_seq_stride,
-                    p->heads_kv, p->v_head_stride))
-    return fail(FL_ERR_INVALID, "v must have 16-byte aligned rows (data pointer and strides)");
-  if (!rows_16_byte(p->o, eb, p->batch, p->o_batch_stride, p->seqlen_q, p->o_seq_stride, p->heads,
-                    p->o_head_stride))
-    return fail(FL_ERR_INVALID, "o must have 16-byte aligned rows (data pointer and strides)");
-  if (!aligned(p->lse, 4)) return fail(FL_ERR_INVALID, "lse must be 4-byte aligned");
-  // Tile loads address K and V rows through 32-bit byte offsets from a per-tile base, and rely on
-  // rows not overlapping (sequence stride >= head_dim) to zero-fill past the end.
-  const int64_t max_seq_stride = ((int64_t{1} << 31) / 2 - p->head_dim) / fl::kPrefillBlockN;
-  if (p->seqlen_k > 1 && (p->k_seq_stride < p->head_dim || p->v_seq_stride < p->head_dim))
-    return fail(FL_ERR_INVALID, "k and v rows must not overlap (sequence stride >= head_dim)");
-  if (p->k_seq_stride > max_seq_stride || p->v_seq_stride > max_seq_stride)
-    return fail(FL_ERR_INVALID, "k or v sequence stride too large");
+  return attention_call(p, 1, nullptr, 0, stream);
+}
 
-  const int64_t q_blocks = (static_cast<int64_t>(p->seqlen_q) + fl::kPrefillBlockM - 1) /
-                           fl::kPrefillBlockM;
-  const int64_t blocks = q_blocks * p->batch * p->heads;
-  if (blocks > (int64_t{1} << 24))
-    return fail(FL_ERR_INVALID, "batch * heads * query blocks exceeds the grid limit");
-
+int fl_attention_plan(const fl_attn_params* p, int32_t requested_splits, int32_t cu_count,
+                      int32_t* num_splits, size_t* workspace_bytes) {
+  if (int rc = check_attention_shape(p)) return rc;
+  if (requested_splits < 0 || requested_splits > fl::kMaxPrefillSplits)
+    return fail(FL_ERR_INVALID, "num_splits must be in [0, 64]");
+  if (num_splits == nullptr || workspace_bytes == nullptr)
+    return fail(FL_ERR_INVALID, "null output pointer");
   fl::PrefillArgs a{};
-  a.q = static_cast<const uint16_t*>(p->q);
-  a.k = static_cast<const uint16_t*>(p->k);
-  a.v = static_cast<const uint16_t*>(p->v);
-  a.o = static_cast<uint16_t*>(p->o);
-  a.lse = p->lse;
-  a.q_bs = p->q_batch_stride;
-  a.q_ss = p->q_seq_stride;
-  a.q_hs = p->q_head_stride;
-  a.k_bs = p->k_batch_stride;
-  a.k_ss = p->k_seq_stride;
-  a.k_hs = p->k_head_stride;
-  a.v_bs = p->v_batch_stride;
-  a.v_ss = p->v_seq_stride;
-  a.v_hs = p->v_head_stride;
-  a.o_bs = p->o_batch_stride;
-  a.o_ss = p->o_seq_stride;
-  a.o_hs = p->o_head_stride;
-  a.batch = p->batch;
-  a.seqlen_q = p->seqlen_q;
-  a.seqlen_k = p->seqlen_k;
-  a.heads = p->heads;
-  a.heads_kv = p->heads_kv;
-  a.group = p->heads / p->heads_kv;
-  a.causal_offset = p->seqlen_k - p->seqlen_q;
-  a.causal = p->causal != 0;
-  a.scale = static_cast<float>(p->softmax_scale);
-  a.scale_log2 = static_cast<float>(p->softmax_scale * 1.4426950408889634);
-  a.q_blocks = static_cast<int>(q_blocks);
-  // The query heads of a KV head share its K and V tiles, so their rows are packed (launch.hpp): a
-  // block then covers 1 / group of the positions, which leaves less of it past a causal diagonal and
-  // past the last row. (B, H, H_kv, S, D) causal, one box, before / after: (16, 32, 8, 700, 128) 128 /
-  // 104 us, (4, 16, 2, 1078, 64) 41 / 23, (8, 24, 8, 28, 64) 5.7 / 4.4, (1, 32, 8, 8192, 128) 439 / 437.
-  // Not where the packed grid is smaller than half the CUs: there the time is that of one
-  // workgroup's rows, and separate heads spread them over more CUs ((1, 64, 8), 18 new rows after
-  // 1,194 keys, D = 128: 23.0 us separate, 25.0 packed). Nor past pack_position's range.
-  const int64_t packed_rows = static_cast<int64_t>(p->seqlen_q) * a.group;
-  const int64_t packed_grid = (packed_rows + fl::kPrefillBlockM - 1) / fl::kPrefillBlockM *
-                              p->batch * p->heads_kv;
-  a.pack = packed_rows < (int64_t{1} << 30) && packed_grid >= 128 ? a.group : 1;
-  a.work_heads = p->heads / a.pack;
-  a.rows = p->seqlen_q * a.pack;
-  // Division by a constant d < 2^31 of any n < 2^31 as a multiplication: with 2^l >= d,
-  // m = floor(2^(31 + l) / d) + 1 exceeds 2^(31 + l) / d by at most 1, so n m / 2^(31 + l) exceeds
-  // n / d by less than 2^31 / 2^(31 + l) <= 1 / d.
-  a.pack_shift = 31;
-  while ((int64_t{1} << (a.pack_shift - 31)) < a.pack) ++a.pack_shift;
-  a.pack_mul = static_cast<uint32_t>((uint64_t{1} << a.pack_shift) / static_cast<uint32_t>(a.pack) + 1);
-
-  const fl::DType dt = p->dtype == FL_DTYPE_BF16 ? fl::DType::bf16 : fl::DType::f16;
-  const hipError_t err = fl::launch_prefill(a, dt, p->head_dim, static_cast<hipStream_t>(stream));
-  if (err != hipSuccess) return fail(FL_ERR_LAUNCH, std::string("prefill launch: ") + hipGetErrorString(err));
+  attention_sizes(p, true, a);
+  *num_splits = requested_splits > 0 ? requested_splits : fl::prefill_splits(a, p->head_dim, cu_count);
+  *workspace_bytes = prefill_workspace_bytes(a, p->head_dim, *num_splits);
   return FL_OK;
+}
+
+int fl_attention_fwd_split(const fl_attn_params* p, int32_t num_splits, int32_t cu_count,
+                           float* workspace, size_t workspace_bytes, fl_stream_t stream) {
+  if (num_splits < 0 || num_splits > fl::kMaxPrefillSplits)
+    return fail(FL_ERR_INVALID, "num_splits must be in [0, 64]");
+  if (num_splits == 0) {
+    size_t need = 0;
+    if (int rc = fl_attention_plan(p, 0, cu_count, &num_splits, &need)) return rc;
+    if (need > 0 && (workspace == nullptr || workspace_bytes < need))
+      return fail(FL_ERR_WORKSPACE, "attention workspace is missing or smaller than fl_attention_plan reports");
+  }
+  return attention_call(p, num_splits, workspace, workspace_bytes, stream);
 }
 
 int fl_decode_plan(const fl_decode_params* p, int32_t requested_splits, int32_t allow_splits,

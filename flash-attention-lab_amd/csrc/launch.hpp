@@ -9,6 +9,10 @@
 
 namespace fl {
 
+struct f32pair {
+  float x, y;
+};
+
 // Prefill problem as the kernels see it. Tensors are [B, S, H, D] with unit stride in D; strides
 // are in elements. Query head h reads KV head h / group; query row i sees key j iff
 // j <= i + causal_offset (bottom-right aligned causal mask).
@@ -36,6 +40,13 @@ struct PrefillArgs {
   // Causal ping-pong calls: 1 = a workgroup runs a heavy and a light block of rows, 0 = one block per
   // workgroup, the heaviest of every work head first.
   int paired;
+  // Split calls (num_splits > 1): split s of a block of rows takes its s-th share of the block's key
+  // tiles and writes unnormalized fp32 partials, which a merge pass combines. Per (block, split,
+  // wave), in the accumulators' own layout: partial_o [D / 8][64 lanes][4], then partial_ml [32 rows]
+  // of (reference point in log2 units or -inf, sum).
+  int num_splits;
+  float* partial_o;
+  f32pair* partial_ml;
 };
 __host__ __device__ __forceinline__ int pack_position(const PrefillArgs& a, int row) {
   return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(row)) * a.pack_mul) >> a.pack_shift);
@@ -98,11 +109,19 @@ int knob(int which);
 // Rows of queries per prefill workgroup (the kernel's tile height) and keys per tile.
 constexpr int kPrefillBlockM = 128;
 constexpr int kPrefillBlockN = 64;
+// Largest key split count of a prefill call.
+constexpr int kMaxPrefillSplits = 64;
 
 hipError_t launch_prefill(const PrefillArgs& args, DType dtype, int head_dim, hipStream_t stream);
 // Ping-pong variant (head_dim 128 and 64): 8 waves, 256 query rows per workgroup.
 hipError_t launch_prefill_pingpong(const PrefillArgs& args, DType dtype, int head_dim,
                                    hipStream_t stream);
+// Key splits of a call of these sizes (pack, rows, work_heads set), 1 where splitting does not pay,
+// and the partials a split call needs (floats, all of its partial_o then all of its partial_ml).
+int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count);
+int64_t prefill_partial_floats(const PrefillArgs& args, int head_dim, int num_splits, int64_t* ml_offset);
+// The ping-pong kernel on args.num_splits shares of each block's key tiles, and the merge pass.
+hipError_t launch_prefill_split(const PrefillArgs& args, DType dtype, int head_dim, hipStream_t stream);
 // The same kernel for causal calls with a pair of query blocks per workgroup run as one stream of
 // key tiles (prefill_causal.hip); launch_prefill_pingpong routes causal calls to it when the
 // FL_KNOB_PREFILL_CAUSAL_STREAM knob is 1.

@@ -53,7 +53,7 @@ namespace prefill {
 namespace pp {
 namespace {
 
-template <typename Tag, int D>
+template <typename Tag, int D, bool kSplit>
 __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     __attribute__((amdgpu_waves_per_eu(kPpGroups<D>, kPpGroups<D>))) prefill_pp_kernel(const PrefillArgs a) {
   using E = Elem<Tag>;
@@ -89,7 +89,10 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   // n + 16 ((m / 4) % 2), which lands in lane n + 16 (m / 4): every register of lane l holds the
   // sum of its own row l % 32 over both halves. Lane l holds A[l % 16][8 (l / 16) + e], e = 0..7,
   // all equal. This sums the probabilities as rounded for P V, so o and l agree exactly on them.
-  constexpr bool kMfmaSums = D == 64;
+  // (Not in split calls: the 4-wave kernel, which those calls run on where they are not split, sums
+  // the unrounded probabilities, and so does the split form, so splitting does not change what the
+  // log-sum-exp is exact to.)
+  constexpr bool kMfmaSums = D == 64 && !kSplit;
   const uint32_t sel_word = ((lane >> 4) & 1) == ((lane >> 2) & 1) ? E::kOnePair : 0u;
   const u32x4 sum_sel{sel_word, sel_word, sel_word, sel_word};
 
@@ -98,8 +101,16 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   // runs about the same number of tiles and the light block's K and V are a prefix of the heavy
   // one's. Causal, not paired: block q_blocks - 1 of every (batch, head), then block q_blocks - 2 of
   // every one, and so on, for grids whose pairs would leave the last round mostly empty.
-  int bh, item;
-  if (a.causal && !a.paired) {
+  // Split: the same order over (batch, head, split), so that the blocks that share a split's tiles
+  // run on one XCD.
+  int bh, item, split = 0;
+  if constexpr (kSplit) {
+    const int units = a.batch * a.work_heads * a.num_splits;
+    item = blockIdx.x / units;
+    const int unit = xcd_remap(blockIdx.x - item * units, units);
+    bh = unit / a.num_splits;
+    split = unit - bh * a.num_splits;
+  } else if (a.causal && !a.paired) {
     const int bhs = a.batch * a.work_heads;
     item = blockIdx.x / bhs;
     bh = xcd_remap(blockIdx.x - item * bhs, bhs);
@@ -115,6 +126,24 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
   const uint16_t* qp = a.q + b * a.q_bs + h * a.q_hs;
   const uint16_t* kp = a.k + b * a.k_bs + hkv * a.k_hs;
   const uint16_t* vp = a.v + b * a.v_bs + hkv * a.v_hs;
+  // Keys the workgroup sees, and the key position of query position 0. A split sees its share of the
+  // block's tiles as if they were all: keys and positions count from its first tile.
+  int seqlen_k = a.seqlen_k;
+  int causal_offset = a.causal_offset;
+  if constexpr (kSplit) {
+    int end = seqlen_k;
+    if (a.causal) {
+      const int last_row = min((a.q_blocks - item) * kBlockM, a.rows) - 1;
+      end = max(min(end, pack_position(a, last_row) + 1 + causal_offset), 0);
+    }
+    const int tiles = (end + kBlockN - 1) / kBlockN;
+    const int t0 = static_cast<int64_t>(tiles) * split / a.num_splits;
+    const int t1 = static_cast<int64_t>(tiles) * (split + 1) / a.num_splits;
+    kp += static_cast<int64_t>(t0) * kBlockN * a.k_ss;
+    vp += static_cast<int64_t>(t0) * kBlockN * a.v_ss;
+    seqlen_k = max(min(seqlen_k, t1 * kBlockN) - t0 * kBlockN, 0);
+    causal_offset -= t0 * kBlockN;
+  }
 
   int k_lds[D / 16];
 #pragma unroll
@@ -182,21 +211,21 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     const int row0 = q0 + wave * kRowsPerWave;
     const int my_pos = pack_position(a, row0 + (lane & 31));
 
-    int kv_end = a.seqlen_k;
+    int kv_end = seqlen_k;
     if (a.causal)
-      kv_end = min(kv_end, pack_position(a, min(q0 + kBlockM, a.rows) - 1) + 1 + a.causal_offset);
+      kv_end = min(kv_end, pack_position(a, min(q0 + kBlockM, a.rows) - 1) + 1 + causal_offset);
     const int num_tiles = kv_end > 0 ? (kv_end + kBlockN - 1) / kBlockN : 0;
     // Tiles this wave sees any key of (a prefix of the workgroup's tiles), and the first tile whose
     // scores need masking (it reaches past the sequence end or, causal, past the diagonal of the
     // wave's first row): every tile before it is fully visible to every row of the wave.
     int my_tiles = num_tiles;
-    int mask_from = a.seqlen_k / kBlockN;
+    int mask_from = seqlen_k / kBlockN;
     if (a.causal) {
       // last key any of its rows sees
-      const int last = pack_position(a, row0 + kRowsPerWave - 1) + a.causal_offset;
+      const int last = pack_position(a, row0 + kRowsPerWave - 1) + causal_offset;
       my_tiles = last < 0 ? 0 : min(num_tiles, last / kBlockN + 1);
       // tile t needs masking iff 64 t > x
-      const int x = pack_position(a, row0) + a.causal_offset - (kBlockN - 1);
+      const int x = pack_position(a, row0) + causal_offset - (kBlockN - 1);
       mask_from = min(mask_from, x < 0 ? 0 : x / kBlockN + 1);
     }
     // A wave whose rows all lie past the sequence (the last block of a ragged S_q) only keeps its
@@ -209,7 +238,7 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     }
     q_loaded = false;
 
-    const int last_rows = num_tiles > 0 ? min(kBlockN, a.seqlen_k - (num_tiles - 1) * kBlockN) : 1;
+    const int last_rows = num_tiles > 0 ? min(kBlockN, seqlen_k - (num_tiles - 1) * kBlockN) : 1;
     const uint32_t full_bytes = static_cast<uint32_t>(((kBlockN - 1) * my_ss + D) * 2);
     const uint32_t last_bytes = static_cast<uint32_t>(((last_rows - 1) * my_ss + D) * 2);
     auto tile_words = [&](int t) -> u32x4s {
@@ -246,7 +275,7 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     float l = 0.f;  // the lane's part of its row's sum; with kMfmaSums, the whole row's
     f32x4 ls = {};  // kMfmaSums: P's row sums from the last MFMA phase, added by the next softmax
     const float sl2 = a.scale_log2;
-    const int last_key = a.causal ? min(a.seqlen_k - 1, my_pos + a.causal_offset) : a.seqlen_k - 1;
+    const int last_key = a.causal ? min(seqlen_k - 1, my_pos + causal_offset) : seqlen_k - 1;
 
     // MFMA phase of a period with slots kS = m % kStages: O += V(m-1) P(m-1) (16 MFMAs) and
     // S = K(m) Q^T (16 MFMAs). No branches: in period 0 the previous P and V are zeros (P starts at
@@ -628,6 +657,24 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
     if (q_loaded) consume_q();
 
     const float lt = kMfmaSums ? l + ls[0] : sum_halves(l);
+    if constexpr (kSplit) {
+      // The wave's partials as its accumulators hold them: every store is 1 KiB in one piece.
+      if (row0 < a.rows) {
+        const int64_t slot =
+            ((static_cast<int64_t>(bh) * a.q_blocks + qb) * a.num_splits + split) * kPpWavesOf<D> + wave;
+        f32x4* po = reinterpret_cast<f32x4*>(a.partial_o) + slot * (D / 8 * 64) + lane;
+#pragma unroll
+        for (int nb = 0; nb < D / 32; ++nb) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            po[(4 * nb + g) * 64] =
+                f32x4{o[nb][4 * g], o[nb][4 * g + 1], o[nb][4 * g + 2], o[nb][4 * g + 3]};
+          }
+        }
+        if (half == 0) a.partial_ml[slot * kRowsPerWave + lane] = f32pair{lt > 0.f ? ref : -INFINITY, lt};
+      }
+      return;
+    }
     const float inv = lt > 0.f ? 1.f / lt : 0.f;
     // Output rows go back whole, 16 bytes per lane (the accumulator layout would store 8 bytes per
     // lane into 32 rows a row stride apart): each wave stages its 32 rows in its own part of the
@@ -684,6 +731,10 @@ __global__ void __launch_bounds__(64 * kPpWavesOf<D>)
 
   // One call site (a loop), so the block body is inlined once.
   const int heavy = a.q_blocks - 1 - item;
+  if constexpr (kSplit) {
+    process(heavy, -1);
+    return;
+  }
   const int blocks_here = a.causal && a.paired && item < heavy ? 2 : 1;
   for (int i = 0; i < blocks_here; ++i) {
     // The next block's prologue refills the ring, which the epilogue's staging reads just used (no
@@ -707,7 +758,78 @@ hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
   const int64_t slots = static_cast<int64_t>((pairs + kCus - 1) / kCus) * kCus;
   args.paired = int64_t{100} * pairs >= (args.q_blocks >= 32 ? 90 : 85) * slots;
   const int blocks = args.causal && args.paired ? pairs : args.q_blocks * args.batch * args.work_heads;
-  hipLaunchKernelGGL((prefill_pp_kernel<Tag, D>), dim3(blocks), dim3(64 * kPpWavesOf<D>), 0, stream, args);
+  hipLaunchKernelGGL((prefill_pp_kernel<Tag, D, false>), dim3(blocks), dim3(64 * kPpWavesOf<D>), 0, stream, args);
+  return hipGetLastError();
+}
+
+// Merge pass of a split call: one workgroup per 32 rows (a wave's slot of a block) and 32 dims, wave g
+// the four-dim groups 8 g .. + 7 of them. With M = max_s m_s, o = sum_s o_s 2^(m_s - M) / sum_s l_s
+// 2^(m_s - M), the splits in order, so the result is the same on every run. Splits in which a row
+// sees no key (m = -inf) contribute nothing. Bound by latency, so the first kFirst partials of a lane
+// are in flight before the maxima are read.
+constexpr int kMergeWaves = 4;
+template <typename Tag, int D>
+__global__ void __launch_bounds__(64 * kMergeWaves) prefill_merge_kernel(const PrefillArgs a) {
+  using E = Elem<Tag>;
+  constexpr int kSlots = kPpWavesOf<D>;
+  constexpr int kFirst = 8;
+  const int lane = threadIdx.x & 63;
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = blockIdx.x % (D / 32);
+  const int wave = blockIdx.x / (D / 32) % kSlots;
+  const int block = blockIdx.x / (D / 32 * kSlots);  // (batch, work head, block of rows)
+  const int bh = block / a.q_blocks;
+  const int row0 = (block - bh * a.q_blocks) * kPpBlockMOf<D> + wave * kRowsPerWave;
+  if (row0 >= a.rows) return;
+  const int n = a.num_splits;
+  const int64_t slot0 = static_cast<int64_t>(block) * n * kSlots + wave;
+  constexpr int64_t kStep = kSlots * (D / 8 * 64);  // float4s from one split to the next
+  const f32x4* po = reinterpret_cast<const f32x4*>(a.partial_o) + slot0 * (D / 8 * 64) + (4 * nb + g) * 64 + lane;
+  const f32pair* ml = a.partial_ml + slot0 * kRowsPerWave + (lane & 31);
+  f32x4 first[kFirst];
+  f32pair first_ml[kFirst];
+#pragma unroll
+  for (int s = 0; s < kFirst; ++s) {
+    first[s] = s < n ? po[s * kStep] : f32x4{};
+    first_ml[s] = s < n ? ml[s * kSlots * kRowsPerWave] : f32pair{-INFINITY, 0.f};
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int s = 0; s < kFirst; ++s) m = fmaxf(m, first_ml[s].x);
+  for (int s = kFirst; s < n; ++s) m = fmaxf(m, ml[s * kSlots * kRowsPerWave].x);
+  float l = 0.f;
+  f32x4 o = {};
+  auto add = [&](const f32x4& o_s, const f32pair& ml_s) {
+    const float f = ml_s.x == -INFINITY ? 0.f : exp2_fast(ml_s.x - m);
+    l += ml_s.y * f;
+    o += o_s * f;
+  };
+#pragma unroll
+  for (int s = 0; s < kFirst; ++s) add(first[s], first_ml[s]);
+#pragma unroll 4
+  for (int s = kFirst; s < n; ++s) add(po[s * kStep], ml[s * kSlots * kRowsPerWave]);
+  const int row = row0 + (lane & 31);
+  if (row >= a.rows) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int b = bh / a.work_heads;
+  const int pos = pack_position(a, row);
+  const int h = (bh - b * a.work_heads) * a.pack + row - pos * a.pack;
+  uint16_t* orow = a.o + b * a.o_bs + pos * a.o_ss + h * a.o_hs + 32 * nb + 8 * g + 4 * (lane >> 5);
+  *reinterpret_cast<u32x2*>(orow) = u32x2{E::pack2(o[0] * inv, o[1] * inv), E::pack2(o[2] * inv, o[3] * inv)};
+  if (nb == 0 && g == 0 && lane < 32)
+    a.lse[(static_cast<int64_t>(b) * a.heads + h) * a.seqlen_q + pos] =
+        l > 0.f ? m * kLn2 + logf(l) : -INFINITY;
+}
+
+template <typename Tag, int D>
+hipError_t launch_split_typed(PrefillArgs args, hipStream_t stream) {
+  args.q_blocks = (args.rows + kPpBlockMOf<D> - 1) / kPpBlockMOf<D>;
+  const int blocks = args.q_blocks * args.batch * args.work_heads;
+  hipLaunchKernelGGL((prefill_pp_kernel<Tag, D, true>), dim3(blocks * args.num_splits),
+                     dim3(64 * kPpWavesOf<D>), 0, stream, args);
+  if (hipError_t err = hipGetLastError()) return err;
+  hipLaunchKernelGGL((prefill_merge_kernel<Tag, D>), dim3(blocks * kPpWavesOf<D> * (D / 32)),
+                     dim3(64 * kMergeWaves), 0, stream, args);
   return hipGetLastError();
 }
 
@@ -717,6 +839,71 @@ hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
 
 int prefill_pp_block_rows(int head_dim) {
   return head_dim == 64 ? prefill::pp::kPpBlockMOf<64> : prefill::pp::kPpBlockMOf<128>;
+}
+
+// Key splits that give the shortest time by a model fitted to device times (us; B, H, H_kv, S_q, S_k,
+// D; causal, bf16): a 64-key tile of a block takes 1.1 us, 0.8 where only one group of waves has rows,
+// and up to 0.3 more as the CUs fill; a block's start and end 5, the second launch and the merge 6,
+// and the partials 0.45 per MB to memory and back. Measured without splits / at the planned count:
+// (1, 32, 8, 300, 8492, 128) 147 / 49, (1, 32, 8, 16, 8192, 128) 138 / 20, (1, 32, 8, 512, 4096, 128)
+// 72 / 44, (1, 64, 8, 18, 1212, 128) 23 / 15, (1, 8, 8, 5000, 5000, 64) 68 / 48; calls whose blocks
+// fill the CUs gain nothing ((1, 32, 8, 2048, 2048, 128) 49, 60 with two splits), nor do short ones
+// ((1, 32, 8, 512, 512, 128) 14, 24 with two).
+int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count) {
+  if (knob(FL_KNOB_PREFILL_PP_MIN_WG) >= 0 || knob(FL_KNOB_PREFILL_CAUSAL_STREAM) >= 0) return 1;
+  const int cus = cu_count > 0 ? cu_count : 256;
+  const int block_rows = prefill_pp_block_rows(head_dim);
+  const int64_t q_blocks = (args.rows + block_rows - 1) / block_rows;
+  const int64_t blocks = q_blocks * args.batch * args.work_heads;
+  if (blocks >= 2 * cus) return 1;
+  // Tiles of the longest block and of the average one.
+  const double longest = (args.seqlen_k + kPrefillBlockN - 1) / kPrefillBlockN;
+  double mean = longest;
+  if (args.causal) {
+    const double first = args.causal_offset + (q_blocks > 1 ? double(block_rows) / args.pack : args.seqlen_q);
+    mean = (longest + (first > 0 ? first / kPrefillBlockN : 0)) / 2;
+  }
+  const int rows = args.rows < block_rows ? (args.rows + 31) / 32 * 32 : block_rows;
+  const double mb = 4e-6 * blocks * rows * head_dim;  // one split's partials
+  auto time = [&](int n) {
+    const double wgs = static_cast<double>(blocks) * n;
+    const double tile = (rows <= 128 ? 0.8 : 1.1) + 0.3 * (wgs < cus ? wgs / cus : 1.0);
+    const double alone = longest / n * tile + 5.0;
+    const double all = (blocks * n + cus - 1) / cus * (mean / n * tile + 5.0);
+    return (alone > all ? alone : all) + (n == 1 ? 3.0 : 6.0 + 0.1 * n + 0.45 * n * mb);
+  };
+  // Without splits: this kernel, or the 4-wave one on blocks of 128 rows, one or two to a CU.
+  const double small_wgs =
+      double((args.seqlen_q + kPrefillBlockM - 1) / kPrefillBlockM) * args.batch * args.heads * mean / longest;
+  const double small = 4.0 + 1.1 * longest * (small_wgs > cus ? small_wgs / cus : 1.0);
+  double least = 0.95 * (small < time(1) ? small : time(1));
+  int best = 1;
+  for (int n = 2; n <= kMaxPrefillSplits && n <= longest; ++n) {
+    if (time(n) < least) {
+      best = n;
+      least = time(n);
+    }
+  }
+  return best;
+}
+
+int64_t prefill_partial_floats(const PrefillArgs& args, int head_dim, int num_splits, int64_t* ml_offset) {
+  const int block_rows = prefill_pp_block_rows(head_dim);
+  const int64_t q_blocks = (args.rows + block_rows - 1) / block_rows;
+  const int64_t rows = q_blocks * block_rows * args.batch * args.work_heads * num_splits;
+  *ml_offset = rows * head_dim;
+  return rows * (head_dim + 2);
+}
+
+hipError_t launch_prefill_split(const PrefillArgs& args, DType dtype, int head_dim, hipStream_t stream) {
+  using namespace prefill::pp;
+  if (head_dim == 64) {
+    return dtype == DType::bf16 ? launch_split_typed<bf16_tag, 64>(args, stream)
+                                : launch_split_typed<f16_tag, 64>(args, stream);
+  }
+  if (head_dim != 128) return hipErrorInvalidValue;
+  return dtype == DType::bf16 ? launch_split_typed<bf16_tag, 128>(args, stream)
+                              : launch_split_typed<f16_tag, 128>(args, stream);
 }
 
 hipError_t launch_prefill_pingpong(const PrefillArgs& args, DType dtype, int head_dim,

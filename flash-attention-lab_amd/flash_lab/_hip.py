@@ -33,6 +33,8 @@ import torch
 LIB_NAME = "libflash_lab_hip.so"
 LIB_PATH = Path(os.environ.get("FLASH_LAB_HIP_LIB", Path(__file__).with_name(LIB_NAME)))
 
+ERR_WORKSPACE = 4  # enum fl_status
+
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
@@ -102,6 +104,27 @@ class DecodeParams(ctypes.Structure):
 # Every symbol include/flash_lab_hip.h declares, with its ctypes signature.
 SIGNATURES = {
     "fl_attention_fwd": (ctypes.c_int, [ctypes.POINTER(AttnParams), ctypes.c_void_p]),
+    "fl_attention_plan": (
+        ctypes.c_int,
+        [
+            ctypes.POINTER(AttnParams),
+            ctypes.c_int32,
+            ctypes.c_int32,
+            ctypes.POINTER(ctypes.c_int32),
+            ctypes.POINTER(ctypes.c_size_t),
+        ],
+    ),
+    "fl_attention_fwd_split": (
+        ctypes.c_int,
+        [
+            ctypes.POINTER(AttnParams),
+            ctypes.c_int32,
+            ctypes.c_int32,
+            ctypes.c_void_p,
+            ctypes.c_size_t,
+            ctypes.c_void_p,
+        ],
+    ),
     "fl_decode_plan": (
         ctypes.c_int,
         [
@@ -239,9 +262,10 @@ def _check_cuda(**tensors: torch.Tensor) -> None:
 # Prefill
 
 
-def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, softmax_scale: float):
-    """Op-boundary checks of the reference (csrc/common/attn_host.h:18-57), output allocation,
-    and the fl_attention_fwd call."""
+def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, softmax_scale: float,
+            num_splits: int = 0):
+    """Op-boundary checks of the reference (csrc/common/attn_host.h:18-57), output and workspace
+    allocation, and fl_attention_fwd_split (num_splits 0: the library's choice)."""
     _check_cuda(q=q, k=k, v=v)
     _require(q.dtype in (torch.bfloat16, torch.float16), "attention_mma_pipelined takes bf16 or fp16")
     _require(k.dtype == q.dtype and v.dtype == q.dtype, "k and v must have dtype %s", q.dtype)
@@ -283,8 +307,21 @@ def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, sof
         DTYPE_CODES[q.dtype],
         float(softmax_scale),
     )
+    index = q.device.index if q.device.index is not None else torch.cuda.current_device()
+    cus = cu_count(index)
     with _on_device(q.device):
-        _check(LIB.fl_attention_fwd(ctypes.byref(p), _stream(q.device)))
+        stream = _stream(q.device)
+        if num_splits == 0:
+            rc = LIB.fl_attention_fwd_split(ctypes.byref(p), 0, cus, None, 0, stream)
+            if rc != ERR_WORKSPACE:
+                _check(rc)
+                return o, lse
+        splits, ws_bytes = ctypes.c_int32(), ctypes.c_size_t()
+        _check(LIB.fl_attention_plan(ctypes.byref(p), num_splits, cus, ctypes.byref(splits),
+                                     ctypes.byref(ws_bytes)))
+        workspace = torch.empty(ws_bytes.value // 4, dtype=torch.float32, device=q.device)
+        _check(LIB.fl_attention_fwd_split(ctypes.byref(p), splits.value, cus, workspace.data_ptr(),
+                                          ws_bytes.value, stream))
     return o, lse
 
 

@@ -34,7 +34,8 @@ enum fl_status {
   FL_OK = 0,
   FL_ERR_INVALID = 1,     /* bad argument: shape, stride, alignment, dtype */
   FL_ERR_UNSUPPORTED = 2, /* valid, but no kernel is built for it (head_dim, dtype) */
-  FL_ERR_LAUNCH = 3       /* the HIP runtime reported an error at launch */
+  FL_ERR_LAUNCH = 3,      /* the HIP runtime reported an error at launch */
+  FL_ERR_WORKSPACE = 4    /* fl_attention_fwd_split with num_splits 0 needs a (larger) workspace */
 };
 
 /*
@@ -68,6 +69,28 @@ typedef struct fl_attn_params {
  * csrc/prefill/mma.cu), head_dim 64 or 128, bf16 or fp16.
  */
 int fl_attention_fwd(const fl_attn_params* p, fl_stream_t stream);
+
+/*
+ * Key splits and workspace size for a prefill call; host-only, touches no device, reads only the
+ * sizes, causal and dtype. No counterpart in the reference. A call with few query rows and many
+ * keys (new tokens after a cached prefix, a long prompt of one sequence with few heads) leaves most
+ * CUs idle; num_splits > 1 then gives each block of rows that many workgroups, each on its share of
+ * the keys, and a merge pass. requested_splits 0 lets the library choose for cu_count (1, and
+ * *workspace_bytes 0, where splitting does not pay); a requested count is in [1, 64].
+ */
+int fl_attention_plan(const fl_attn_params* p, int32_t requested_splits, int32_t cu_count,
+                      int32_t* num_splits, size_t* workspace_bytes);
+
+/*
+ * fl_attention_fwd with num_splits key splits, resolved by fl_attention_plan, or 0: the count that
+ * fl_attention_plan would choose for cu_count. If that count needs a larger workspace than given,
+ * nothing is launched and the call returns FL_ERR_WORKSPACE, so that a caller can try without one
+ * (most calls need none) and allocate it only when asked to. workspace is 16-byte aligned fp32 device memory of at least the size fl_attention_plan
+ * reports for that count (unused, may be NULL, when num_splits == 1). The splits are merged in a
+ * fixed order: results are bitwise reproducible for a given split count.
+ */
+int fl_attention_fwd_split(const fl_attn_params* p, int32_t num_splits, int32_t cu_count,
+                           float* workspace, size_t workspace_bytes, fl_stream_t stream);
 
 /*
  * Decode. Replaces DecodeParams (reference csrc/common/params.h:31-53) as
