@@ -161,6 +161,62 @@ int mfma_span_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, 
   return mfma_span(p, layout, n) == kMfmaSpan ? n : 0;
 }
 
+// Balanced calls (decode_sched.hpp) on `wgs` workgroups: KV heads per workgroup (as in the split forms:
+// the widest span that leaves a workgroup 512 keys of its KV heads, 1,024 on the matrix-core kernel),
+// keys per unit and what one more segment costs a workgroup, in units (a segment's start is about
+// 2.5 us, in which a CU streams about 64 KiB). At most kMaxBalancedBatch sequences, a line within
+// 2^22 units, and, paged, segments whose block numbers fit LDS whatever the lengths are.
+struct BalancedLayout {
+  bool fits;
+  int span, unit_shift, min_units, ramp_units;
+  int64_t rows;  // work heads of all sequences
+};
+BalancedLayout balanced_layout(const fl_decode_params* p, const fl::DecodeLayout& layout, int wgs) {
+  const int64_t chunks = layout.mfma ? 1 : p->heads / p->heads_kv / layout.heads_per_wg;
+  const int64_t keys_per_wg = layout.mfma ? kMfmaSpanSplitKeys : 512;
+  BalancedLayout r{};
+  const int forced = layout.mfma ? fl::knob(FL_KNOB_DECODE_MFMA_SPAN) : -1;
+  for (r.span = layout.mfma ? kMfmaSpan : layout.kv_span; r.span > 1; r.span /= 2) {
+    if (p->heads_kv % r.span != 0 || (layout.mfma && r.span != kMfmaSpan) || forced == 1) continue;
+    const double keys = double(p->batch) * (p->heads_kv / r.span) * chunks * p->max_seqlen;
+    if (forced == r.span || keys >= double(keys_per_wg) * wgs) break;
+  }
+  r.unit_shift = 5;
+  r.min_units = 4;
+  r.ramp_units = layout.mfma ? (r.span == 1 ? 4 : 1) : 2;
+  r.rows = p->batch * (p->heads_kv / r.span) * chunks;
+  const int64_t longest = (int64_t{p->max_seqlen} + (1 << r.unit_shift) - 1) >> r.unit_shift;
+  const int64_t units = r.rows * (longest + r.ramp_units);
+  const int64_t chunk = (units + wgs - 1) / wgs + r.min_units;
+  const int64_t keys = (chunk < longest ? chunk : longest) << r.unit_shift;
+  r.fits = p->batch <= fl::kMaxBalancedBatch && units + (r.rows + 2) * chunk + wgs < (int64_t{1} << 22) &&
+           (p->block_tables == nullptr || keys / p->page_size + 2 <= fl::kMaxSplitPages);
+  return r;
+}
+
+// Partials (one head's D floats, maximum and sum) of a balanced call: kRowSlots slots per row, and an
+// overflow slot per workgroup and row.
+size_t balanced_partials(const fl_decode_params* p, const BalancedLayout& layout, int wgs) {
+  return (wgs + static_cast<size_t>(layout.rows) * (fl::kRowSlots + 1)) *
+         (static_cast<size_t>(p->batch) * p->heads / layout.rows);
+}
+
+// Whether a call that could be balanced is. The host does not know the lengths, so what equal ones
+// lose counts too: deriving the schedule takes a workgroup about 1.5 us before its first load, and a
+// fixed plan of one split needs no merge pass. So it takes several sequences and a cache that the CUs
+// stream for some 40 us (1 MiB each). A paged cache holds unequal sequences in most uses, and its
+// fixed plan leaves most of the time to the longest one; a contiguous cache often holds equal ones,
+// and there only the vector kernel with one query head gains more than it may lose. Device us, fixed
+// / balanced, bf16, D = 128, lengths spread evenly up to the longest (and all equal to it): paged (24,
+// 32, 8, 8000) 129 / 79 (150 / 136), (8, 32, 8, 32768) 140 / 109 (173 / 176), (64, 32, 8, 2048) 74 / 62
+// (93 / 95); contiguous (8, 32, 32, 8192) 124 / 96 (161 / 161). Smaller: paged (4, 32, 8, 8192) equal
+// 31 / 33, (32, 32, 8, 500) 15 / 24.
+bool worth_balancing(const fl_decode_params* p, const fl::DecodeLayout& layout, int num_splits, int cus) {
+  const double bytes = 2.0 * p->batch * p->heads_kv * p->max_seqlen * p->head_dim * elem_bytes(p->dtype);
+  if (p->batch < 6 || bytes < 1048576.0 * cus) return false;
+  return p->block_tables != nullptr || (!layout.mfma && layout.heads_per_wg == 1 && num_splits > 1);
+}
+
 int check_decode_shape(const fl_decode_params* p) {
   if (p == nullptr) return fail(FL_ERR_INVALID, "null decode parameters");
   if (p->block_tables != nullptr && (p->page_size <= 0 || p->num_blocks <= 0))
@@ -187,13 +243,13 @@ namespace {
 // Checks, parameter derivation and launch of a decode call whose split workspace (used when
 // num_splits > 1) is `workspace`, `workspace_bytes` long: the caller's (fl_decode) or the
 // library's scratch array (fl_decode_noalloc).
-int decode_call(const fl_decode_params* p, float* workspace, size_t workspace_bytes,
+int decode_call(const fl_decode_params* p, int balanced_wgs, float* workspace, size_t workspace_bytes,
                 fl_stream_t stream) {
   if (int rc = check_decode_shape(p)) return rc;
   if (!p->q || !p->k_cache || !p->v_cache || !p->o || !p->lse || !p->seq_lens)
     return fail(FL_ERR_INVALID, "null tensor pointer");
   if (!valid_scale(p->softmax_scale)) return fail(FL_ERR_INVALID, "softmax_scale must be positive");
-  if (p->num_splits < 1 || p->num_splits > fl::kMaxSplits)
+  if (balanced_wgs == 0 && (p->num_splits < 1 || p->num_splits > fl::kMaxSplits))
     return fail(FL_ERR_INVALID, "num_splits must be in [1, 128]");
   const int eb = elem_bytes(p->dtype);
   if (!rows_16_byte(p->q, eb, p->batch, p->q_batch_stride, p->heads, p->q_head_stride, 1, 0))
@@ -216,7 +272,8 @@ int decode_call(const fl_decode_params* p, float* workspace, size_t workspace_by
   const fl::DType dt = decode_dtype(p->dtype);
   const fl::DecodeLayout layout = fl::decode_layout(dt, p->head_dim, p->heads_kv, group);
   const int head_chunks = group / layout.heads_per_wg;
-  const int64_t blocks = static_cast<int64_t>(p->batch) * p->heads_kv * head_chunks * p->num_splits;
+  const int num_splits = balanced_wgs > 0 ? 0 : p->num_splits;
+  const int64_t blocks = static_cast<int64_t>(p->batch) * p->heads_kv * head_chunks * num_splits;
   if (blocks > (int64_t{1} << 24) || static_cast<int64_t>(p->batch) * p->heads > (int64_t{1} << 24))
     return fail(FL_ERR_INVALID, "batch * heads too large");
 
@@ -242,31 +299,46 @@ int decode_call(const fl_decode_params* p, float* workspace, size_t workspace_by
   a.heads_kv = p->heads_kv;
   a.group = group;
   a.max_seqlen = p->max_seqlen;
-  a.num_splits = p->num_splits;
+  a.num_splits = num_splits;
   a.head_chunks = head_chunks;
-  a.kv_span = decode_span(p, layout, p->num_splits);
   a.mfma = layout.mfma;
-  a.mfma_span = mfma_span(p, layout, p->num_splits);
   a.block_tables = p->block_tables;
   a.block_tables_stride = p->block_tables_stride;
   a.page_size = p->page_size;
   a.num_blocks = p->num_blocks;
-  a.page_table_global =
-      p->block_tables != nullptr &&
-      pages_per_split(p->max_seqlen, p->num_splits, p->page_size) > fl::kMaxSplitPages;
-  if (a.page_table_global) a.kv_span = 1;
+  if (balanced_wgs > 0) {
+    const BalancedLayout balanced = balanced_layout(p, layout, balanced_wgs);
+    if (!balanced.fits)
+      return fail(FL_ERR_INVALID, "this call has no balanced schedule (fl_decode_schedule reports none)");
+    a.balanced_wgs = balanced_wgs;
+    a.kv_span = a.mfma_span = balanced.span;
+    a.unit_shift = balanced.unit_shift;
+    a.min_units = balanced.min_units;
+    a.ramp_units = balanced.ramp_units;
+  } else {
+    a.kv_span = decode_span(p, layout, num_splits);
+    a.mfma_span = mfma_span(p, layout, num_splits);
+    a.page_table_global =
+        p->block_tables != nullptr &&
+        pages_per_split(p->max_seqlen, num_splits, p->page_size) > fl::kMaxSplitPages;
+    if (a.page_table_global) a.kv_span = 1;
+  }
   a.page_shift = -1;
   for (int s = 0; s < 31; ++s)
     if (p->page_size == (1 << s)) a.page_shift = s;
   a.scale_log2 = static_cast<float>(p->softmax_scale * 1.4426950408889634);
-  if (p->num_splits > 1) {
-    const size_t need =
-        static_cast<size_t>(p->batch) * p->heads * p->num_splits * (p->head_dim + 2) * sizeof(float);
-    if (workspace == nullptr || workspace_bytes < need)
-      return fail(FL_ERR_INVALID, "decode workspace is missing or smaller than fl_decode_plan reports");
+  if (num_splits != 1) {
+    const size_t partials = balanced_wgs > 0
+                                ? balanced_partials(p, balanced_layout(p, layout, balanced_wgs), balanced_wgs)
+                                : static_cast<size_t>(p->batch) * p->heads * num_splits;
+    const size_t rows = balanced_wgs > 0 ? balanced_layout(p, layout, balanced_wgs).rows : 0;
+    if (workspace == nullptr ||
+        workspace_bytes < partials * (p->head_dim + 2) * sizeof(float) + rows * sizeof(int2))
+      return fail(FL_ERR_INVALID, "decode workspace is missing or smaller than the plan reports");
     if (!aligned(workspace, 16)) return fail(FL_ERR_INVALID, "decode workspace must be 16-byte aligned");
     a.partial_o = workspace;
-    a.partial_ml = workspace + static_cast<size_t>(p->batch) * p->heads * p->num_splits * p->head_dim;
+    a.partial_ml = workspace + partials * p->head_dim;
+    a.row_slots = reinterpret_cast<int2*>(a.partial_ml + 2 * partials);
   }
   const hipError_t err = fl::launch_decode(a, dt, p->head_dim, static_cast<hipStream_t>(stream));
   if (err != hipSuccess) return fail(FL_ERR_LAUNCH, std::string("decode launch: ") + hipGetErrorString(err));
@@ -535,9 +607,44 @@ int fl_decode_plan(const fl_decode_params* p, int32_t requested_splits, int32_t 
   return FL_OK;
 }
 
+int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num_splits,
+                       int32_t* workgroups, size_t* workspace_bytes) {
+  if (workgroups == nullptr) return fail(FL_ERR_INVALID, "null output pointer");
+  if (int rc = fl_decode_plan(p, 0, 1, cu_count, num_splits, workspace_bytes)) return rc;
+  *workgroups = 0;
+  const fl::DecodeLayout layout =
+      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, p->heads / p->heads_kv);
+  // Short caches: one workgroup per KV head and no merge pass, while the keys that more workgroups
+  // would take off it cost less than the pass (about 3.9 us, against 11.5 us per 1,000 keys): (B, H,
+  // H_kv, S) (16, 32, 8, 320) 10.3 us with one split, 11.9 with two, (2, 8, 8, 90) 3.8 and 6.3, (4, 32,
+  // 8, 640) 13.2 and 9.6 with eight.
+  const double fill = double(p->batch) * p->heads_kv / (cu_count > 0 ? cu_count : 256);
+  if (p->max_seqlen < 640 && p->max_seqlen * (fill < 1.0 ? 1.0 - fill : 0.0) < 340.0) {
+    *num_splits = 1;
+    *workspace_bytes = 0;
+    return FL_OK;
+  }
+  if (!worth_balancing(p, layout, *num_splits, cu_count > 0 ? cu_count : 256)) return FL_OK;
+  const int64_t wgs = resident_capacity(cu_count, planned_per_cu(p, layout));
+  const BalancedLayout balanced = balanced_layout(p, layout, static_cast<int>(wgs));
+  if (!balanced.fits) return FL_OK;
+  *num_splits = 0;
+  *workgroups = static_cast<int32_t>(wgs);
+  *workspace_bytes = balanced_partials(p, balanced, static_cast<int>(wgs)) * (p->head_dim + 2) * sizeof(float) +
+                     balanced.rows * sizeof(int2);
+  return FL_OK;
+}
+
+int fl_decode_balanced(const fl_decode_params* p, int32_t workgroups, fl_stream_t stream) {
+  if (p == nullptr) return fail(FL_ERR_INVALID, "null decode parameters");
+  if (workgroups < 1 || workgroups > (1 << 16))
+    return fail(FL_ERR_INVALID, "workgroups must be in [1, 65536]");
+  return decode_call(p, workgroups, p->workspace, p->workspace_bytes, stream);
+}
+
 int fl_decode(const fl_decode_params* p, fl_stream_t stream) {
   if (p == nullptr) return fail(FL_ERR_INVALID, "null decode parameters");
-  return decode_call(p, p->workspace, p->workspace_bytes, stream);
+  return decode_call(p, 0, p->workspace, p->workspace_bytes, stream);
 }
 
 int fl_decode_noalloc(const fl_decode_params* p, fl_stream_t stream) {
@@ -554,7 +661,7 @@ int fl_decode_noalloc(const fl_decode_params* p, fl_stream_t stream) {
                       static_cast<long long>(need)));
     if (int rc = scratch_for_current_device(&ws)) return rc;
   }
-  return decode_call(p, ws, kScratchBytes, stream);
+  return decode_call(p, 0, ws, kScratchBytes, stream);
 }
 
 int fl_smoke_axpy(const float* x, const float* y, float alpha, float* out, int64_t n,

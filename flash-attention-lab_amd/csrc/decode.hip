@@ -28,6 +28,7 @@
 //    workgroup then has to wait for its partials to reach device scope and for an atomic before it
 //    frees its slot, which costs more than the second launch.)
 
+#include "decode_sched.hpp"
 #include "gfx950.hpp"
 #include "launch.hpp"
 
@@ -127,7 +128,17 @@ struct MergeShape {
   static_assert(kVecs <= kThreads && kThreads % kVecs == 0, "one thread per vector and part");
 };
 
-// Combines the splits of the kHeads consecutive query heads h0 .. h0 + kHeads - 1 of sequence b:
+// Where the partials of a head group are: split s of head g (of the group) at index first + g head_step
+// + s split_step of partial_o and partial_ml. In a balanced call that holds for s < kRowSlots, with
+// `over` in place of first from there on, and the number of splits comes from memory: the first
+// kRowSlots partials (written or not) are loaded before it is known.
+struct Partials {
+  int64_t first, over;
+  int head_step, split_step;
+};
+
+// Combines the splits of the kHeads consecutive query heads h0 .. h0 + kHeads - 1 of sequence b;
+// splits() gives their number n:
 // m = max_s m_s, l = sum_s l_s 2^(m_s - m), o = sum_s o_s 2^(m_s - m) / l, lse = m ln 2 + ln l;
 // empty splits (m_s = -inf) contribute nothing. All threads of the workgroup take part. Thread t
 // owns one 4-column output vector (t % kVecs) and the splits p, p + kParts, ... (p = t / kVecs), so
@@ -136,8 +147,9 @@ struct MergeShape {
 // latency-bound: the first kFirst partial-output loads of each thread do not depend on the maxima
 // and are issued before the (max, sum) pairs are read, so the two loads overlap.
 // `lds` must hold MergeShape::kFloats floats, 16-byte aligned.
-template <typename Tag, int D, int kHeads>
-__device__ __forceinline__ void merge_splits(const DecodeArgs& a, int b, int h0, float* lds) {
+template <typename Tag, int D, int kHeads, bool kBalanced, typename Count>
+__device__ __forceinline__ void merge_splits(const DecodeArgs& a, int b, int h0, const Partials& at,
+                                             Count&& splits, float* lds) {
   using S = typename Elem<Tag>::storage;
   using Shape = MergeShape<kHeads, D>;
   constexpr int kVecs = Shape::kVecs;
@@ -145,53 +157,82 @@ __device__ __forceinline__ void merge_splits(const DecodeArgs& a, int b, int h0,
   constexpr int kVecsPerRow = D / 4;
   constexpr int kFirst = 8;
   const int tid = threadIdx.x;
-  const int n = a.num_splits;
-  const int n4 = (n + 3) & ~3;
-  float* ms = lds;                        // [kHeads][kMaxSplits], -inf past n up to n4
+  float* ms = lds;                        // [kHeads][kMaxSplits]
   float* ls = lds + kHeads * kMaxSplits;  // [kHeads][kMaxSplits]
   const int vec = tid % kVecs;
   const int part = tid / kVecs;
   const int g = vec / kVecsPerRow;
-  // Slots of the heads are consecutive: slot(g, s) = (b H + h0) n + g n + s.
-  const int64_t slot0 = (static_cast<int64_t>(b) * a.heads + h0) * n;
-  const f32x4* po =
-      reinterpret_cast<const f32x4*>(a.partial_o + (slot0 + g * n) * D) + vec % kVecsPerRow;
+  auto index = [&](int gi, int s) {
+    const int64_t base = !kBalanced || s < kRowSlots ? at.first : at.over;
+    return base + gi * at.head_step + static_cast<int64_t>(s) * at.split_step;
+  };
+  auto po = [&](int s) -> const f32x4& {
+    return reinterpret_cast<const f32x4*>(a.partial_o + index(g, s) * D)[vec % kVecsPerRow];
+  };
+  const int known = kBalanced ? kRowSlots : splits();
   f32x4 first[kFirst];
 #pragma unroll
   for (int j = 0; j < kFirst; ++j) {
     const int s = part + j * kParts;
-    first[j] = s < n ? po[s * kVecsPerRow] : f32x4{0.f, 0.f, 0.f, 0.f};
+    first[j] = s < known ? po(s) : f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  for (int i = tid; i < kHeads * n4; i += kThreads) {
-    const int gi = i / n4;
-    const int s = i - gi * n4;
-    f32x2 ml = {-INFINITY, 0.f};
-    if (s < n) ml = *reinterpret_cast<const f32x2*>(a.partial_ml + 2 * (slot0 + gi * n + s));
-    ms[gi * kMaxSplits + s] = ml[0];
-    ls[gi * kMaxSplits + s] = ml[1];
-  }
-  __syncthreads();
+  // The (max, sum) pairs of splits base + from .. base + to - 1.
+  auto stage = [&](int base, int from, int to) {
+    const int width = to - from;
+    for (int i = tid; i < kHeads * width; i += kThreads) {
+      const int gi = i / width;
+      const int s = from + i - gi * width;
+      const f32x2 ml = *reinterpret_cast<const f32x2*>(a.partial_ml + 2 * index(gi, base + s));
+      ms[gi * kMaxSplits + s] = ml[0];
+      ls[gi * kMaxSplits + s] = ml[1];
+    }
+  };
+  stage(0, 0, known);
+  const int n = kBalanced ? splits() : known;
   float mm = -INFINITY;
-  const f32x4* ms4 = reinterpret_cast<const f32x4*>(ms + g * kMaxSplits);
-  for (int s4 = 0; s4 < n4 / 4; ++s4) {
-    const f32x4 v = ms4[s4];
-    mm = fmaxf(mm, fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
-  }
   f32x4 num = {0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
-  auto add = [&](int s, const f32x4& o_s) {
-    const float m_s = ms[g * kMaxSplits + s];
-    const float f = m_s == -INFINITY ? 0.f : exp2_fast(m_s - mm);
-    den += ls[g * kMaxSplits + s] * f;
-    num += o_s * f;
-  };
+  // kMaxSplits splits at a time (only a balanced call has more).
+  for (int base = 0; base < n; base += kMaxSplits) {
+    const int count = kBalanced ? min(n - base, kMaxSplits) : n;
+    if constexpr (kBalanced) {
+      if (base > 0) __syncthreads();
+      const int staged = base == 0 ? known : 0;
+      if (count > staged) stage(base, staged, count);
+    }
+    __syncthreads();
+    float top = mm;
+    const f32x4* ms4 = reinterpret_cast<const f32x4*>(ms + g * kMaxSplits);
+    int s4 = 0;
+    for (; s4 < count / 4; ++s4) {
+      const f32x4 v = ms4[s4];
+      top = fmaxf(top, fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+    }
+    for (int s = 4 * s4; s < count; ++s) top = fmaxf(top, ms[g * kMaxSplits + s]);
+    if (kBalanced && base > 0) {
+      const float f = mm == -INFINITY ? 0.f : exp2_fast(mm - top);
+      num *= f;
+      den *= f;
+    }
+    mm = top;
+    auto add = [&](int s, const f32x4& o_s) {
+      const float m_s = ms[g * kMaxSplits + s];
+      const float f = m_s == -INFINITY ? 0.f : exp2_fast(m_s - mm);
+      den += ls[g * kMaxSplits + s] * f;
+      num += o_s * f;
+    };
+    if (base == 0) {
 #pragma unroll
-  for (int j = 0; j < kFirst; ++j) {
-    const int s = part + j * kParts;
-    if (s < n) add(s, first[j]);
-  }
+      for (int j = 0; j < kFirst; ++j) {
+        const int s = part + j * kParts;
+        if (s < count) add(s, !kBalanced || s < known ? first[j] : po(s));
+      }
+    }
 #pragma unroll 8
-  for (int s = part + kFirst * kParts; s < n; s += kParts) add(s, po[s * kVecsPerRow]);
+    for (int s = part + (base == 0 ? kFirst * kParts : 0); s < count; s += kParts)
+      add(s, po(base + s));
+    if constexpr (!kBalanced) break;
+  }
   if constexpr (kParts > 1) {
     f32x4* part_o = reinterpret_cast<f32x4*>(lds + 2 * kHeads * kMaxSplits);  // [kParts][kVecs]
     float* part_l = reinterpret_cast<float*>(part_o + kThreads);              // [kParts][kVecs]
@@ -222,7 +263,7 @@ __device__ __forceinline__ void merge_splits(const DecodeArgs& a, int b, int h0,
 template <int kHeads>
 constexpr int kWavesPerSimd = kHeads == 1 ? 5 : kHeads <= 4 ? 3 : 2;
 
-template <typename Tag, int D, int kHeads, int kSpan, int kPageMode>
+template <typename Tag, int D, int kHeads, int kSpan, int kPageMode, bool kBalanced>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kWavesPerSimd<kHeads>)))
 decode_split_kernel(const DecodeArgs a) {
   constexpr bool kPaged = kPageMode != kContiguous;
@@ -247,26 +288,55 @@ decode_split_kernel(const DecodeArgs a) {
   const int sp = (lane / kLPR) % kSpan;            // which KV head of the workgroup's span
   const int group = wave * kGPW + lane / kLPK;     // row group within the workgroup
 
-  int w = blockIdx.x;
-  const int split = w % a.num_splits;
-  w /= a.num_splits;
-  const int hchunk = w % a.head_chunks;
-  w /= a.head_chunks;
   const int hblocks = a.heads_kv / kSpan;
-  const int hblk = w % hblocks;
-  const int b = w / hblocks;
+  const int rows = hblocks * a.head_chunks;  // work heads per sequence
+  using P = Piece<Tag>;
+
+  // A workgroup runs one segment, a key range of one work head: its split of a sequence, or, in a
+  // balanced call, each row segment of its share of the line (decode_sched.hpp).
+  Schedule sched{};
+  int pos = 0;
+  int end = 1;
+  if constexpr (kBalanced) {
+    sched = make_schedule(a, rows);
+    pos = blockIdx.x * sched.chunk;
+    end = min(pos + sched.chunk, sched.total);
+  }
+  while (pos < end) {  // (once, where not balanced)
+  int b, head, k_begin, k_end, head_step;
+  int64_t partial;  // index of the segment's first partial; the next head's is head_step on
+  if constexpr (kBalanced) {
+    const Segment g = segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
+    pos = g.next;
+    if (g.k_begin == g.k_end) continue;
+    b = g.b;
+    head = g.head;
+    k_begin = g.k_begin;
+    k_end = g.k_end;
+    partial = g.slot * (kSpan * kHeads);
+    head_step = 1;
+  } else {
+    pos = end;
+    const int split = blockIdx.x % a.num_splits;
+    const int work = blockIdx.x / a.num_splits;
+    b = work / rows;
+    head = work - b * rows;
+    // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
+    // out-of-range value cannot read outside it.
+    const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
+    const int per_split =
+        ((len + a.num_splits - 1) / a.num_splits + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
+    k_begin = split * per_split;
+    k_end = min(len, k_begin + per_split);
+    partial = (static_cast<int64_t>(b) * a.heads + (head / a.head_chunks * kSpan) * a.group +
+               head % a.head_chunks * kHeads) * a.num_splits + split;
+    head_step = a.num_splits;
+  }
+  const int hblk = head / a.head_chunks;
+  const int hchunk = head - hblk * a.head_chunks;
   const int hkv = hblk * kSpan + sp;
   const int h0 = hkv * a.group + hchunk * kHeads;
 
-  // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
-  // out-of-range value cannot read outside it.
-  const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
-  const int per_split =
-      ((len + a.num_splits - 1) / a.num_splits + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
-  const int k_begin = split * per_split;
-  const int k_end = min(len, k_begin + per_split);
-
-  using P = Piece<Tag>;
   typename P::QPiece q[kHeads];
 #pragma unroll
   for (int g = 0; g < kHeads; ++g) {
@@ -451,7 +521,8 @@ decode_split_kernel(const DecodeArgs a) {
       orow[d] = Elem<Tag>::from_float(den > 0.f ? num / den : 0.f);
       if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
     } else {
-      const int64_t slot = (static_cast<int64_t>(b) * a.heads + h) * a.num_splits + split;
+      const int64_t slot =
+          partial + static_cast<int64_t>(kBalanced ? g : h - hblk * kSpan * a.group - hchunk * kHeads) * head_step;
       a.partial_o[slot * D + d] = num;
       if (d == 0) {
         a.partial_ml[2 * slot] = mm;
@@ -459,10 +530,13 @@ decode_split_kernel(const DecodeArgs a) {
       }
     }
   }
+  if constexpr (!kBalanced) return;
+  if (pos < end) __syncthreads();  // the next segment reuses the merge's LDS
+  }
 }
 
 // Merge pass: one workgroup per head group (kHeads query heads of one KV head).
-template <typename Tag, int D, int kHeads>
+template <typename Tag, int D, int kHeads, bool kBalanced>
 __global__ void __launch_bounds__(kThreads) decode_merge_kernel(const DecodeArgs a) {
   __shared__ __attribute__((aligned(16))) float lds[MergeShape<kHeads, D>::kFloats];
   int w = blockIdx.x;
@@ -470,7 +544,28 @@ __global__ void __launch_bounds__(kThreads) decode_merge_kernel(const DecodeArgs
   w /= a.head_chunks;
   const int hkv = w % a.heads_kv;
   const int b = w / a.heads_kv;
-  merge_splits<Tag, D, kHeads>(a, b, hkv * a.group + hchunk * kHeads, lds);
+  const int h0 = hkv * a.group + hchunk * kHeads;
+  if constexpr (kBalanced) {
+    // The split kernel's work head: a span of KV heads with this chunk of each one's query heads
+    // (vector kernel) or with all of them (matrix-core kernel).
+    const int span = a.mfma ? a.mfma_span : a.kv_span;
+    const int chunks = a.mfma ? 1 : a.head_chunks;
+    const int wg_heads = a.mfma ? span * a.group : span * kHeads;
+    const int rows = a.heads_kv / span * chunks;
+    const int row = b * rows + hkv / span * chunks + (a.mfma ? 0 : hchunk);
+    const int head = hkv % span * (wg_heads / span) + (a.mfma ? hchunk * kHeads : 0);
+    Partials at{row * int64_t{kRowSlots} * wg_heads + head, 0, 1, wg_heads};
+    merge_splits<Tag, D, kHeads, true>(a, b, h0, at, [&] {
+      const int2 slots = a.row_slots[row];
+      const int keys = a.seq_lens[b];
+      at.over = (int64_t{a.batch} * rows * kRowSlots + slots.y) * wg_heads + head;
+      return keys > 0 ? slots.x : 0;
+    }, lds);
+  } else {
+    const int64_t first = (static_cast<int64_t>(b) * a.heads + h0) * a.num_splits;
+    const int n = a.num_splits;
+    merge_splits<Tag, D, kHeads, false>(a, b, h0, Partials{first, first, n, 1}, [&] { return n; }, lds);
+  }
 }
 
 // Launches the vector split kernel; a (span, page mode) pair with no instantiation (a span whose
@@ -480,19 +575,30 @@ template <typename Tag, int D, int kHeads, int kSpan>
 hipError_t launch_split(const DecodeArgs& args, int groups, hipStream_t stream) {
   constexpr int kLPR = D * static_cast<int>(sizeof(typename Elem<Tag>::storage)) / 16;
   if constexpr (kSpan * kLPR <= 64) {
-    const dim3 grid(groups / kSpan * args.num_splits);
+    const dim3 grid(args.balanced_wgs ? args.balanced_wgs : groups / kSpan * args.num_splits);
     if (args.block_tables == nullptr) {
-      hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kContiguous>), grid,
-                         dim3(kThreads), 0, stream, args);
+      if (args.balanced_wgs) {
+        hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kContiguous, true>), grid,
+                           dim3(kThreads), 0, stream, args);
+      } else {
+        hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kContiguous, false>), grid,
+                           dim3(kThreads), 0, stream, args);
+      }
       return hipGetLastError();
     }
     if (!args.page_table_global) {
-      hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kPagedLds>), grid,
-                         dim3(kThreads), 0, stream, args);
+      if (args.balanced_wgs) {
+        hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kPagedLds, true>), grid,
+                           dim3(kThreads), 0, stream, args);
+      } else {
+        hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, kSpan, kPagedLds, false>), grid,
+                           dim3(kThreads), 0, stream, args);
+      }
       return hipGetLastError();
     }
+    if (args.balanced_wgs) return hipErrorInvalidValue;
     if constexpr (kSpan == 1) {  // the rare long-split case: one instantiation per type
-      hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, 1, kPagedGlobal>), grid,
+      hipLaunchKernelGGL((decode_split_kernel<Tag, D, kHeads, 1, kPagedGlobal, false>), grid,
                          dim3(kThreads), 0, stream, args);
       return hipGetLastError();
     }
@@ -515,8 +621,11 @@ hipError_t launch_heads(const DecodeArgs& args, DType dtype, hipStream_t stream)
     }
   }
   if (err != hipSuccess || args.num_splits == 1) return err;
-  hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kHeads>), dim3(groups), dim3(kThreads), 0, stream,
-                     args);
+  if (args.balanced_wgs) {
+    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kHeads, true>), dim3(groups), dim3(kThreads), 0, stream, args);
+  } else {
+    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kHeads, false>), dim3(groups), dim3(kThreads), 0, stream, args);
+  }
   return hipGetLastError();
 }
 

@@ -40,6 +40,7 @@
 //    (one split) or its unnormalized partial output and (reference point, sum), which decode.hip's
 //    merge pass combines as it would (max, sum). No atomics: results are bitwise reproducible for a
 //    given split count.
+#include "decode_sched.hpp"
 #include "gfx950.hpp"
 #include "launch.hpp"
 #include "prefill_tile.hpp"
@@ -85,7 +86,7 @@ constexpr int kRedBytes = 4 * (2 * kWaves * kMaxDecodeMfmaHeads + kWaves * kMaxD
 template <int D>
 constexpr int kSmemBytes = kLdsBytes<D> > kRedBytes<D> ? kLdsBytes<D> : kRedBytes<D>;
 
-template <typename Tag, int D, int kPageMode>
+template <typename Tag, int D, int kPageMode, bool kBalanced>
 __global__ void __launch_bounds__(kThreads) decode_mfma_kernel(const DecodeArgs a) {
   using E = Elem<Tag>;
   constexpr bool kPaged = kPageMode != kContiguous;
@@ -100,23 +101,51 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_kernel(const DecodeArgs 
   const int half = lane >> 5;
   const int col = lane & 31;  // the query head (within the group) of this lane's column
 
-  int w = blockIdx.x;
-  const int split = w % a.num_splits;
-  w /= a.num_splits;
   const int span = a.mfma_span;  // 1, or 4: wave w takes KV head 4 q + w over all the split's tiles
-  const int hq = w % (a.heads_kv / span);
-  const int b = w / (a.heads_kv / span);
-  const int hkv = span == 1 ? hq : hq * span + wave;
+  const int rows = a.heads_kv / span;  // work heads per sequence
   const int group = a.group;  // <= kCols (checked on the host)
-  const int h0 = hkv * group;
 
-  // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
-  // out-of-range value cannot read outside it.
-  const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
-  const int per_split =
-      ((len + a.num_splits - 1) / a.num_splits + kTileKeys - 1) / kTileKeys * kTileKeys;
-  const int k_begin = split * per_split;
-  const int k_end = min(len, k_begin + per_split);
+  // A workgroup runs one segment, a key range of one work head: its split of a sequence, or, in a
+  // balanced call, each row segment of its share of the line (decode_sched.hpp).
+  decode::Schedule sched{};
+  int pos = 0;
+  int end = 1;
+  if constexpr (kBalanced) {
+    sched = decode::make_schedule(a, rows);
+    pos = blockIdx.x * sched.chunk;
+    end = min(pos + sched.chunk, sched.total);
+  }
+  while (pos < end) {  // (once, where not balanced)
+  int b, hq, k_begin, k_end, head_step;
+  int64_t partial;  // index of the segment's first partial; the next head's is head_step on
+  if constexpr (kBalanced) {
+    const decode::Segment g = decode::segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
+    pos = g.next;
+    if (g.k_begin == g.k_end) continue;
+    b = g.b;
+    hq = g.head;
+    k_begin = g.k_begin;
+    k_end = g.k_end;
+    partial = g.slot * (span * group);
+    head_step = 1;
+  } else {
+    pos = end;
+    const int split = blockIdx.x % a.num_splits;
+    const int work = blockIdx.x / a.num_splits;
+    b = work / rows;
+    hq = work - b * rows;
+    // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
+    // out-of-range value cannot read outside it.
+    const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
+    const int per_split =
+        ((len + a.num_splits - 1) / a.num_splits + kTileKeys - 1) / kTileKeys * kTileKeys;
+    k_begin = split * per_split;
+    k_end = min(len, k_begin + per_split);
+    partial = (static_cast<int64_t>(b) * a.heads + hq * span * group) * a.num_splits + split;
+    head_step = a.num_splits;
+  }
+  const int hkv = span == 1 ? hq : hq * span + wave;
+  const int h0 = hkv * group;
   const int tiles = k_begin < k_end ? (k_end - k_begin + kTileKeys - 1) / kTileKeys : 0;
   const int my_tiles = span == 1 ? (tiles > wave ? (tiles - wave + kWaves - 1) / kWaves : 0) : tiles;
 
@@ -347,7 +376,7 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_kernel(const DecodeArgs 
       orow[d] = E::from_float(den > 0.f ? num / den : 0.f);
       if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
     } else {
-      const int64_t slot = (static_cast<int64_t>(b) * a.heads + h) * a.num_splits + split;
+      const int64_t slot = partial + static_cast<int64_t>(wv0 * group + g) * head_step;
       a.partial_o[slot * D + d] = num;
       if (d == 0) {
         a.partial_ml[2 * slot] = mm;
@@ -355,17 +384,30 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_kernel(const DecodeArgs 
       }
     }
   }
+  if constexpr (!kBalanced) return;
+  if (pos < end) __syncthreads();  // the next segment reuses the LDS
+  }
 }
 
 template <typename Tag, int D>
 hipError_t launch_typed(const DecodeArgs& args, hipStream_t stream) {
-  const dim3 grid(args.batch * (args.heads_kv / args.mfma_span) * args.num_splits);
+  const dim3 grid(args.balanced_wgs ? args.balanced_wgs
+                                    : args.batch * (args.heads_kv / args.mfma_span) * args.num_splits);
+  if (args.balanced_wgs && args.page_table_global) return hipErrorInvalidValue;
   if (args.block_tables == nullptr) {
-    hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kContiguous>), grid, dim3(kThreads), 0, stream, args);
+    if (args.balanced_wgs) {
+      hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kContiguous, true>), grid, dim3(kThreads), 0, stream, args);
+    } else {
+      hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kContiguous, false>), grid, dim3(kThreads), 0, stream, args);
+    }
   } else if (!args.page_table_global) {
-    hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kPagedLds>), grid, dim3(kThreads), 0, stream, args);
+    if (args.balanced_wgs) {
+      hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kPagedLds, true>), grid, dim3(kThreads), 0, stream, args);
+    } else {
+      hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kPagedLds, false>), grid, dim3(kThreads), 0, stream, args);
+    }
   } else {
-    hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kPagedGlobal>), grid, dim3(kThreads), 0, stream, args);
+    hipLaunchKernelGGL((decode_mfma_kernel<Tag, D, kPagedGlobal, false>), grid, dim3(kThreads), 0, stream, args);
   }
   return hipGetLastError();
 }

@@ -86,6 +86,13 @@ struct DecodeArgs {
   // Matrix-core kernel: KV heads per workgroup, 1 (the four waves share one KV head's tiles) or 4
   // (wave w takes KV head 4 q + w over all of the split's tiles).
   int mfma_span;
+  // Balanced calls (decode_sched.hpp): workgroups that share all sequences' keys (0: each sequence is
+  // cut into num_splits), log2 of the keys per unit, fewest units of a workgroup, and the units that
+  // starting one more segment costs. Partials are then [slot][head of the workgroup]: partial_o D
+  // floats each, partial_ml two; row_slots holds every row's partial count and its first overflow slot
+  // less kRowSlots (unwritten for a sequence without keys).
+  int balanced_wgs, unit_shift, min_units, ramp_units;
+  int2* row_slots;
 };
 
 // How the decode kernels find cache rows: contiguous cache, paged cache with the split's block
@@ -95,6 +102,10 @@ enum PageMode { kContiguous = 0, kPagedLds = 1, kPagedGlobal = 2 };
 
 // Largest split count a decode call may use.
 constexpr int kMaxSplits = 128;
+// Most sequences a balanced decode call may have.
+constexpr int kMaxBalancedBatch = 256;
+// Partials of a row of a balanced call that the merge pass can read before it knows their number.
+constexpr int kRowSlots = 8;
 // Most cache blocks one split of a paged decode may touch (its block numbers are staged in LDS).
 constexpr int kMaxSplitPages = 1024;
 // Most query heads per KV head the matrix-core decode kernel serves (its MFMA tile's columns).

@@ -136,6 +136,20 @@ SIGNATURES = {
             ctypes.POINTER(ctypes.c_size_t),
         ],
     ),
+    "fl_decode_schedule": (
+        ctypes.c_int,
+        [
+            ctypes.POINTER(DecodeParams),
+            ctypes.c_int32,
+            ctypes.POINTER(ctypes.c_int32),
+            ctypes.POINTER(ctypes.c_int32),
+            ctypes.POINTER(ctypes.c_size_t),
+        ],
+    ),
+    "fl_decode_balanced": (
+        ctypes.c_int,
+        [ctypes.POINTER(DecodeParams), ctypes.c_int32, ctypes.c_void_p],
+    ),
     "fl_decode": (ctypes.c_int, [ctypes.POINTER(DecodeParams), ctypes.c_void_p]),
     "fl_decode_noalloc": (ctypes.c_int, [ctypes.POINTER(DecodeParams), ctypes.c_void_p]),
     "fl_smoke_axpy": (
@@ -370,7 +384,8 @@ def _decode_params(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale,
 def decode(q, k_cache, v_cache, seq_lens, softmax_scale: float, num_splits: int, allow_splits: bool,
            block_tables=None):
     """Op-boundary checks of the reference (csrc/decode/decode_host.h:18-53,
-    csrc/decode/decode.cu:286-311), output and workspace allocation, fl_decode_plan + fl_decode.
+    csrc/decode/decode.cu:286-311), output and workspace allocation, and fl_decode_schedule or fl_decode_plan with the call
+    they ask for.
     With block_tables the caches are paged, [num_blocks, page_size, H_kv, D] (a layout the
     reference defines but none of its kernels runs)."""
     _check_cuda(q=q, k_cache=k_cache, v_cache=v_cache, seq_lens=seq_lens)
@@ -411,18 +426,25 @@ def decode(q, k_cache, v_cache, seq_lens, softmax_scale: float, num_splits: int,
     lse = torch.empty(q.shape[:2], dtype=torch.float32, device=q.device)
     p = _decode_params(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale, block_tables)
     index = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    splits, ws_bytes = ctypes.c_int32(), ctypes.c_size_t()
-    _check(LIB.fl_decode_plan(ctypes.byref(p), int(num_splits), int(bool(allow_splits)),
-                              cu_count(index), ctypes.byref(splits), ctypes.byref(ws_bytes)))
-    splits, ws_bytes = splits.value, ws_bytes.value
-    p.num_splits = splits
+    splits, wgs, ws_bytes = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
+    if allow_splits and num_splits == 0:
+        _check(LIB.fl_decode_schedule(ctypes.byref(p), cu_count(index), ctypes.byref(splits),
+                                      ctypes.byref(wgs), ctypes.byref(ws_bytes)))
+    else:
+        _check(LIB.fl_decode_plan(ctypes.byref(p), int(num_splits), int(bool(allow_splits)),
+                                  cu_count(index), ctypes.byref(splits), ctypes.byref(ws_bytes)))
+    ws_bytes = ws_bytes.value
+    p.num_splits = splits.value
     workspace = None
     if ws_bytes:
         workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device)
         p.workspace = workspace.data_ptr()
         p.workspace_bytes = ws_bytes
     with _on_device(q.device):
-        _check(LIB.fl_decode(ctypes.byref(p), _stream(q.device)))
+        if wgs.value:
+            _check(LIB.fl_decode_balanced(ctypes.byref(p), wgs.value, _stream(q.device)))
+        else:
+            _check(LIB.fl_decode(ctypes.byref(p), _stream(q.device)))
     return o, lse
 
 

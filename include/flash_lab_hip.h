@@ -146,6 +146,23 @@ int fl_decode_plan(const fl_decode_params* p, int32_t requested_splits, int32_t 
                    int32_t cu_count, int32_t* num_splits, size_t* workspace_bytes);
 
 /*
+ * How a decode call whose caller asks for no split count is shared out; host-only, touches no device.
+ * No counterpart in the reference. Either *num_splits >= 1 and *workgroups == 0: pass the count to
+ * fl_decode; or *num_splits == 0 and *workgroups > 0: pass it to fl_decode_balanced. *workspace_bytes
+ * is what that call needs.
+ */
+int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num_splits,
+                       int32_t* workgroups, size_t* workspace_bytes);
+
+/*
+ * Decode with the keys of all sequences shared evenly between `workgroups` workgroups, by the lengths
+ * in seq_lens as the device finds them (num_splits is ignored). Unequal sequences then end together
+ * instead of all waiting for the longest one's splits. A merge pass combines the partials in a fixed
+ * order: results are bitwise reproducible for the same lengths and workgroups.
+ */
+int fl_decode_balanced(const fl_decode_params* p, int32_t workgroups, fl_stream_t stream);
+
+/*
  * Split-KV decode: partial passes over contiguous key ranges with fp32
  * partials, then a fixed-order log-sum-exp merge (reference
  * csrc/decode/decode.cu:40-235). With num_splits == 1 the single pass
