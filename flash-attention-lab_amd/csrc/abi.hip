@@ -49,6 +49,11 @@ bool rows_16_byte(const void* p, int elem_bytes, int64_t size0, int64_t stride0,
 
 int elem_bytes(int32_t dtype) { return dtype == FL_DTYPE_F32 ? 4 : 2; }
 
+// K (or V) rows of all sequences' caches.
+int64_t cache_rows(const fl_decode_params* p) {
+  return static_cast<int64_t>(p->batch) * p->heads_kv * p->max_seqlen;
+}
+
 bool valid_scale(double s) { return std::isfinite(s) && s > 0.0; }
 
 fl::DType decode_dtype(int32_t dtype) {
@@ -201,6 +206,28 @@ size_t balanced_partials(const fl_decode_params* p, const BalancedLayout& layout
          (static_cast<size_t>(p->batch) * p->heads / layout.rows);
 }
 
+// Split count of a call that nobody asked for one of, from the plan's (fl_decode_plan's, which long
+// caches were tuned on). One workgroup per CU, one KV head each, is the fastest for short caches on
+// every kernel, and on the vector kernel with several query heads for all of them (device us, plan /
+// this; B, H, H_kv, S, D = 128): matrix cores, down to 64 keys a split, (1, 32, 8, 640) 11.0 / 9.6, (1,
+// 32, 8, 2600) 11.9 / 11.0; several query heads, (8, 16, 8, 32000) bf16 163 / 153, (1, 32, 8, 8320) fp32
+// 23 / 19, (4, 32, 8, 4000) fp32 30 / 27; one, (4, 8, 8, 3000) 14.3 / 13.8. Where several workgroups
+// read the same keys (a group of 3 in fp32), splits of some 200 keys keep those reads close together:
+// (14, 24, 8, 1600, D = 64) 49 / 32, (4, 24, 8, 4000) 69 / 41.
+int scheduled_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, int cus, int planned) {
+  const int64_t chunks = p->heads / p->heads_kv / layout.wg_heads;
+  const int64_t work = static_cast<int64_t>(p->batch) * p->heads_kv * chunks;
+  int n = largest_splits(work, p->max_seqlen, cus, 64);
+  if (layout.mfma) return mfma_span(p, layout, planned) == 1 ? n : planned;
+  if (chunks > 1)
+    while (n < fl::kMaxSplits && work * 2 * n <= 16 * static_cast<int64_t>(cus) && p->max_seqlen / (2 * n) >= 180) n *= 2;
+  // Not where the power of two leaves a tenth of the CUs without a workgroup: (20, 32, 8, 1500) fp32 with
+  // unequal lengths 33 us as planned, 50 with one split.
+  if (layout.heads_per_wg > 1 || chunks > 1) return 10 * work * n >= 9 * static_cast<int64_t>(cus) ? n : planned;
+  const double bytes = 2.0 * cache_rows(p) * p->head_dim * elem_bytes(p->dtype);
+  return bytes < 64e6 && n >= 8 && n < planned ? n : planned;
+}
+
 // Whether a call that could be balanced is. The host does not know the lengths, so what equal ones
 // lose counts too: deriving the schedule takes a workgroup about 1.5 us before its first load, and a
 // fixed plan of one split needs no merge pass. So it takes several sequences and a cache that the CUs
@@ -270,7 +297,7 @@ int decode_call(const fl_decode_params* p, int balanced_wgs, float* workspace, s
 
   const int group = p->heads / p->heads_kv;
   const fl::DType dt = decode_dtype(p->dtype);
-  const fl::DecodeLayout layout = fl::decode_layout(dt, p->head_dim, p->heads_kv, group);
+  const fl::DecodeLayout layout = fl::decode_layout(dt, p->head_dim, p->heads_kv, group, cache_rows(p));
   const int head_chunks = group / layout.heads_per_wg;
   const int num_splits = balanced_wgs > 0 ? 0 : p->num_splits;
   const int64_t blocks = static_cast<int64_t>(p->batch) * p->heads_kv * head_chunks * num_splits;
@@ -562,7 +589,7 @@ int fl_decode_plan(const fl_decode_params* p, int32_t requested_splits, int32_t 
     return fail(FL_ERR_INVALID, "null output pointer");
   const int group = p->heads / p->heads_kv;
   const fl::DecodeLayout layout =
-      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, group);
+      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, group, cache_rows(p));
   int n = 1;
   if (allow_splits && requested_splits > 0) {
     n = requested_splits;
@@ -613,7 +640,7 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
   if (int rc = fl_decode_plan(p, 0, 1, cu_count, num_splits, workspace_bytes)) return rc;
   *workgroups = 0;
   const fl::DecodeLayout layout =
-      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, p->heads / p->heads_kv);
+      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, p->heads / p->heads_kv, cache_rows(p));
   // Short caches: one workgroup per KV head and no merge pass, while the keys that more workgroups
   // would take off it cost less than the pass (about 3.9 us, against 11.5 us per 1,000 keys): (B, H,
   // H_kv, S) (16, 32, 8, 320) 10.3 us with one split, 11.9 with two, (2, 8, 8, 90) 3.8 and 6.3, (4, 32,
@@ -624,7 +651,18 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
     *workspace_bytes = 0;
     return FL_OK;
   }
-  if (!worth_balancing(p, layout, *num_splits, cu_count > 0 ? cu_count : 256)) return FL_OK;
+  const int cus = cu_count > 0 ? cu_count : 256;
+  if (!worth_balancing(p, layout, *num_splits, cus)) {
+    // (A paged plan also keeps each split's block numbers within LDS: never fewer splits then.)
+    const int n = fl::knob(FL_KNOB_DECODE_WG_PER_CU) >= 1 ? *num_splits
+                                                          : scheduled_splits(p, layout, cus, *num_splits);
+    if (p->block_tables == nullptr || pages_per_split(p->max_seqlen, n, p->page_size) <= fl::kMaxSplitPages)
+      *num_splits = n;
+    *workspace_bytes = *num_splits > 1 ? static_cast<size_t>(p->batch) * p->heads * *num_splits *
+                                             (p->head_dim + 2) * sizeof(float)
+                                       : 0;
+    return FL_OK;
+  }
   const int64_t wgs = resident_capacity(cu_count, planned_per_cu(p, layout));
   const BalancedLayout balanced = balanced_layout(p, layout, static_cast<int>(wgs));
   if (!balanced.fits) return FL_OK;

@@ -655,19 +655,21 @@ hipError_t launch_type(const DecodeArgs& args, DType dtype, int head_dim, int k_
 // D = 64, B=8 86.4 vs 93.8, B=4 50.7 vs 56.2, B=1 23.4 vs 24.4, one 8.4K-key sequence 14.9 vs
 // 18.0. With 2 it is mixed (D = 128: B=2 54.3 vs 49.3, B=4 89.3 vs 90.6; D = 64: B=2 33.7 vs
 // 30.4, B=8 85.7 vs 89.5), so groups of 2 stay on the vector kernel.
-int decode_mfma_min_group(int head_dim) {
-  (void)head_dim;
+// A group of 3 has no vector form of its own (one query head per workgroup, three passes over the
+// cache), so it goes to the matrix cores too, from 16K cache rows: (10, 24, 8, 15868) 277 vs 102 us, (4,
+// 24, 8, 2000) 23 vs 14, (1, 24, 8, 2600) 10.2 for both, (1, 24, 8, 640) 7.7 on the vector kernel, 9.3.
+int decode_mfma_min_group(int64_t cache_rows) {
   const int v = knob(FL_KNOB_DECODE_MFMA_MIN_GROUP);
   if (v >= 1) return v;
-  return 4;
+  return cache_rows >= 16384 ? 3 : 4;
 }
 
-DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group) {
+DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows) {
   DecodeLayout layout{};
   int k = 1;
   while (k < 8 && group % (2 * k) == 0) k *= 2;
   layout.heads_per_wg = k;
-  if (dtype != DType::f32 && group >= decode_mfma_min_group(head_dim) &&
+  if (dtype != DType::f32 && group >= decode_mfma_min_group(cache_rows) &&
       group <= kMaxDecodeMfmaHeads) {
     // One KV head per workgroup. Two fit a CU (256 registers per lane, 64 KiB of LDS at D = 128),
     // but one per CU streamed faster (B=8, 8 KV heads, 32K keys: 6.03-6.09 TB/s against

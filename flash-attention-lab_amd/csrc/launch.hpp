@@ -153,7 +153,8 @@ struct DecodeLayout {
   int mfma;
   int wg_heads;  // query heads per KV head in one split workgroup
 };
-DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group);
+// cache_rows: K (or V) rows of all sequences and KV heads.
+DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows);
 hipError_t launch_decode(const DecodeArgs& args, DType dtype, int head_dim, hipStream_t stream);
 // The matrix-core split kernel alone (launch_decode runs it and the merge pass when args.mfma).
 hipError_t launch_decode_mfma_split(const DecodeArgs& args, DType dtype, int head_dim,

@@ -127,6 +127,23 @@ def test_plan():
     assert plan(2, 8, 8, 64, 64) == (1, 0, 0)  # too short to be worth a merge pass
 
 
+def test_split_counts():
+    # One workgroup per CU where nobody asked for a count: matrix cores down to 64 keys, several query
+    # heads on the vector kernel (fp32 here), and no more than that for short caches of one.
+    assert plan(1, 32, 8, 128, 640)[:2] == (8, 0)
+    assert plan(1, 32, 8, 128, 8448)[:2] == (32, 0)
+    assert plan(8, 32, 8, 128, 32768)[:2] == (16, 0)  # four KV heads per workgroup, as planned
+    assert plan(8, 32, 8, 128, 16000, dtype=2)[:2] == (4, 0)
+    assert plan(4, 8, 8, 128, 3000)[:2] == (8, 0)
+    assert plan(1, 32, 32, 128, 32768)[:2] == (16, 0)  # long: as planned
+    # Groups of 3: matrix cores (one KV head per workgroup: 32 splits), and in fp32, where three workgroups
+    # read the same keys, splits of 180 keys or more.
+    assert plan(1, 24, 8, 128, 8192)[:2] == (32, 0)
+    assert plan(4, 24, 8, 128, 4000, dtype=2)[:2] == (16, 0)
+    # A paged call keeps a split's block numbers within LDS.
+    assert plan(1, 16, 8, 128, 131072, page_size=1)[0] == 128
+
+
 def test_balanced_call_is_checked_before_any_launch():
     p = _hip.DecodeParams()
     p.q = p.k_cache = p.v_cache = p.o = p.lse = p.seq_lens = 256
