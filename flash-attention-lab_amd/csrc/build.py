@@ -1,10 +1,12 @@
-"""Builds the gfx950 C-ABI library, flash_lab/libflash_lab_hip.so, with hipcc.
+"""Builds the gfx950 C-ABI library, flash_lab/libflash_lab_hip.so, with hipcc, and the torch ops over
+it, flash_lab/libflash_lab_torch.so, with the host compiler.
 
     python flash-attention-lab_amd/csrc/build.py [-v]
 
 Each .hip file is compiled to an object in csrc/_build (in parallel), then linked into one shared
 library next to the Python package, which loads it with ctypes. No CMake, no torch extension
-machinery: the library has a plain C ABI (include/flash_lab_hip.h).
+machinery: the library has a plain C ABI (include/flash_lab_hip.h), and torch_ops.cpp, host code
+only, is one compilation against torch's headers.
 """
 
 from __future__ import annotations
@@ -29,6 +31,8 @@ OUTPUT = PKG_ROOT / "flash_lab" / "libflash_lab_hip.so"
 
 SOURCES = ("abi.hip", "prefill_fwd.hip", "prefill_pp.hip", "prefill_causal.hip", "decode.hip",
            "decode_mfma.hip", "smoke.hip")
+TORCH_SOURCE = "torch_ops.cpp"
+TORCH_OUTPUT = PKG_ROOT / "flash_lab" / "libflash_lab_torch.so"
 ARCH = "gfx950"
 FLAGS = (
     f"--offload-arch={ARCH}",
@@ -52,6 +56,22 @@ def hipcc() -> str:
     return found
 
 
+def torch_ops_command() -> list[str]:
+    """The host compiler's command for TORCH_OUTPUT. torch's HIP headers want the platform named."""
+    import torch
+
+    torch_dir = Path(torch.__file__).resolve().parent
+    compiler = shutil.which("g++") or shutil.which("c++") or "/opt/rocm/llvm/bin/clang++"
+    return [
+        compiler, "-std=c++17", "-O2", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+        f"-I{INCLUDE}", f"-isystem{torch_dir / 'include'}",
+        f"-isystem{torch_dir / 'include' / 'torch' / 'csrc' / 'api' / 'include'}", "-isystem/opt/rocm/include",
+        str(CSRC / TORCH_SOURCE), "-o", str(TORCH_OUTPUT.with_suffix(".so.tmp")), f"-L{torch_dir / 'lib'}",
+        "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip",
+    ]
+
+
 def _run(cmd: list[str], verbose: bool) -> None:
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -71,8 +91,8 @@ def build(
     defines: tuple[str, ...] = (),
     output: Path | None = None,
 ) -> Path:
-    """Compiles every source and links the library (OUTPUT unless `output` is given); always
-    rebuilds. `defines` are NAME=VALUE preprocessor settings of the kernels' tuning knobs."""
+    """Compiles every source and links the library (OUTPUT, with the torch ops beside it, unless
+    `output` is given); always rebuilds. `defines` are NAME=VALUE preprocessor settings of the kernels' tuning knobs."""
     compiler = hipcc()
     output = Path(output) if output is not None else OUTPUT
     build_dir = BUILD_DIR if output == OUTPUT else output.parent / f"_build_{output.stem}"
@@ -87,6 +107,8 @@ def build(
         commands.append(
             [compiler, *FLAGS, *macro_flags, *includes, "-c", str(CSRC / src), "-o", str(obj)]
         )
+    if output == OUTPUT:
+        commands.append(torch_ops_command())
     workers = jobs or min(len(commands), os.cpu_count() or 1)
     with concurrent.futures.ThreadPoolExecutor(max_workers=workers) as pool:
         for fut in [pool.submit(_run, cmd, verbose) for cmd in commands]:
@@ -95,6 +117,8 @@ def build(
     _run([compiler, f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)],
          verbose)
     os.replace(tmp, output)
+    if output == OUTPUT:
+        os.replace(TORCH_OUTPUT.with_suffix(".so.tmp"), TORCH_OUTPUT)
     write_build_record(output, compiler, defines)
     return output
 
@@ -114,7 +138,7 @@ def write_build_record(output: Path, compiler: str, defines: tuple[str, ...]) ->
     and the flags. It travels with the library, so a benchmark run on another machine, where
     the checkout has no git metadata, can still say what it ran."""
     digest = hashlib.sha256()
-    for path in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.hpp"), *INCLUDE.glob("*.h")]):
+    for path in sorted([*CSRC.glob("*.hip"), *CSRC.glob("*.hpp"), *CSRC.glob("*.cpp"), *INCLUDE.glob("*.h")]):
         digest.update(path.name.encode())
         digest.update(path.read_bytes())
     status = _git("status", "--porcelain", "--", str(CSRC), str(INCLUDE))

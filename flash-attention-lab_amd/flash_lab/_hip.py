@@ -1,22 +1,24 @@
-"""The gfx950 kernels as torch ops: ctypes over the C ABI of libflash_lab_hip.so.
+"""The gfx950 kernels as torch ops, over the C ABI of libflash_lab_hip.so.
 
-This module replaces the reference's compiled op registry (csrc/bindings.cpp:7-42) and its C++
-host wrappers (csrc/common/attn_host.h, csrc/decode/decode.cu:282-347). Importing it loads the
-library and registers, under torch.ops.flash_lab, ops with the reference's names and schemas:
+This module replaces the reference's compiled op registry (csrc/bindings.cpp:7-42). Importing it
+loads the kernel library and the native ops over it (csrc/torch_ops.cpp, libflash_lab_torch.so) and
+registers, under torch.ops.flash_lab, ops with the reference's names and schemas:
 
     attention_mma_pipelined / attention_mma
         (Tensor q, Tensor k, Tensor v, bool causal, float softmax_scale) -> (Tensor, Tensor)
     decode_splitkv / decode_inplace
         (Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens, float softmax_scale,
          int num_splits) -> (Tensor, Tensor)
+    decode_splitkv_paged / decode_inplace_paged: the same with block_tables after seq_lens
     smoke_axpy(Tensor x, Tensor y, float alpha) -> Tensor
     mma_tile_test(Tensor a, Tensor b, bool trans_b) -> Tensor
 
-Each op allocates its outputs (and the decode workspace) with torch on the input's device, passes
-the current stream, and raises RuntimeError with the library's message when a call fails. Nothing
-here synchronizes, reads seq_lens on the host or allocates outside torch's caching allocator, so
-the ops can be captured in a HIP graph. If the library cannot be loaded, importing this module
-raises ImportError; there is no other code path.
+Each op allocates its outputs (and its workspace) with torch on the input's device, passes the
+current stream, and raises RuntimeError with the library's message when a call fails. Nothing here
+synchronizes, reads seq_lens on the host or allocates outside torch's caching allocator, so the ops
+can be captured in a HIP graph. If a library cannot be loaded, importing this module raises
+ImportError; there is no other code path. Also here: the library's own entry points through ctypes,
+for what the ops do not offer (plans, knobs, the allocation-free decode).
 """
 
 from __future__ import annotations
@@ -34,7 +36,6 @@ LIB_NAME = "libflash_lab_hip.so"
 LIB_PATH = Path(os.environ.get("FLASH_LAB_HIP_LIB", Path(__file__).with_name(LIB_NAME)))
 
 ERR_WORKSPACE = 4  # enum fl_status
-
 DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
@@ -201,6 +202,28 @@ def load_library(path: Path = LIB_PATH) -> ctypes.CDLL:
 
 LIB = load_library()
 
+TORCH_LIB_PATH = Path(__file__).with_name("libflash_lab_torch.so")
+# The library functions that fl_torch_bind takes, in its order.
+TORCH_BOUND = ("fl_attention_plan", "fl_attention_fwd_split", "fl_decode_plan", "fl_decode_schedule", "fl_decode",
+               "fl_decode_balanced", "fl_last_error")
+
+
+def load_torch_ops(path: Path = TORCH_LIB_PATH) -> ctypes.CDLL:
+    """Loads the native ops (which registers them with torch) and binds them to LIB's functions."""
+    if not path.exists():
+        raise ImportError(
+            f"{path} is missing; build it with `python flash-attention-lab_amd/csrc/build.py`"
+        )
+    try:
+        ops = ctypes.CDLL(str(path))
+    except OSError as exc:
+        raise ImportError(f"could not load {path}: {exc}") from exc
+    ops.fl_torch_bind.restype = None
+    ops.fl_torch_bind.argtypes = [ctypes.c_void_p] * len(TORCH_BOUND)
+    ops.fl_torch_bind(*(ctypes.cast(getattr(LIB, name), ctypes.c_void_p) for name in TORCH_BOUND))
+    return ops
+
+
 
 def _check(rc: int) -> None:
     if rc != 0:
@@ -273,73 +296,6 @@ def _check_cuda(**tensors: torch.Tensor) -> None:
 
 
 # ----------------------------------------------------------------------------------------------
-# Prefill
-
-
-def prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, softmax_scale: float,
-            num_splits: int = 0):
-    """Op-boundary checks of the reference (csrc/common/attn_host.h:18-57), output and workspace
-    allocation, and fl_attention_fwd_split (num_splits 0: the library's choice)."""
-    _check_cuda(q=q, k=k, v=v)
-    _require(q.dtype in (torch.bfloat16, torch.float16), "attention_mma_pipelined takes bf16 or fp16")
-    _require(k.dtype == q.dtype and v.dtype == q.dtype, "k and v must have dtype %s", q.dtype)
-    _require(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "q, k, v must be [B, S, H, D]")
-    _require(k.shape == v.shape, "k and v must have the same shape")
-    _require(
-        q.shape[0] == k.shape[0] and q.shape[3] == k.shape[3],
-        "q and k must agree on batch size and head_dim",
-    )
-    _require(q.device == k.device and q.device == v.device, "q, k, v on different devices")
-    for name, x in (("q", q), ("k", k), ("v", v)):
-        _require(x.stride(-1) == 1, "%s must be contiguous in its last dimension", name)
-    batch, seqlen_q, heads, head_dim = q.shape
-    # The kernel needs non-overlapping K and V rows (sequence stride >= head_dim); broadcast or
-    # overlapping views, which the reference also accepts, are passed as contiguous copies.
-    if k.shape[1] > 1 and k.stride(1) < head_dim:
-        k = k.contiguous()
-    if v.shape[1] > 1 and v.stride(1) < head_dim:
-        v = v.contiguous()
-    o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    lse = torch.empty((batch, heads, seqlen_q), dtype=torch.float32, device=q.device)
-    p = AttnParams(
-        q.data_ptr(),
-        k.data_ptr(),
-        v.data_ptr(),
-        o.data_ptr(),
-        lse.data_ptr(),
-        *q.stride()[:3],
-        *k.stride()[:3],
-        *v.stride()[:3],
-        *o.stride()[:3],
-        batch,
-        seqlen_q,
-        k.shape[1],
-        heads,
-        k.shape[2],
-        head_dim,
-        int(bool(causal)),
-        DTYPE_CODES[q.dtype],
-        float(softmax_scale),
-    )
-    index = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    cus = cu_count(index)
-    with _on_device(q.device):
-        stream = _stream(q.device)
-        if num_splits == 0:
-            rc = LIB.fl_attention_fwd_split(ctypes.byref(p), 0, cus, None, 0, stream)
-            if rc != ERR_WORKSPACE:
-                _check(rc)
-                return o, lse
-        splits, ws_bytes = ctypes.c_int32(), ctypes.c_size_t()
-        _check(LIB.fl_attention_plan(ctypes.byref(p), num_splits, cus, ctypes.byref(splits),
-                                     ctypes.byref(ws_bytes)))
-        workspace = torch.empty(ws_bytes.value // 4, dtype=torch.float32, device=q.device)
-        _check(LIB.fl_attention_fwd_split(ctypes.byref(p), splits.value, cus, workspace.data_ptr(),
-                                          ws_bytes.value, stream))
-    return o, lse
-
-
-# ----------------------------------------------------------------------------------------------
 # Decode
 
 
@@ -381,73 +337,6 @@ def _decode_params(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale,
     )
 
 
-def decode(q, k_cache, v_cache, seq_lens, softmax_scale: float, num_splits: int, allow_splits: bool,
-           block_tables=None):
-    """Op-boundary checks of the reference (csrc/decode/decode_host.h:18-53,
-    csrc/decode/decode.cu:286-311), output and workspace allocation, and fl_decode_schedule or fl_decode_plan with the call
-    they ask for.
-    With block_tables the caches are paged, [num_blocks, page_size, H_kv, D] (a layout the
-    reference defines but none of its kernels runs)."""
-    _check_cuda(q=q, k_cache=k_cache, v_cache=v_cache, seq_lens=seq_lens)
-    _require(q.dtype in DTYPE_CODES, "decode takes bf16, fp16, or fp32")
-    _require(
-        k_cache.dtype == q.dtype and v_cache.dtype == q.dtype,
-        "k_cache and v_cache must have dtype %s",
-        q.dtype,
-    )
-    _require(seq_lens.dtype == torch.int32, "seq_lens must have dtype int32")
-    _require(q.dim() == 3 and k_cache.dim() == 4, "q must be [B, H, D], caches [B, S_max, H_kv, D]")
-    _require(k_cache.shape == v_cache.shape, "k_cache and v_cache must have the same shape")
-    if block_tables is None:
-        _require(
-            k_cache.shape[0] == q.shape[0] and k_cache.shape[3] == q.shape[2],
-            "q and the caches must agree on batch size and head_dim",
-        )
-    else:
-        _check_cuda(block_tables=block_tables)
-        _require(block_tables.dtype == torch.int32, "block_tables must have dtype int32")
-        _require(
-            block_tables.dim() == 2 and block_tables.shape[0] == q.shape[0]
-            and block_tables.shape[1] >= 1 and block_tables.stride(1) == 1,
-            "block_tables must be [B, max_blocks] with unit stride in its last dimension",
-        )
-        _require(k_cache.shape[3] == q.shape[2], "q and the caches must agree on head_dim")
-        _require(
-            block_tables.shape[1] * k_cache.shape[1] < 2**31,
-            "paged cache too long (max_blocks * page_size must fit in int32)",
-        )
-    _require(seq_lens.dim() == 1 and seq_lens.shape[0] == q.shape[0], "seq_lens must be [B]")
-    _require(seq_lens.is_contiguous(), "seq_lens must be contiguous")
-    for name, x in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache)):
-        _require(x.stride(-1) == 1, "%s must be contiguous in its last dimension", name)
-    _require(0 <= num_splits <= 128, "num_splits must be in [0, 128]")
-
-    o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    lse = torch.empty(q.shape[:2], dtype=torch.float32, device=q.device)
-    p = _decode_params(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale, block_tables)
-    index = q.device.index if q.device.index is not None else torch.cuda.current_device()
-    splits, wgs, ws_bytes = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
-    if allow_splits and num_splits == 0:
-        _check(LIB.fl_decode_schedule(ctypes.byref(p), cu_count(index), ctypes.byref(splits),
-                                      ctypes.byref(wgs), ctypes.byref(ws_bytes)))
-    else:
-        _check(LIB.fl_decode_plan(ctypes.byref(p), int(num_splits), int(bool(allow_splits)),
-                                  cu_count(index), ctypes.byref(splits), ctypes.byref(ws_bytes)))
-    ws_bytes = ws_bytes.value
-    p.num_splits = splits.value
-    workspace = None
-    if ws_bytes:
-        workspace = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device)
-        p.workspace = workspace.data_ptr()
-        p.workspace_bytes = ws_bytes
-    with _on_device(q.device):
-        if wgs.value:
-            _check(LIB.fl_decode_balanced(ctypes.byref(p), wgs.value, _stream(q.device)))
-        else:
-            _check(LIB.fl_decode(ctypes.byref(p), _stream(q.device)))
-    return o, lse
-
-
 def decode_noalloc(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale: float, num_splits: int,
                    block_tables=None) -> int:
     """fl_decode_noalloc on caller-provided outputs o [B, H, D] and lse [B, H]: the split workspace
@@ -482,74 +371,8 @@ def decode_plan(batch, heads, heads_kv, head_dim, max_seqlen, dtype, num_splits=
 # Op registration
 
 
-# The reference's schemas, verbatim (csrc/bindings.cpp:9-41).
-PREFILL_SCHEMA = "(Tensor q, Tensor k, Tensor v, bool causal, float softmax_scale) -> (Tensor, Tensor)"
-DECODE_SCHEMA = (
-    "(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens, float softmax_scale,"
-    " int num_splits) -> (Tensor, Tensor)"
-)
-# Paged-cache decode has no op in the reference (its kernels reject paged caches): the same
-# schema with the block tables after seq_lens.
-PAGED_DECODE_SCHEMA = (
-    "(Tensor q, Tensor k_cache, Tensor v_cache, Tensor seq_lens, Tensor block_tables,"
-    " float softmax_scale, int num_splits) -> (Tensor, Tensor)"
-)
-
-
 def _register() -> None:
     lib = "flash_lab"
-
-    def prefill_op(name):
-        @torch.library.custom_op(
-            f"{lib}::{name}", mutates_args=(), device_types="cuda", schema=PREFILL_SCHEMA
-        )
-        def op(
-            q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, softmax_scale: float
-        ) -> tuple[torch.Tensor, torch.Tensor]:
-            return prefill(q, k, v, causal, softmax_scale)
-
-        return op
-
-    def decode_op(name, allow_splits):
-        @torch.library.custom_op(
-            f"{lib}::{name}", mutates_args=(), device_types="cuda", schema=DECODE_SCHEMA
-        )
-        def op(
-            q: torch.Tensor,
-            k_cache: torch.Tensor,
-            v_cache: torch.Tensor,
-            seq_lens: torch.Tensor,
-            softmax_scale: float,
-            num_splits: int,
-        ) -> tuple[torch.Tensor, torch.Tensor]:
-            return decode(q, k_cache, v_cache, seq_lens, softmax_scale, num_splits, allow_splits)
-
-        return op
-
-    prefill_op("attention_mma_pipelined")
-    prefill_op("attention_mma")
-    def paged_decode_op(name, allow_splits):
-        @torch.library.custom_op(
-            f"{lib}::{name}", mutates_args=(), device_types="cuda", schema=PAGED_DECODE_SCHEMA
-        )
-        def op(
-            q: torch.Tensor,
-            k_cache: torch.Tensor,
-            v_cache: torch.Tensor,
-            seq_lens: torch.Tensor,
-            block_tables: torch.Tensor,
-            softmax_scale: float,
-            num_splits: int,
-        ) -> tuple[torch.Tensor, torch.Tensor]:
-            return decode(q, k_cache, v_cache, seq_lens, softmax_scale, num_splits, allow_splits,
-                          block_tables)
-
-        return op
-
-    decode_op("decode_splitkv", True)
-    decode_op("decode_inplace", False)
-    paged_decode_op("decode_splitkv_paged", True)
-    paged_decode_op("decode_inplace_paged", False)
 
     @torch.library.custom_op(
         f"{lib}::smoke_axpy", mutates_args=(), device_types="cuda",
@@ -602,6 +425,9 @@ def _register() -> None:
         return a.new_empty((16, 16), dtype=torch.float32)
 
 
+# The attention and decode ops, native (csrc/torch_ops.cpp): loading the library registers them, and
+# they call the functions of the kernel library loaded above.
+TORCH_LIB = load_torch_ops()
 _register()
 
 OPS = (

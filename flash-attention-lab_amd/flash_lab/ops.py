@@ -142,6 +142,10 @@ _BUILT_OPS = frozenset(
 )
 
 
+# The ops' overloads, looked up once: the packet's own lookup takes a call about 2 us.
+_OVERLOADS = {op: getattr(torch.ops.flash_lab, op).default for op in _BUILT_OPS}
+
+
 def available_impls() -> dict[str, list[str]]:
     """Implementations compiled into this build, by entry point."""
     return {
@@ -202,7 +206,7 @@ def attention(
         ),
         lambda s: s.unsupported_reason(shape, q.dtype, causal),
     )
-    out, lse = getattr(torch.ops.flash_lab, spec.op)(q, k, v, causal, scale)
+    out, lse = _OVERLOADS[spec.op](q, k, v, causal, scale)
     return (out, lse) if return_lse else out
 
 
@@ -238,11 +242,11 @@ def decode(
         lambda s: s.unsupported_reason(shape, q.dtype),
     )
     if block_tables is not None:
-        out, lse = getattr(torch.ops.flash_lab, spec.paged_op)(
+        out, lse = _OVERLOADS[spec.paged_op](
             q3, k_cache, v_cache, seq_lens, block_tables, scale, num_splits or 0
         )
     else:
-        out, lse = getattr(torch.ops.flash_lab, spec.op)(
+        out, lse = _OVERLOADS[spec.op](
             q3, k_cache, v_cache, seq_lens, scale, num_splits or 0
         )
     if q.dim() == 4:
