@@ -7,7 +7,8 @@
 // definitions (csrc/prefill/mma_tile.cuh:60-174, flash_lab/reference.py:90-152), the mapping onto
 // the machine is this file's own:
 //
-//  * Workgroup: 4 waves x 32 query rows = 128 rows of one (batch, head). Lane layouts are in
+//  * Workgroup: 4 waves x 32 query rows = 128 rows of one (batch, head), or 2 x 32 rows with two waves
+//    to each 32 and half of every tile each, for grids that leave CUs idle (kParts). Lane layouts are in
 //    prefill_tile.hpp: scores and outputs are held transposed so a lane owns one query row.
 //  * K and V tiles of 64 keys go global -> registers -> LDS through a two-slot LDS ring: the next
 //    tile's global loads are issued before the current tile's math and written to the other slot
@@ -52,12 +53,19 @@ __device__ __forceinline__ int xcd_remap(int id, int n) {
 constexpr int kSchedMfma = 0x008;
 constexpr int kSchedDsRead = 0x100;
 
-template <typename Tag, int D>
+// kParts = 2: the wave pairs w, w + 2 share 32 rows, each taking one 32-key half of every tile, and the
+// halves are merged through LDS at the end; the workgroup then has 64 rows. For grids that leave CUs
+// without a workgroup, where the time is one workgroup's run through its tiles: the half-tile step is
+// the shorter one.
+template <typename Tag, int D, int kParts>
 __global__ void __launch_bounds__(kThreads)
     __attribute__((amdgpu_waves_per_eu(FL_PREFILL_WAVES_PER_EU, FL_PREFILL_WAVES_PER_EU)))
     prefill_fwd_kernel(const PrefillArgs a) {
   using E = Elem<Tag>;
   constexpr int kTile = kTileElems<D>;
+  constexpr int kRowWaves = kWaves / kParts;
+  constexpr int kRows = kRowsPerWave * kRowWaves;  // of the workgroup
+  constexpr bool kWhole = kParts == 1;             // a wave takes whole tiles
   // Two K and two V tile slots, each its own array: slot addresses are compile-time constants in
   // the unrolled loop below (every LDS read is one per-lane offset register plus an immediate),
   // and the compiler can tell that loads into one slot do not alias reads of another, so it does
@@ -79,8 +87,9 @@ __global__ void __launch_bounds__(kThreads)
   const int b = bh / a.work_heads;
   const int h = (bh - b * a.work_heads) * a.pack;  // first query head
   const int hkv = h / a.group;
-  const int q0 = qb * kBlockM;
-  const int row0 = q0 + wave * kRowsPerWave;  // first query row of this wave
+  const int q0 = qb * kRows;
+  const int part = kWhole ? 0 : wave / kRowWaves;             // the wave's key block of every tile
+  const int row0 = q0 + wave % kRowWaves * kRowsPerWave;  // first query row of this wave
   const int my_row = row0 + (lane & 31);      // the query row this lane owns
   const int my_pos = pack_position(a, my_row);
   const int my_head = my_row - my_pos * a.pack;  // of the packed heads
@@ -91,7 +100,7 @@ __global__ void __launch_bounds__(kThreads)
 
   int kv_end = a.seqlen_k;
   if (a.causal)
-    kv_end = min(kv_end, pack_position(a, min(q0 + kBlockM, a.rows) - 1) + 1 + a.causal_offset);
+    kv_end = min(kv_end, pack_position(a, min(q0 + kRows, a.rows) - 1) + 1 + a.causal_offset);
   const int num_tiles = kv_end > 0 ? (kv_end + kBlockN - 1) / kBlockN : 0;
 
   // Q^T fragments, the B operand of every S^T step: row my_row, dims 16 ks + 8 half .. + 7.
@@ -165,9 +174,12 @@ __global__ void __launch_bounds__(kThreads)
       dma(kSlot == 0 ? k_lds1 : k_lds0, kp, a.k_ss, k_off, t + 1);
       dma(kSlot == 0 ? v_lds1 : v_lds0, vp, a.v_ss, v_off, t + 1);
     }
-    const int k0 = t * kBlockN;
+    const int k0 = t * kBlockN + 32 * part;  // first key of the wave's share of the tile
+    constexpr int kKeys = kBlockN / kParts;
+    kt += part * kKeyBlockBytes<D>;
+    vt += part * 2 * kKeyStepBytes<D>;
     // A wave that sees no key of this tile sees none of the later ones either (causal).
-    const bool active = !(a.causal && k0 > wave_limit);
+    const bool active = k0 < a.seqlen_k && !(a.causal && k0 > wave_limit);
     if (active) {
       // S^T = K Q^T, K fragments read kAhead steps ahead of their MFMAs.
       constexpr int kSteps = D / 16;
@@ -180,33 +192,33 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
         for (int ks = 0; ks < kAhead; ++ks) {
           a0[ks] = lds_load16(kt, k_lds[ks]);
-          a1[ks] = lds_load16(kt + kKeyBlockBytes<D>, k_lds[ks]);
+          if constexpr (kWhole) a1[ks] = lds_load16(kt + kKeyBlockBytes<D>, k_lds[ks]);
         }
 #pragma unroll
         for (int ks = 0; ks < kSteps; ++ks) {
           if (ks + kAhead < kSteps) {
             a0[ks + kAhead] = lds_load16(kt, k_lds[ks + kAhead]);
-            a1[ks + kAhead] = lds_load16(kt + kKeyBlockBytes<D>, k_lds[ks + kAhead]);
+            if constexpr (kWhole) a1[ks + kAhead] = lds_load16(kt + kKeyBlockBytes<D>, k_lds[ks + kAhead]);
           }
           s0 = E::mfma32(a0[ks], qf[ks], s0);
-          s1 = E::mfma32(a1[ks], qf[ks], s1);
+          if constexpr (kWhole) s1 = E::mfma32(a1[ks], qf[ks], s1);
         }
 #if FL_PREFILL_QK_SCHED
         // Keep the reads kAhead steps ahead: the scheduler otherwise pulls each read down to its
         // MFMA and the LDS latency is exposed on every step.
-        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * kAhead, 1);
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 / kParts * kAhead, 1);
 #pragma unroll
         for (int ks = 0; ks < kSteps - kAhead; ++ks) {
-          __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2, 1);
-          __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 1);
+          __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2 / kParts, 1);
+          __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 / kParts, 1);
         }
-        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2 * kAhead, 1);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 2 / kParts * kAhead, 1);
 #endif
       }
       // Keys past the end or above the diagonal: only edge and diagonal tiles (wave-uniform
       // branch; the empty asm keeps the compiler from turning it into selects on every tile).
-      if ((k0 + kBlockN > a.seqlen_k) ||
-          (a.causal && k0 + kBlockN - 1 > first_limit)) {
+      if ((k0 + kKeys > a.seqlen_k) ||
+          (a.causal && k0 + kKeys - 1 > first_limit)) {
         asm volatile("" ::: "memory");
         // acc_key(j, half) = acc_key(j, 0) + 4 half: fold the lane's part into the limit so every
         // comparison is against a compile-time constant (no per-key registers live in the loop).
@@ -216,7 +228,7 @@ __global__ void __launch_bounds__(kThreads)
           constexpr int kBase = 0;
           const int kj = acc_key(j, kBase);
           if (kj > lim) s0[j] = -INFINITY;
-          if (kj + 32 > lim) s1[j] = -INFINITY;
+          if (kWhole && kj + 32 > lim) s1[j] = -INFINITY;
         }
       }
       // Online softmax in the exp2 domain on raw scores: with scale > 0,
@@ -224,7 +236,7 @@ __global__ void __launch_bounds__(kThreads)
       // `ref` of o and l moves to the row's running max when it has grown by more than
       // kMoveSlack over it (prefill_tile.hpp), so probabilities stay at most 2^kMoveSlack and most
       // tiles of a long row skip the rescale of o.
-      float mx = max_of(s0, s1);
+      float mx = kWhole ? max_of(s0, s1) : max_of(s0);
       mx = max2_f32(mx, xor_lane(mx, 32));
       const float cand = mx * sl2;  // -inf while the row has seen only hidden keys
       const bool move = cand > ref + kMoveSlack;
@@ -242,15 +254,17 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         s0[j] = exp2_fast(fmaf(s0[j], sl2, -shift));
-        s1[j] = exp2_fast(fmaf(s1[j], sl2, -shift));
         rs0 += s0[j];
-        rs1 += s1[j];
+        if constexpr (kWhole) {
+          s1[j] = exp2_fast(fmaf(s1[j], sl2, -shift));
+          rs1 += s1[j];
+        }
       }
       l = fmaf(l, alpha, rs0 + rs1);
       const u32x4 pf[4] = {p_frag<Tag, 0>(s0), p_frag<Tag, 1>(s0), p_frag<Tag, 0>(s1),
                            p_frag<Tag, 1>(s1)};
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
+      for (int kk = 0; kk < 4 / kParts; ++kk) {
 #pragma unroll
         for (int nb = 0; nb < D / 32; ++nb) {
           const u32x4 vf = v_frag_at(vt + kk * kKeyStepBytes<D>, v_lds[nb][0], v_lds[nb][1]);
@@ -274,7 +288,41 @@ __global__ void __launch_bounds__(kThreads)
   }
 
   // Epilogue: l over both halves, 1/l (0 for rows that saw no key, which then store zeros).
-  const float lt = l + xor_lane(l, 32);
+  float lt = l + xor_lane(l, 32);
+  if constexpr (!kWhole) {
+    // The second key blocks' waves leave their state in the tile slots (free: the loop ends with a
+    // barrier), 1 KiB per store instruction, and the first ones' take it up. A row without a key in a
+    // part has ref = -inf and l = 0 there.
+    // Row wave r's state: planes of 64 lanes x 16 bytes, D / 8 of o and one of ref and l. r = 0 in the
+    // K slots, r = 1 in the V slots (each D / 8 planes long: the last plane opens the second slot).
+    static_assert(kRowWaves == 2 && 2 * kTile == D / 8 * 1024, "a slot holds a state's output");
+    const bool upper = wave % kRowWaves != 0;
+    auto plane = [&](int n) {
+      uint16_t* slot = n < D / 8 ? (upper ? v_lds0 : k_lds0) : (upper ? v_lds1 : k_lds1);
+      return reinterpret_cast<f32x4*>(slot) + n % (D / 8) * 64 + lane;
+    };
+    if (part == 1) {
+#pragma unroll
+      for (int n = 0; n < D / 8; ++n)
+        *plane(n) = f32x4{o[n / 4][4 * (n % 4)], o[n / 4][4 * (n % 4) + 1], o[n / 4][4 * (n % 4) + 2],
+                          o[n / 4][4 * (n % 4) + 3]};
+      *plane(D / 8) = f32x4{ref, lt, 0.f, 0.f};
+    }
+    __syncthreads();
+    if (part == 1) return;
+    const f32x4 other = *plane(D / 8);
+    const float top = fmaxf(ref, other[0]);
+    const float f0 = ref == -INFINITY ? 0.f : exp2_fast(ref - top);
+    const float f1 = other[0] == -INFINITY ? 0.f : exp2_fast(other[0] - top);
+#pragma unroll
+    for (int n = 0; n < D / 8; ++n) {
+      const f32x4 x = *plane(n);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[n / 4][4 * (n % 4) + e] = o[n / 4][4 * (n % 4) + e] * f0 + x[e] * f1;
+    }
+    lt = lt * f0 + other[1] * f1;
+    ref = top;
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   if (my_row < a.rows) {
     uint16_t* orow = a.o + b * a.o_bs + my_pos * a.o_ss + (h + my_head) * a.o_hs;
@@ -352,12 +400,27 @@ __global__ void __launch_bounds__(64) mfma_tile_test_kernel(const uint16_t* a, c
   }
 }
 
-template <typename Tag, int D>
-hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
-  args.q_blocks = (args.rows + kBlockM - 1) / kBlockM;
+template <typename Tag, int D, int kParts>
+hipError_t launch_parts(PrefillArgs args, hipStream_t stream) {
+  constexpr int kRows = kBlockM / kParts;
+  args.q_blocks = (args.rows + kRows - 1) / kRows;
   const int blocks = args.q_blocks * args.batch * args.work_heads;
-  hipLaunchKernelGGL((prefill_fwd_kernel<Tag, D>), dim3(blocks), dim3(kThreads), 0, stream, args);
+  hipLaunchKernelGGL((prefill_fwd_kernel<Tag, D, kParts>), dim3(blocks), dim3(kThreads), 0, stream, args);
   return hipGetLastError();
+}
+
+// Half tiles per wave (kParts = 2) where 128-row blocks leave CUs idle or nearly so: up to 192 of them
+// (256 for long causal calls, whose last blocks run alone), of more than one tile. Device us, whole /
+// half, bf16: (1, 32, 8, 512, 128) causal (128 blocks) 14.0 / 10.9, (1, 32, 8, 256, 128) (64) 9.8 / 7.7,
+// (1, 16, 16, 1000, 64) (128) 17.1 / 11.6, (5, 16, 2, 197, 128) full (130) 9.9 / 8.4, (1, 32, 8, 1024,
+// 128) causal (256) 24.4 / 21.1; not (3, 32, 8, 300, 128) causal (240) 12.2 / 12.7, (2, 32, 8, 447, 128)
+// full (224) 15.1 / 15.3, (7, 32, 8, 176, 128) full (336) 13.6 / 16.6, (1, 32, 8, 64, 128) 5.2 / 5.5.
+template <typename Tag, int D>
+hipError_t launch_typed(const PrefillArgs& args, hipStream_t stream) {
+  const int64_t blocks = static_cast<int64_t>((args.rows + kBlockM - 1) / kBlockM) * args.batch * args.work_heads;
+  const int most = args.causal && args.seqlen_k >= 10 * kBlockN ? 256 : 192;
+  if (blocks <= most && args.seqlen_k > kBlockN) return launch_parts<Tag, D, 2>(args, stream);
+  return launch_parts<Tag, D, 1>(args, stream);
 }
 
 }  // namespace

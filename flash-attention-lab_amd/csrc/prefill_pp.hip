@@ -845,10 +845,10 @@ int prefill_pp_block_rows(int head_dim) {
 // D; causal, bf16): a 64-key tile of a block takes 1.1 us, 0.8 where only one group of waves has rows,
 // and up to 0.3 more as the CUs fill; a block's start and end 5, the second launch and the merge 6,
 // and the partials 0.45 per MB to memory and back. Measured without splits / at the planned count:
-// (1, 32, 8, 300, 8492, 128) 147 / 49, (1, 32, 8, 16, 8192, 128) 138 / 20, (1, 32, 8, 512, 4096, 128)
-// 72 / 44, (1, 64, 8, 18, 1212, 128) 23 / 15, (1, 8, 8, 5000, 5000, 64) 68 / 48; calls whose blocks
+// (1, 32, 8, 300, 8492, 128) 107 / 51, (1, 32, 8, 16, 2048, 128) 27 / 12, (1, 32, 8, 512, 4096, 128)
+// 56 / 45, (1, 64, 8, 18, 1212, 128) 18 / 14, (1, 32, 32, 1, 5000, 128) 71 / 23; calls whose blocks
 // fill the CUs gain nothing ((1, 32, 8, 2048, 2048, 128) 49, 60 with two splits), nor do short ones
-// ((1, 32, 8, 512, 512, 128) 14, 24 with two).
+// ((1, 32, 8, 512, 1024, 128) 17, 28 with two).
 int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count) {
   if (knob(FL_KNOB_PREFILL_PP_MIN_WG) >= 0 || knob(FL_KNOB_PREFILL_CAUSAL_STREAM) >= 0) return 1;
   const int cus = cu_count > 0 ? cu_count : 256;
@@ -872,10 +872,15 @@ int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count) {
     const double all = (blocks * n + cus - 1) / cus * (mean / n * tile + 5.0);
     return (alone > all ? alone : all) + (n == 1 ? 3.0 : 6.0 + 0.1 * n + 0.45 * n * mb);
   };
-  // Without splits: this kernel, or the 4-wave one on blocks of 128 rows, one or two to a CU.
-  const double small_wgs =
-      double((args.seqlen_q + kPrefillBlockM - 1) / kPrefillBlockM) * args.batch * args.heads * mean / longest;
-  const double small = 4.0 + 1.1 * longest * (small_wgs > cus ? small_wgs / cus : 1.0);
+  // Without splits: this kernel, or the 4-wave one on blocks of 128 rows (packed where abi.hip packs
+  // them): a tile in 0.78 us (0.52 at head_dim 64) on half tiles per wave, and with more than 128 blocks
+  // in 1.1 us for as many as there are CUs.
+  const double packed = double((args.rows + kPrefillBlockM - 1) / kPrefillBlockM) * args.batch * args.work_heads;
+  const double single = double((args.seqlen_q + kPrefillBlockM - 1) / kPrefillBlockM) * args.batch * args.heads;
+  const double small_wgs = packed < 128 ? single : packed;
+  const double small_tile = small_wgs > 128 ? 1.1 : head_dim == 64 ? 0.52 : 0.78;
+  const double load = small_wgs * mean / longest / cus;
+  const double small = 4.0 + small_tile * longest * (load > 1.0 ? load : 1.0);
   double least = 0.95 * (small < time(1) ? small : time(1));
   int best = 1;
   for (int n = 2; n <= kMaxPrefillSplits && n <= longest; ++n) {

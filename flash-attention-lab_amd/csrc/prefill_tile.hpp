@@ -148,4 +148,12 @@ __device__ __forceinline__ float max_of(const f32x16& x, const f32x16& y) {
   return max2_f32(max3_f32(u0, u1, u2), u3);
 }
 
+// Max of the 16 scores of one 32-key block.
+__device__ __forceinline__ float max_of(const f32x16& x) {
+  float t[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) t[i] = max3_f32(x[3 * i], x[3 * i + 1], x[3 * i + 2]);
+  return max2_f32(max3_f32(t[0], t[1], t[2]), max3_f32(t[3], t[4], x[15]));
+}
+
 }  // namespace fl::prefill
