@@ -303,235 +303,235 @@ decode_split_kernel(const DecodeArgs a) {
     end = min(pos + sched.chunk, sched.total);
   }
   while (pos < end) {  // (once, where not balanced)
-  int b, head, k_begin, k_end, head_step;
-  int64_t partial;  // index of the segment's first partial; the next head's is head_step on
-  if constexpr (kBalanced) {
-    const Segment g = segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
-    pos = g.next;
-    if (g.k_begin == g.k_end) continue;
-    b = g.b;
-    head = g.head;
-    k_begin = g.k_begin;
-    k_end = g.k_end;
-    partial = g.slot * (kSpan * kHeads);
-    head_step = 1;
-  } else {
-    pos = end;
-    const int split = blockIdx.x % a.num_splits;
-    const int work = blockIdx.x / a.num_splits;
-    b = work / rows;
-    head = work - b * rows;
-    // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
-    // out-of-range value cannot read outside it.
-    const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
-    const int per_split =
-        ((len + a.num_splits - 1) / a.num_splits + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
-    k_begin = split * per_split;
-    k_end = min(len, k_begin + per_split);
-    partial = (static_cast<int64_t>(b) * a.heads + (head / a.head_chunks * kSpan) * a.group +
-               head % a.head_chunks * kHeads) * a.num_splits + split;
-    head_step = a.num_splits;
-  }
-  const int hblk = head / a.head_chunks;
-  const int hchunk = head - hblk * a.head_chunks;
-  const int hkv = hblk * kSpan + sp;
-  const int h0 = hkv * a.group + hchunk * kHeads;
+    int b, head, k_begin, k_end, head_step;
+    int64_t partial;  // index of the segment's first partial; the next head's is head_step on
+    if constexpr (kBalanced) {
+      const Segment g = segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
+      pos = g.next;
+      if (g.k_begin == g.k_end) continue;
+      b = g.b;
+      head = g.head;
+      k_begin = g.k_begin;
+      k_end = g.k_end;
+      partial = g.slot * (kSpan * kHeads);
+      head_step = 1;
+    } else {
+      pos = end;
+      const int split = blockIdx.x % a.num_splits;
+      const int work = blockIdx.x / a.num_splits;
+      b = work / rows;
+      head = work - b * rows;
+      // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
+      // out-of-range value cannot read outside it.
+      const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
+      const int per_split =
+          ((len + a.num_splits - 1) / a.num_splits + kKeysPerIter - 1) / kKeysPerIter * kKeysPerIter;
+      k_begin = split * per_split;
+      k_end = min(len, k_begin + per_split);
+      partial = (static_cast<int64_t>(b) * a.heads + (head / a.head_chunks * kSpan) * a.group +
+                 head % a.head_chunks * kHeads) * a.num_splits + split;
+      head_step = a.num_splits;
+    }
+    const int hblk = head / a.head_chunks;
+    const int hchunk = head - hblk * a.head_chunks;
+    const int hkv = hblk * kSpan + sp;
+    const int h0 = hkv * a.group + hchunk * kHeads;
 
-  typename P::QPiece q[kHeads];
+    typename P::QPiece q[kHeads];
 #pragma unroll
-  for (int g = 0; g < kHeads; ++g) {
-    const S* qrow = static_cast<const S*>(a.q) + b * a.q_bs + (h0 + g) * a.q_hs;
-    q[g] = P::load_q(qrow + piece * kEPL);
-  }
-  const float sl2 = a.scale_log2;  // scores are q.k * scale_log2 (log2 domain)
+    for (int g = 0; g < kHeads; ++g) {
+      const S* qrow = static_cast<const S*>(a.q) + b * a.q_bs + (h0 + g) * a.q_hs;
+      q[g] = P::load_q(qrow + piece * kEPL);
+    }
+    const float sl2 = a.scale_log2;  // scores are q.k * scale_log2 (log2 domain)
 
-  float o[kHeads][kEPL];
-  float m[kHeads];  // running max, log2 units (same on every lane of a row group)
-  float l[kHeads];  // running sum (same on every lane of a row group)
+    float o[kHeads][kEPL];
+    float m[kHeads];  // running max, log2 units (same on every lane of a row group)
+    float l[kHeads];  // running sum (same on every lane of a row group)
 #pragma unroll
-  for (int g = 0; g < kHeads; ++g) {
-    m[g] = -INFINITY;
-    l[g] = 0.f;
+    for (int g = 0; g < kHeads; ++g) {
+      m[g] = -INFINITY;
+      l[g] = 0.f;
 #pragma unroll
-    for (int e = 0; e < kEPL; ++e) o[g][e] = 0.f;
-  }
+      for (int e = 0; e < kEPL; ++e) o[g][e] = 0.f;
+    }
 
-  // Contiguous cache: rows of sequence b at b * bs + key * ss. Paged cache
-  // ([num_blocks, page_size, H_kv, D]): key lives in block block_tables[b][key / page_size], row
-  // key % page_size, block numbers clamped to the pool so a bad table entry cannot read outside
-  // it. kPagedLds stages the split's block numbers in LDS once (the host picks it when every split
-  // touches at most kMaxSplitPages blocks): LDS reads do not wait behind the rows in flight.
-  // kPagedGlobal reads each block number from the table in global memory.
-  __shared__ int page_table[kPageMode == kPagedLds ? kMaxSplitPages : 1];
-  int page0 = 0;
-  const int32_t* table_row = nullptr;
-  if constexpr (kPaged) table_row = a.block_tables + static_cast<int64_t>(b) * a.block_tables_stride;
-  if constexpr (kPageMode == kPagedLds) {
-    if (k_begin < k_end) {
-      page0 = k_begin / a.page_size;
-      const int pages = (k_end - 1) / a.page_size - page0 + 1;
-      for (int i = tid; i < pages; i += kThreads)
-        page_table[i] = min(max(table_row[page0 + i], 0), a.num_blocks - 1);
+    // Contiguous cache: rows of sequence b at b * bs + key * ss. Paged cache
+    // ([num_blocks, page_size, H_kv, D]): key lives in block block_tables[b][key / page_size], row
+    // key % page_size, block numbers clamped to the pool so a bad table entry cannot read outside
+    // it. kPagedLds stages the split's block numbers in LDS once (the host picks it when every split
+    // touches at most kMaxSplitPages blocks): LDS reads do not wait behind the rows in flight.
+    // kPagedGlobal reads each block number from the table in global memory.
+    __shared__ int page_table[kPageMode == kPagedLds ? kMaxSplitPages : 1];
+    int page0 = 0;
+    const int32_t* table_row = nullptr;
+    if constexpr (kPaged) table_row = a.block_tables + static_cast<int64_t>(b) * a.block_tables_stride;
+    if constexpr (kPageMode == kPagedLds) {
+      if (k_begin < k_end) {
+        page0 = k_begin / a.page_size;
+        const int pages = (k_end - 1) / a.page_size - page0 + 1;
+        for (int i = tid; i < pages; i += kThreads)
+          page_table[i] = min(max(table_row[page0 + i], 0), a.num_blocks - 1);
+      }
+      __syncthreads();
+    }
+    const S* kbase = static_cast<const S*>(a.k) + (kPaged ? 0 : b * a.k_bs) + hkv * a.k_hs + piece * kEPL;
+    const S* vbase = static_cast<const S*>(a.v) + (kPaged ? 0 : b * a.v_bs) + hkv * a.v_hs + piece * kEPL;
+    // (block, row) of a key; page sizes that are powers of two (the usual ones) take a shift.
+    auto locate = [&](int key, int& block, int& row) {
+      const int page = a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size;
+      if constexpr (kPageMode == kPagedLds) {
+        block = page_table[page - page0];
+      } else {
+        block = min(max(table_row[page], 0), a.num_blocks - 1);
+      }
+      row = key - page * a.page_size;
+    };
+    auto k_row = [&](int key) -> const S* {
+      if constexpr (kPaged) {
+        int block, row;
+        locate(key, block, row);
+        return kbase + static_cast<int64_t>(block) * a.k_bs + static_cast<int64_t>(row) * a.k_ss;
+      } else {
+        return kbase + static_cast<int64_t>(key) * a.k_ss;
+      }
+    };
+    auto v_row = [&](int key) -> const S* {
+      if constexpr (kPaged) {
+        int block, row;
+        locate(key, block, row);
+        return vbase + static_cast<int64_t>(block) * a.v_bs + static_cast<int64_t>(row) * a.v_ss;
+      } else {
+        return vbase + static_cast<int64_t>(key) * a.v_ss;
+      }
+    };
+
+    // Batches of kKeysPerIter keys, double-buffered in registers: the next batch's loads are issued
+    // before the current batch is used, so each wave keeps rows in flight while it computes. Keys past
+    // the split's end are clamped to its last row (always a valid, finite row) and masked out of the
+    // softmax, so every load is issued unconditionally.
+    auto load_batch = [&](int base, u32x4 (&kr)[kUnroll], u32x4 (&vr)[kUnroll]) {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const int key = min(base + u * kGroups + group, k_end - 1);
+        kr[u] = load16_stream(k_row(key));
+        vr[u] = load16_stream(v_row(key));
+      }
+    };
+    auto use_batch = [&](int base, const u32x4 (&kr)[kUnroll], const u32x4 (&vr)[kUnroll]) {
+#pragma unroll
+      for (int g = 0; g < kHeads; ++g) {
+        float s[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+          const float dot = group_sum<kLPR>(P::dot(q[g], kr[u])) * sl2;
+          s[u] = base + u * kGroups + group < k_end ? dot : -INFINITY;
+        }
+        float mx = s[0];
+#pragma unroll
+        for (int u = 1; u < kUnroll; ++u) mx = fmaxf(mx, s[u]);
+        const float m_new = fmaxf(m[g], mx);
+        const float ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = exp2_fast(m[g] - ref);
+        m[g] = m_new;
+        float lsum = l[g] * alpha;
+#pragma unroll
+        for (int e = 0; e < kEPL; ++e) o[g][e] *= alpha;
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) {
+          const float p = exp2_fast(s[u] - ref);
+          lsum += p;
+#pragma unroll
+          for (int e = 0; e < kEPL; ++e) o[g][e] = fmaf(p, P::elem(vr[u], e), o[g][e]);
+        }
+        l[g] = lsum;
+      }
+    };
+    // The prefetches are unconditional (past the end they re-read the split's last row, which the
+    // cache serves), and a scheduling barrier keeps them ahead of the current batch's use. Without
+    // either, the compiler waits for every load in flight, the prefetch included, before it uses the
+    // current batch, or moves the K loads down to their dot products: one batch in flight instead of
+    // two (B1-MHA 89.2 -> 88.5 us, B=1 with 8 KV heads on this kernel 41.8 -> 38.3 us).
+    u32x4 ka[kUnroll], va[kUnroll], kb[kUnroll], vb[kUnroll];
+    if (k_begin < k_end) load_batch(k_begin, ka, va);
+    for (int base = k_begin; base < k_end; base += 2 * kKeysPerIter) {
+      load_batch(base + kKeysPerIter, kb, vb);
+      __builtin_amdgcn_sched_barrier(0);
+      use_batch(base, ka, va);
+      if (base + kKeysPerIter >= k_end) break;
+      load_batch(base + 2 * kKeysPerIter, ka, va);
+      __builtin_amdgcn_sched_barrier(0);
+      use_batch(base + kKeysPerIter, kb, vb);
+    }
+
+    // Merge the row groups of this wave: butterfly over lanes with the same piece.
+#pragma unroll
+    for (int mask = kLPK; mask < 64; mask <<= 1) {
+#pragma unroll
+      for (int g = 0; g < kHeads; ++g) {
+        const float m_o = __shfl_xor(m[g], mask);
+        const float l_o = __shfl_xor(l[g], mask);
+        const float m_new = fmaxf(m[g], m_o);
+        // Groups without keys (m = -inf) contribute nothing; two empty groups stay empty.
+        const float f = m[g] == -INFINITY ? 0.f : exp2_fast(m[g] - m_new);
+        const float f_o = m_o == -INFINITY ? 0.f : exp2_fast(m_o - m_new);
+        l[g] = l[g] * f + l_o * f_o;
+#pragma unroll
+        for (int e = 0; e < kEPL; ++e) {
+          const float o_o = __shfl_xor(o[g][e], mask);
+          o[g][e] = o[g][e] * f + o_o * f_o;
+        }
+        m[g] = m_new;
+      }
+    }
+    if (lane < kLPK) {  // row group 0 of the wave: one lane per (head of the span, piece)
+#pragma unroll
+      for (int g = 0; g < kHeads; ++g) {
+#pragma unroll
+        for (int e = 0; e < kEPL; ++e) red_o[wave][sp * kHeads + g][piece * kEPL + e] = o[g][e];
+        if (piece == 0) {
+          red_m[wave][sp * kHeads + g] = m[g];
+          red_l[wave][sp * kHeads + g] = l[g];
+        }
+      }
     }
     __syncthreads();
-  }
-  const S* kbase = static_cast<const S*>(a.k) + (kPaged ? 0 : b * a.k_bs) + hkv * a.k_hs + piece * kEPL;
-  const S* vbase = static_cast<const S*>(a.v) + (kPaged ? 0 : b * a.v_bs) + hkv * a.v_hs + piece * kEPL;
-  // (block, row) of a key; page sizes that are powers of two (the usual ones) take a shift.
-  auto locate = [&](int key, int& block, int& row) {
-    const int page = a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size;
-    if constexpr (kPageMode == kPagedLds) {
-      block = page_table[page - page0];
-    } else {
-      block = min(max(table_row[page], 0), a.num_blocks - 1);
-    }
-    row = key - page * a.page_size;
-  };
-  auto k_row = [&](int key) -> const S* {
-    if constexpr (kPaged) {
-      int block, row;
-      locate(key, block, row);
-      return kbase + static_cast<int64_t>(block) * a.k_bs + static_cast<int64_t>(row) * a.k_ss;
-    } else {
-      return kbase + static_cast<int64_t>(key) * a.k_ss;
-    }
-  };
-  auto v_row = [&](int key) -> const S* {
-    if constexpr (kPaged) {
-      int block, row;
-      locate(key, block, row);
-      return vbase + static_cast<int64_t>(block) * a.v_bs + static_cast<int64_t>(row) * a.v_ss;
-    } else {
-      return vbase + static_cast<int64_t>(key) * a.v_ss;
-    }
-  };
 
-  // Batches of kKeysPerIter keys, double-buffered in registers: the next batch's loads are issued
-  // before the current batch is used, so each wave keeps rows in flight while it computes. Keys past
-  // the split's end are clamped to its last row (always a valid, finite row) and masked out of the
-  // softmax, so every load is issued unconditionally.
-  auto load_batch = [&](int base, u32x4 (&kr)[kUnroll], u32x4 (&vr)[kUnroll]) {
+    // Merge the four waves in order and write o/lse (one split) or the partials.
+    for (int idx = tid; idx < kSpan * kHeads * D; idx += kThreads) {
+      const int g = idx / D;  // (head of the span) * kHeads + query head
+      const int d = idx - g * D;
+      float mm = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int key = min(base + u * kGroups + group, k_end - 1);
-      kr[u] = load16_stream(k_row(key));
-      vr[u] = load16_stream(v_row(key));
-    }
-  };
-  auto use_batch = [&](int base, const u32x4 (&kr)[kUnroll], const u32x4 (&vr)[kUnroll]) {
+      for (int wv = 0; wv < kWaves; ++wv) mm = fmaxf(mm, red_m[wv][g]);
+      float num = 0.f;
+      float den = 0.f;
 #pragma unroll
-    for (int g = 0; g < kHeads; ++g) {
-      float s[kUnroll];
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const float dot = group_sum<kLPR>(P::dot(q[g], kr[u])) * sl2;
-        s[u] = base + u * kGroups + group < k_end ? dot : -INFINITY;
+      for (int wv = 0; wv < kWaves; ++wv) {
+        const float mw = red_m[wv][g];
+        if (mw != -INFINITY) {
+          const float f = exp2_fast(mw - mm);
+          num += red_o[wv][g][d] * f;
+          den += red_l[wv][g] * f;
+        }
       }
-      float mx = s[0];
-#pragma unroll
-      for (int u = 1; u < kUnroll; ++u) mx = fmaxf(mx, s[u]);
-      const float m_new = fmaxf(m[g], mx);
-      const float ref = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = exp2_fast(m[g] - ref);
-      m[g] = m_new;
-      float lsum = l[g] * alpha;
-#pragma unroll
-      for (int e = 0; e < kEPL; ++e) o[g][e] *= alpha;
-#pragma unroll
-      for (int u = 0; u < kUnroll; ++u) {
-        const float p = exp2_fast(s[u] - ref);
-        lsum += p;
-#pragma unroll
-        for (int e = 0; e < kEPL; ++e) o[g][e] = fmaf(p, P::elem(vr[u], e), o[g][e]);
-      }
-      l[g] = lsum;
-    }
-  };
-  // The prefetches are unconditional (past the end they re-read the split's last row, which the
-  // cache serves), and a scheduling barrier keeps them ahead of the current batch's use. Without
-  // either, the compiler waits for every load in flight, the prefetch included, before it uses the
-  // current batch, or moves the K loads down to their dot products: one batch in flight instead of
-  // two (B1-MHA 89.2 -> 88.5 us, B=1 with 8 KV heads on this kernel 41.8 -> 38.3 us).
-  u32x4 ka[kUnroll], va[kUnroll], kb[kUnroll], vb[kUnroll];
-  if (k_begin < k_end) load_batch(k_begin, ka, va);
-  for (int base = k_begin; base < k_end; base += 2 * kKeysPerIter) {
-    load_batch(base + kKeysPerIter, kb, vb);
-    __builtin_amdgcn_sched_barrier(0);
-    use_batch(base, ka, va);
-    if (base + kKeysPerIter >= k_end) break;
-    load_batch(base + 2 * kKeysPerIter, ka, va);
-    __builtin_amdgcn_sched_barrier(0);
-    use_batch(base + kKeysPerIter, kb, vb);
-  }
-
-  // Merge the row groups of this wave: butterfly over lanes with the same piece.
-#pragma unroll
-  for (int mask = kLPK; mask < 64; mask <<= 1) {
-#pragma unroll
-    for (int g = 0; g < kHeads; ++g) {
-      const float m_o = __shfl_xor(m[g], mask);
-      const float l_o = __shfl_xor(l[g], mask);
-      const float m_new = fmaxf(m[g], m_o);
-      // Groups without keys (m = -inf) contribute nothing; two empty groups stay empty.
-      const float f = m[g] == -INFINITY ? 0.f : exp2_fast(m[g] - m_new);
-      const float f_o = m_o == -INFINITY ? 0.f : exp2_fast(m_o - m_new);
-      l[g] = l[g] * f + l_o * f_o;
-#pragma unroll
-      for (int e = 0; e < kEPL; ++e) {
-        const float o_o = __shfl_xor(o[g][e], mask);
-        o[g][e] = o[g][e] * f + o_o * f_o;
-      }
-      m[g] = m_new;
-    }
-  }
-  if (lane < kLPK) {  // row group 0 of the wave: one lane per (head of the span, piece)
-#pragma unroll
-    for (int g = 0; g < kHeads; ++g) {
-#pragma unroll
-      for (int e = 0; e < kEPL; ++e) red_o[wave][sp * kHeads + g][piece * kEPL + e] = o[g][e];
-      if (piece == 0) {
-        red_m[wave][sp * kHeads + g] = m[g];
-        red_l[wave][sp * kHeads + g] = l[g];
+      const int h = (hblk * kSpan + g / kHeads) * a.group + hchunk * kHeads + g % kHeads;
+      if (a.num_splits == 1) {
+        S* orow = static_cast<S*>(a.o) + b * a.o_bs + h * a.o_hs;
+        orow[d] = Elem<Tag>::from_float(den > 0.f ? num / den : 0.f);
+        if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
+      } else {
+        const int64_t slot =
+            partial + static_cast<int64_t>(kBalanced ? g : h - hblk * kSpan * a.group - hchunk * kHeads) * head_step;
+        a.partial_o[slot * D + d] = num;
+        if (d == 0) {
+          a.partial_ml[2 * slot] = mm;
+          a.partial_ml[2 * slot + 1] = den;
+        }
       }
     }
-  }
-  __syncthreads();
-
-  // Merge the four waves in order and write o/lse (one split) or the partials.
-  for (int idx = tid; idx < kSpan * kHeads * D; idx += kThreads) {
-    const int g = idx / D;  // (head of the span) * kHeads + query head
-    const int d = idx - g * D;
-    float mm = -INFINITY;
-#pragma unroll
-    for (int wv = 0; wv < kWaves; ++wv) mm = fmaxf(mm, red_m[wv][g]);
-    float num = 0.f;
-    float den = 0.f;
-#pragma unroll
-    for (int wv = 0; wv < kWaves; ++wv) {
-      const float mw = red_m[wv][g];
-      if (mw != -INFINITY) {
-        const float f = exp2_fast(mw - mm);
-        num += red_o[wv][g][d] * f;
-        den += red_l[wv][g] * f;
-      }
-    }
-    const int h = (hblk * kSpan + g / kHeads) * a.group + hchunk * kHeads + g % kHeads;
-    if (a.num_splits == 1) {
-      S* orow = static_cast<S*>(a.o) + b * a.o_bs + h * a.o_hs;
-      orow[d] = Elem<Tag>::from_float(den > 0.f ? num / den : 0.f);
-      if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
-    } else {
-      const int64_t slot =
-          partial + static_cast<int64_t>(kBalanced ? g : h - hblk * kSpan * a.group - hchunk * kHeads) * head_step;
-      a.partial_o[slot * D + d] = num;
-      if (d == 0) {
-        a.partial_ml[2 * slot] = mm;
-        a.partial_ml[2 * slot + 1] = den;
-      }
-    }
-  }
-  if constexpr (!kBalanced) return;
-  if (pos < end) __syncthreads();  // the next segment reuses the merge's LDS
+    if constexpr (!kBalanced) return;
+    if (pos < end) __syncthreads();  // the next segment reuses the merge's LDS
   }
 }
 

@@ -116,276 +116,276 @@ __global__ void __launch_bounds__(kThreads) decode_mfma_kernel(const DecodeArgs 
     end = min(pos + sched.chunk, sched.total);
   }
   while (pos < end) {  // (once, where not balanced)
-  int b, hq, k_begin, k_end, head_step;
-  int64_t partial;  // index of the segment's first partial; the next head's is head_step on
-  if constexpr (kBalanced) {
-    const decode::Segment g = decode::segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
-    pos = g.next;
-    if (g.k_begin == g.k_end) continue;
-    b = g.b;
-    hq = g.head;
-    k_begin = g.k_begin;
-    k_end = g.k_end;
-    partial = g.slot * (span * group);
-    head_step = 1;
-  } else {
-    pos = end;
-    const int split = blockIdx.x % a.num_splits;
-    const int work = blockIdx.x / a.num_splits;
-    b = work / rows;
-    hq = work - b * rows;
-    // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
-    // out-of-range value cannot read outside it.
-    const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
-    const int per_split =
-        ((len + a.num_splits - 1) / a.num_splits + kTileKeys - 1) / kTileKeys * kTileKeys;
-    k_begin = split * per_split;
-    k_end = min(len, k_begin + per_split);
-    partial = (static_cast<int64_t>(b) * a.heads + hq * span * group) * a.num_splits + split;
-    head_step = a.num_splits;
-  }
-  const int hkv = span == 1 ? hq : hq * span + wave;
-  const int h0 = hkv * group;
-  const int tiles = k_begin < k_end ? (k_end - k_begin + kTileKeys - 1) / kTileKeys : 0;
-  const int my_tiles = span == 1 ? (tiles > wave ? (tiles - wave + kWaves - 1) / kWaves : 0) : tiles;
-
-  // Q^T, the B operand: lane (col, half) holds q[h0 + col][16 ks + 8 half .. + 7], zero past the
-  // group.
-  u32x4 qf[D / 16];
-  {
-    const bool ok = col < group;
-    const uint16_t* qrow =
-        static_cast<const uint16_t*>(a.q) + b * a.q_bs + (h0 + (ok ? col : 0)) * a.q_hs + 8 * half;
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) qf[ks] = ok ? load16(qrow + 16 * ks) : u32x4{0, 0, 0, 0};
-  }
-
-  // Paged cache: the split's block numbers, clamped to the pool (kPagedLds), or the table row.
-  __shared__ int page_table[kPageMode == kPagedLds ? kMaxSplitPages : 1];
-  int page0 = 0;
-  const int32_t* table_row = nullptr;
-  if constexpr (kPaged) table_row = a.block_tables + static_cast<int64_t>(b) * a.block_tables_stride;
-  if constexpr (kPageMode == kPagedLds) {
-    if (k_begin < k_end) {
-      page0 = k_begin / a.page_size;
-      const int pages = (k_end - 1) / a.page_size - page0 + 1;
-      for (int i = tid; i < pages; i += kThreads)
-        page_table[i] = min(max(table_row[page0 + i], 0), a.num_blocks - 1);
-    }
-    __syncthreads();
-  }
-
-  // Tile loads: load j of a tensor tile gives lane l row kRowsPerLoad j + l / kChunksPerRow, chunk
-  // l % kChunksPerRow (whole rows per instruction), which it stores at that row's swizzled chunk.
-  const int lane_row = lane / kChunksPerRow;
-  const int lane_col = 8 * (lane % kChunksPerRow);
-  const uint16_t* kbase =
-      static_cast<const uint16_t*>(a.k) + (kPaged ? 0 : b * a.k_bs) + hkv * a.k_hs + lane_col;
-  const uint16_t* vbase =
-      static_cast<const uint16_t*>(a.v) + (kPaged ? 0 : b * a.v_bs) + hkv * a.v_hs + lane_col;
-  // Offsets (elements) of a key's K and V rows from kbase / vbase.
-  auto row_offsets = [&](int key, int64_t& ko, int64_t& vo) __attribute__((always_inline)) {
-    if constexpr (kPaged) {
-      const int page = a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size;
-      int block;
-      if constexpr (kPageMode == kPagedLds) {
-        block = page_table[page - page0];
-      } else {
-        block = min(max(table_row[page], 0), a.num_blocks - 1);
-      }
-      const int row = key - page * a.page_size;
-      ko = static_cast<int64_t>(block) * a.k_bs + static_cast<int64_t>(row) * a.k_ss;
-      vo = static_cast<int64_t>(block) * a.v_bs + static_cast<int64_t>(row) * a.v_ss;
+    int b, hq, k_begin, k_end, head_step;
+    int64_t partial;  // index of the segment's first partial; the next head's is head_step on
+    if constexpr (kBalanced) {
+      const decode::Segment g = decode::segment_at(a, sched, blockIdx.x, pos, end, tid == 0);
+      pos = g.next;
+      if (g.k_begin == g.k_end) continue;
+      b = g.b;
+      hq = g.head;
+      k_begin = g.k_begin;
+      k_end = g.k_end;
+      partial = g.slot * (span * group);
+      head_step = 1;
     } else {
-      ko = static_cast<int64_t>(key) * a.k_ss;
-      vo = static_cast<int64_t>(key) * a.v_ss;
+      pos = end;
+      const int split = blockIdx.x % a.num_splits;
+      const int work = blockIdx.x / a.num_splits;
+      b = work / rows;
+      hq = work - b * rows;
+      // Lengths are not checked on the host (that would need a sync); clamp them to the cache so an
+      // out-of-range value cannot read outside it.
+      const int len = min(max(a.seq_lens[b], 0), a.max_seqlen);
+      const int per_split =
+          ((len + a.num_splits - 1) / a.num_splits + kTileKeys - 1) / kTileKeys * kTileKeys;
+      k_begin = split * per_split;
+      k_end = min(len, k_begin + per_split);
+      partial = (static_cast<int64_t>(b) * a.heads + hq * span * group) * a.num_splits + split;
+      head_step = a.num_splits;
     }
-  };
-  char* wave_lds = reinterpret_cast<char*>(smem) + wave * kWaveBytes<D>;
-  auto tile_start = [&](int i) __attribute__((always_inline)) {
-    return k_begin + (span == 1 ? wave + kWaves * i : i) * kTileKeys;
-  };
-  using Regs = u32x4[2 * kLoads<D>];  // K loads, then V loads
-  auto load_tile = [&](int i, Regs& r) __attribute__((always_inline)) {
-    const int t0 = tile_start(i);
-#pragma unroll
-    for (int j = 0; j < kLoads<D>; ++j) {
-      const int key = min(t0 + kRowsPerLoad * j + lane_row, k_end - 1);
-      int64_t ko, vo;
-      row_offsets(key, ko, vo);
-      r[j] = load16_stream(kbase + ko);
-      r[kLoads<D> + j] = load16_stream(vbase + vo);
-    }
-  };
-  auto store_tile = [&](const Regs& r) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < kLoads<D>; ++j) {
-      const int off = 2 * prefill::tile_offset<D>(kRowsPerLoad * j + lane_row, lane_col);
-      *reinterpret_cast<u32x4*>(wave_lds + off) = r[j];
-      *reinterpret_cast<u32x4*>(wave_lds + kTileBytes<D> + off) = r[kLoads<D> + j];
-    }
-  };
+    const int hkv = span == 1 ? hq : hq * span + wave;
+    const int h0 = hkv * group;
+    const int tiles = k_begin < k_end ? (k_end - k_begin + kTileKeys - 1) / kTileKeys : 0;
+    const int my_tiles = span == 1 ? (tiles > wave ? (tiles - wave + kWaves - 1) / kWaves : 0) : tiles;
 
-  f32x16 o[D / 32];
+    // Q^T, the B operand: lane (col, half) holds q[h0 + col][16 ks + 8 half .. + 7], zero past the
+    // group.
+    u32x4 qf[D / 16];
+    {
+      const bool ok = col < group;
+      const uint16_t* qrow =
+          static_cast<const uint16_t*>(a.q) + b * a.q_bs + (h0 + (ok ? col : 0)) * a.q_hs + 8 * half;
 #pragma unroll
-  for (int nb = 0; nb < D / 32; ++nb) o[nb] = f32x16{};
-  // Reference point of o and l for the lane's head (log2 units, the same in both halves of a
-  // column; kNoRef until the first tile): the running max of its scores, as in the reference's
-  // online softmax. Probabilities are 2^(s scale_log2 - ref) <= 1, and the largest key seen so far
-  // has p = 1 exactly, which the rounding of P to the input type keeps exact.
-  float ref = kNoRef;
-  float l = 0.f;  // the lane's part of the running sum (its 16 keys of each tile)
-  const float sl2 = a.scale_log2;
-
-  // Tile i from register set r: into LDS, fragments back, the set refilled with tile i + kAhead,
-  // then S^T, the softmax and O^T. LDS operations of a wave complete in order, so the fragment
-  // reads see the stores before them and the next tile's stores come after these reads.
-  auto step = [&](int i, Regs& r) __attribute__((always_inline)) {
-    store_tile(r);
-    const uint16_t* kt = reinterpret_cast<const uint16_t*>(wave_lds);
-    const uint16_t* vt = reinterpret_cast<const uint16_t*>(wave_lds + kTileBytes<D>);
-    u32x4 kf[D / 16];
-    u32x4 vf[2][D / 32];
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) kf[ks] = k_frag<D>(kt, 0, ks, lane);
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb) vf[kk][nb] = v_frag<D>(vt, nb, kk, lane);
+      for (int ks = 0; ks < D / 16; ++ks) qf[ks] = ok ? load16(qrow + 16 * ks) : u32x4{0, 0, 0, 0};
     }
-    // Unconditional (past the split the keys clamp to its last row): a load skipped on some path
-    // leaves the compiler unsure how many are in flight, and it then waits for all of them.
-    load_tile(i + kAhead, r);
-    __builtin_amdgcn_sched_barrier(0);
 
-    f32x16 s = f32x16{};
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) s = E::mfma32(kf[ks], qf[ks], s);
-    const int t0 = tile_start(i);
-    if (t0 + kTileKeys > k_end) {  // the split's last, partial tile (wave-uniform)
-      const int lim = k_end - 1 - t0 - 4 * half;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        if (acc_key(j, 0) > lim) s[j] = -INFINITY;
+    // Paged cache: the split's block numbers, clamped to the pool (kPagedLds), or the table row.
+    __shared__ int page_table[kPageMode == kPagedLds ? kMaxSplitPages : 1];
+    int page0 = 0;
+    const int32_t* table_row = nullptr;
+    if constexpr (kPaged) table_row = a.block_tables + static_cast<int64_t>(b) * a.block_tables_stride;
+    if constexpr (kPageMode == kPagedLds) {
+      if (k_begin < k_end) {
+        page0 = k_begin / a.page_size;
+        const int pages = (k_end - 1) / a.page_size - page0 + 1;
+        for (int i = tid; i < pages; i += kThreads)
+          page_table[i] = min(max(table_row[page0 + i], 0), a.num_blocks - 1);
       }
+      __syncthreads();
     }
-    // The running max moves (and O and l are rescaled, a wave-uniform branch) only on tiles where
-    // some head's max grows, so O, which the compiler keeps in accumulator registers, is left
-    // alone on most tiles of a long sequence.
-    float mx = s[0];
-#pragma unroll
-    for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
-    // scale_log2 > 0, so the max commutes with it; every column sees a valid key of the tile.
-    mx = max_halves(mx) * sl2;
-    if (wave_any(mx > ref)) {
-      const float moved = fmaxf(ref, mx);
-      const float alpha = exp2_fast(ref - moved);  // 0 on the first tile
-      ref = moved;
-#pragma unroll
-      for (int nb = 0; nb < D / 32; ++nb) o[nb] *= alpha;
-      l *= alpha;
-    }
-    f32x16 p;
-    float rs = 0.f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      p[j] = exp2_fast(fmaf(s[j], sl2, -ref));
-      rs += p[j];
-    }
-    l += rs;
-    const u32x4 p0 = p_frag<Tag, 0>(p);
-    const u32x4 p1 = p_frag<Tag, 1>(p);
-#pragma unroll
-    for (int nb = 0; nb < D / 32; ++nb) {
-      o[nb] = E::mfma32(vf[0][nb], p0, o[nb]);
-      o[nb] = E::mfma32(vf[1][nb], p1, o[nb]);
-    }
-  };
 
-  // Guarded as a whole so the first loads are unconditional too (a split with no tile for this
-  // wave has no valid row to clamp to).
-  if (my_tiles > 0) {
-    Regs r[kAhead];
-    static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
-      load_tile(decltype(t)::value, r[decltype(t)::value]);
-    });
-    int i = 0;
-    for (; i + kAhead <= my_tiles; i += kAhead) {
-      static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
-        step(i + decltype(t)::value, r[decltype(t)::value]);
-      });
-    }
-    static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
-      if (i + decltype(t)::value < my_tiles) step(i + decltype(t)::value, r[decltype(t)::value]);
-    });
-  }
+    // Tile loads: load j of a tensor tile gives lane l row kRowsPerLoad j + l / kChunksPerRow, chunk
+    // l % kChunksPerRow (whole rows per instruction), which it stores at that row's swizzled chunk.
+    const int lane_row = lane / kChunksPerRow;
+    const int lane_col = 8 * (lane % kChunksPerRow);
+    const uint16_t* kbase =
+        static_cast<const uint16_t*>(a.k) + (kPaged ? 0 : b * a.k_bs) + hkv * a.k_hs + lane_col;
+    const uint16_t* vbase =
+        static_cast<const uint16_t*>(a.v) + (kPaged ? 0 : b * a.v_bs) + hkv * a.v_hs + lane_col;
+    // Offsets (elements) of a key's K and V rows from kbase / vbase.
+    auto row_offsets = [&](int key, int64_t& ko, int64_t& vo) __attribute__((always_inline)) {
+      if constexpr (kPaged) {
+        const int page = a.page_shift >= 0 ? key >> a.page_shift : key / a.page_size;
+        int block;
+        if constexpr (kPageMode == kPagedLds) {
+          block = page_table[page - page0];
+        } else {
+          block = min(max(table_row[page], 0), a.num_blocks - 1);
+        }
+        const int row = key - page * a.page_size;
+        ko = static_cast<int64_t>(block) * a.k_bs + static_cast<int64_t>(row) * a.k_ss;
+        vo = static_cast<int64_t>(block) * a.v_bs + static_cast<int64_t>(row) * a.v_ss;
+      } else {
+        ko = static_cast<int64_t>(key) * a.k_ss;
+        vo = static_cast<int64_t>(key) * a.v_ss;
+      }
+    };
+    char* wave_lds = reinterpret_cast<char*>(smem) + wave * kWaveBytes<D>;
+    auto tile_start = [&](int i) __attribute__((always_inline)) {
+      return k_begin + (span == 1 ? wave + kWaves * i : i) * kTileKeys;
+    };
+    using Regs = u32x4[2 * kLoads<D>];  // K loads, then V loads
+    auto load_tile = [&](int i, Regs& r) __attribute__((always_inline)) {
+      const int t0 = tile_start(i);
+#pragma unroll
+      for (int j = 0; j < kLoads<D>; ++j) {
+        const int key = min(t0 + kRowsPerLoad * j + lane_row, k_end - 1);
+        int64_t ko, vo;
+        row_offsets(key, ko, vo);
+        r[j] = load16_stream(kbase + ko);
+        r[kLoads<D> + j] = load16_stream(vbase + vo);
+      }
+    };
+    auto store_tile = [&](const Regs& r) __attribute__((always_inline)) {
+#pragma unroll
+      for (int j = 0; j < kLoads<D>; ++j) {
+        const int off = 2 * prefill::tile_offset<D>(kRowsPerLoad * j + lane_row, lane_col);
+        *reinterpret_cast<u32x4*>(wave_lds + off) = r[j];
+        *reinterpret_cast<u32x4*>(wave_lds + kTileBytes<D> + off) = r[kLoads<D> + j];
+      }
+    };
 
-  // Merge the four waves in order; the tile buffers are free after the barrier.
-  __syncthreads();
-  float* red_m = reinterpret_cast<float*>(smem);  // [kWaves][kCols]
-  float* red_l = red_m + kWaves * kCols;          // [kWaves][kCols]
-  float* red_o = red_l + kWaves * kCols;          // [kWaves][kCols][kRedPitch]
-  const float lt = sum_halves(l);
-  if (half == 0) {
-    // A wave that saw no key (l = 0, ref still kNoRef) records -inf, as the merges expect.
-    red_m[wave * kCols + col] = lt > 0.f ? ref : -INFINITY;
-    red_l[wave * kCols + col] = lt;
-  }
-  if (col < group) {
-    float* row = red_o + (wave * kCols + col) * kRedPitch<D>;
+    f32x16 o[D / 32];
 #pragma unroll
-    for (int nb = 0; nb < D / 32; ++nb) {
+    for (int nb = 0; nb < D / 32; ++nb) o[nb] = f32x16{};
+    // Reference point of o and l for the lane's head (log2 units, the same in both halves of a
+    // column; kNoRef until the first tile): the running max of its scores, as in the reference's
+    // online softmax. Probabilities are 2^(s scale_log2 - ref) <= 1, and the largest key seen so far
+    // has p = 1 exactly, which the rounding of P to the input type keeps exact.
+    float ref = kNoRef;
+    float l = 0.f;  // the lane's part of the running sum (its 16 keys of each tile)
+    const float sl2 = a.scale_log2;
+
+    // Tile i from register set r: into LDS, fragments back, the set refilled with tile i + kAhead,
+    // then S^T, the softmax and O^T. LDS operations of a wave complete in order, so the fragment
+    // reads see the stores before them and the next tile's stores come after these reads.
+    auto step = [&](int i, Regs& r) __attribute__((always_inline)) {
+      store_tile(r);
+      const uint16_t* kt = reinterpret_cast<const uint16_t*>(wave_lds);
+      const uint16_t* vt = reinterpret_cast<const uint16_t*>(wave_lds + kTileBytes<D>);
+      u32x4 kf[D / 16];
+      u32x4 vf[2][D / 32];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) row[32 * nb + acc_key(j, half)] = o[nb][j];
-    }
-  }
-  __syncthreads();
-  // Span 1: the four waves' states of one KV head are merged in wave order. Span 4: each wave's
-  // state is its own KV head's and is written as it is.
-  const int outs = span == 1 ? group * D : kWaves * group * D;
-  for (int idx = tid; idx < outs; idx += kThreads) {
-    const int wv0 = span == 1 ? 0 : idx / (group * D);
-    const int r = idx - wv0 * group * D;
-    const int g = r / D;
-    const int d = r - g * D;
-    float mm = -INFINITY;
-    float num = 0.f;
-    float den = 0.f;
-    if (span == 1) {
+      for (int ks = 0; ks < D / 16; ++ks) kf[ks] = k_frag<D>(kt, 0, ks, lane);
 #pragma unroll
-      for (int wv = 0; wv < kWaves; ++wv) mm = fmaxf(mm, red_m[wv * kCols + g]);
+      for (int kk = 0; kk < 2; ++kk) {
 #pragma unroll
-      for (int wv = 0; wv < kWaves; ++wv) {
-        const float mw = red_m[wv * kCols + g];
-        if (mw != -INFINITY) {
-          const float f = exp2_fast(mw - mm);
-          num += red_o[(wv * kCols + g) * kRedPitch<D> + d] * f;
-          den += red_l[wv * kCols + g] * f;
+        for (int nb = 0; nb < D / 32; ++nb) vf[kk][nb] = v_frag<D>(vt, nb, kk, lane);
+      }
+      // Unconditional (past the split the keys clamp to its last row): a load skipped on some path
+      // leaves the compiler unsure how many are in flight, and it then waits for all of them.
+      load_tile(i + kAhead, r);
+      __builtin_amdgcn_sched_barrier(0);
+
+      f32x16 s = f32x16{};
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) s = E::mfma32(kf[ks], qf[ks], s);
+      const int t0 = tile_start(i);
+      if (t0 + kTileKeys > k_end) {  // the split's last, partial tile (wave-uniform)
+        const int lim = k_end - 1 - t0 - 4 * half;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          if (acc_key(j, 0) > lim) s[j] = -INFINITY;
         }
       }
-    } else {
-      mm = red_m[wv0 * kCols + g];
-      if (mm != -INFINITY) {
-        num = red_o[(wv0 * kCols + g) * kRedPitch<D> + d];
-        den = red_l[wv0 * kCols + g];
+      // The running max moves (and O and l are rescaled, a wave-uniform branch) only on tiles where
+      // some head's max grows, so O, which the compiler keeps in accumulator registers, is left
+      // alone on most tiles of a long sequence.
+      float mx = s[0];
+#pragma unroll
+      for (int j = 1; j < 16; ++j) mx = fmaxf(mx, s[j]);
+      // scale_log2 > 0, so the max commutes with it; every column sees a valid key of the tile.
+      mx = max_halves(mx) * sl2;
+      if (wave_any(mx > ref)) {
+        const float moved = fmaxf(ref, mx);
+        const float alpha = exp2_fast(ref - moved);  // 0 on the first tile
+        ref = moved;
+#pragma unroll
+        for (int nb = 0; nb < D / 32; ++nb) o[nb] *= alpha;
+        l *= alpha;
+      }
+      f32x16 p;
+      float rs = 0.f;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        p[j] = exp2_fast(fmaf(s[j], sl2, -ref));
+        rs += p[j];
+      }
+      l += rs;
+      const u32x4 p0 = p_frag<Tag, 0>(p);
+      const u32x4 p1 = p_frag<Tag, 1>(p);
+#pragma unroll
+      for (int nb = 0; nb < D / 32; ++nb) {
+        o[nb] = E::mfma32(vf[0][nb], p0, o[nb]);
+        o[nb] = E::mfma32(vf[1][nb], p1, o[nb]);
+      }
+    };
+
+    // Guarded as a whole so the first loads are unconditional too (a split with no tile for this
+    // wave has no valid row to clamp to).
+    if (my_tiles > 0) {
+      Regs r[kAhead];
+      static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
+        load_tile(decltype(t)::value, r[decltype(t)::value]);
+      });
+      int i = 0;
+      for (; i + kAhead <= my_tiles; i += kAhead) {
+        static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
+          step(i + decltype(t)::value, r[decltype(t)::value]);
+        });
+      }
+      static_for<0, kAhead>([&](auto t) __attribute__((always_inline)) {
+        if (i + decltype(t)::value < my_tiles) step(i + decltype(t)::value, r[decltype(t)::value]);
+      });
+    }
+
+    // Merge the four waves in order; the tile buffers are free after the barrier.
+    __syncthreads();
+    float* red_m = reinterpret_cast<float*>(smem);  // [kWaves][kCols]
+    float* red_l = red_m + kWaves * kCols;          // [kWaves][kCols]
+    float* red_o = red_l + kWaves * kCols;          // [kWaves][kCols][kRedPitch]
+    const float lt = sum_halves(l);
+    if (half == 0) {
+      // A wave that saw no key (l = 0, ref still kNoRef) records -inf, as the merges expect.
+      red_m[wave * kCols + col] = lt > 0.f ? ref : -INFINITY;
+      red_l[wave * kCols + col] = lt;
+    }
+    if (col < group) {
+      float* row = red_o + (wave * kCols + col) * kRedPitch<D>;
+#pragma unroll
+      for (int nb = 0; nb < D / 32; ++nb) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) row[32 * nb + acc_key(j, half)] = o[nb][j];
       }
     }
-    const int h = (span == 1 ? h0 : (hq * span + wv0) * group) + g;
-    if (a.num_splits == 1) {
-      uint16_t* orow = static_cast<uint16_t*>(a.o) + b * a.o_bs + h * a.o_hs;
-      orow[d] = E::from_float(den > 0.f ? num / den : 0.f);
-      if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
-    } else {
-      const int64_t slot = partial + static_cast<int64_t>(wv0 * group + g) * head_step;
-      a.partial_o[slot * D + d] = num;
-      if (d == 0) {
-        a.partial_ml[2 * slot] = mm;
-        a.partial_ml[2 * slot + 1] = den;
+    __syncthreads();
+    // Span 1: the four waves' states of one KV head are merged in wave order. Span 4: each wave's
+    // state is its own KV head's and is written as it is.
+    const int outs = span == 1 ? group * D : kWaves * group * D;
+    for (int idx = tid; idx < outs; idx += kThreads) {
+      const int wv0 = span == 1 ? 0 : idx / (group * D);
+      const int r = idx - wv0 * group * D;
+      const int g = r / D;
+      const int d = r - g * D;
+      float mm = -INFINITY;
+      float num = 0.f;
+      float den = 0.f;
+      if (span == 1) {
+#pragma unroll
+        for (int wv = 0; wv < kWaves; ++wv) mm = fmaxf(mm, red_m[wv * kCols + g]);
+#pragma unroll
+        for (int wv = 0; wv < kWaves; ++wv) {
+          const float mw = red_m[wv * kCols + g];
+          if (mw != -INFINITY) {
+            const float f = exp2_fast(mw - mm);
+            num += red_o[(wv * kCols + g) * kRedPitch<D> + d] * f;
+            den += red_l[wv * kCols + g] * f;
+          }
+        }
+      } else {
+        mm = red_m[wv0 * kCols + g];
+        if (mm != -INFINITY) {
+          num = red_o[(wv0 * kCols + g) * kRedPitch<D> + d];
+          den = red_l[wv0 * kCols + g];
+        }
+      }
+      const int h = (span == 1 ? h0 : (hq * span + wv0) * group) + g;
+      if (a.num_splits == 1) {
+        uint16_t* orow = static_cast<uint16_t*>(a.o) + b * a.o_bs + h * a.o_hs;
+        orow[d] = E::from_float(den > 0.f ? num / den : 0.f);
+        if (d == 0) a.lse[b * a.heads + h] = den > 0.f ? mm * kLn2 + logf(den) : -INFINITY;
+      } else {
+        const int64_t slot = partial + static_cast<int64_t>(wv0 * group + g) * head_step;
+        a.partial_o[slot * D + d] = num;
+        if (d == 0) {
+          a.partial_ml[2 * slot] = mm;
+          a.partial_ml[2 * slot + 1] = den;
+        }
       }
     }
-  }
-  if constexpr (!kBalanced) return;
-  if (pos < end) __syncthreads();  // the next segment reuses the LDS
+    if constexpr (!kBalanced) return;
+    if (pos < end) __syncthreads();  // the next segment reuses the LDS
   }
 }
 

@@ -444,7 +444,9 @@ static_assert(kPrefillBlockN == prefill::kBlockN, "host and kernel tile widths d
 // more than a quarter padding (at head_dim 64, S = 512 pads 256 of 768 rows) and that needs more
 // than one round of workgroups, where the padded blocks take a round's time for a third of its
 // rows: H=32, D = 64, S = 512, B=16 523 / 618, B=32 537 / 654; one round (B=4) 276 / 230; 11%
-// padding (S = 2048, B=8, H=16) 931 / 819. The FL_KNOB_PREFILL_PP_MIN_WG knob replaces all of
+// padding (S = 2048, B=8, H=16) 931 / 819. (Those figures are
+// without packed heads and half tiles; with them, us, causal, H=32, H_kv=8, D = 128: B=1 S=1024 33 / 21,
+// B=4 S=512 20 / 24, B=8 S=512 29 / 38, B=4 S=2048 139 / 162.) The FL_KNOB_PREFILL_PP_MIN_WG knob replaces all of
 // this with its own workgroup threshold (so tests can route one shape to either kernel).
 bool prefill_on_pingpong(const PrefillArgs& args, int head_dim) {
   const int rows = prefill_pp_block_rows(head_dim);
