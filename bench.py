@@ -534,8 +534,8 @@ def bench_decode(name: str, steps: int, warmup: int, flush, cpu: bool) -> dict:
     # from HBM.
     gpu = gpu_window(run, stats["median"])
     kv = decode_kv_bytes(b, hkv, ctx, d, 2)
-    splits, _ = _hip.decode_plan(b, h, hkv, d, ctx, torch.bfloat16,
-                                 cu_count_=_hip.cu_count(torch.cuda.current_device()))
+    splits, workgroups, _ = _hip.decode_schedule(b, h, hkv, d, ctx, torch.bfloat16, page_size or 0,
+                                                 cu_count_=_hip.cu_count(torch.cuda.current_device()))
     del q, k_used, v_used, tables
     torch.cuda.empty_cache()
     result = {
@@ -543,7 +543,8 @@ def bench_decode(name: str, steps: int, warmup: int, flush, cpu: bool) -> dict:
         "page_size": page_size,
         "kv_bytes": kv,
         "bytes_with_q_o": decode_bytes_with_qo(b, h, hkv, ctx, d, 2),
-        "num_splits": splits,
+        "num_splits": splits,  # 0: balanced over `workgroups`
+        "workgroups": workgroups,
         "ms": stats,
         "mean_ms": mean_ms,
         "gbps": kv / (stats["median"] / 1e3) / 1e9,

@@ -456,10 +456,11 @@ bool prefill_on_pingpong(const PrefillArgs& args, int head_dim) {
   const int v = knob(FL_KNOB_PREFILL_PP_MIN_WG);
   if (v >= 0) return workgroups >= v;
   if (args.causal) return workgroups >= 128;
-  // One head's padding, as it was measured; with packed heads both kernels take the same time there.
+  // One head's padding and workgroups, as they were measured; with packed heads both kernels take the
+  // same time there.
   const int64_t head_blocks = (args.seqlen_q + rows - 1) / rows;
   const int64_t padding = head_blocks * rows - args.seqlen_q;
-  if (4 * padding > head_blocks * rows && workgroups > 256) return false;
+  if (4 * padding > head_blocks * rows && head_blocks * args.batch * args.heads > 256) return false;
   return workgroups >= 256;
 }
 

@@ -354,6 +354,21 @@ def decode_noalloc(q, k_cache, v_cache, seq_lens, o, lse, softmax_scale: float, 
     return splits.value
 
 
+def decode_schedule(batch, heads, heads_kv, head_dim, max_seqlen, dtype, page_size=0,
+                    cu_count_=256) -> tuple[int, int, int]:
+    """(num_splits, workgroups, workspace bytes) of a decode call that asks for no split count:
+    workgroups > 0 (and num_splits 0) for a balanced one. Host-only."""
+    p = DecodeParams()
+    p.batch, p.heads, p.heads_kv, p.head_dim, p.max_seqlen = batch, heads, heads_kv, head_dim, max_seqlen
+    p.dtype = DTYPE_CODES[dtype]
+    if page_size:  # only whether the cache is paged, and its page size, count here
+        p.block_tables, p.page_size, p.num_blocks = 16, page_size, 1
+    splits, wgs, ws = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
+    _check(LIB.fl_decode_schedule(ctypes.byref(p), cu_count_, ctypes.byref(splits), ctypes.byref(wgs),
+                                  ctypes.byref(ws)))
+    return splits.value, wgs.value, ws.value
+
+
 def decode_plan(batch, heads, heads_kv, head_dim, max_seqlen, dtype, num_splits=0,
                 allow_splits=True, cu_count_=256) -> tuple[int, int]:
     """(num_splits, workspace bytes) the library picks for a decode shape; host-only."""

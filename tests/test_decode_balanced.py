@@ -99,16 +99,11 @@ def test_floor_by_reciprocal():
             assert torch.equal(q.long(), n // c), c
 
 
+DTYPES = {0: torch.bfloat16, 2: torch.float32}
+
+
 def plan(batch, heads, heads_kv, head_dim, max_seqlen, dtype=0, page_size=0):
-    p = _hip.DecodeParams()
-    p.batch, p.heads, p.heads_kv, p.head_dim, p.max_seqlen, p.dtype = (
-        batch, heads, heads_kv, head_dim, max_seqlen, dtype)
-    if page_size:
-        p.block_tables, p.page_size, p.num_blocks = 256, page_size, 1 << 20
-    splits, wgs, ws = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_size_t()
-    assert _hip.LIB.fl_decode_schedule(ctypes.byref(p), 256, ctypes.byref(splits), ctypes.byref(wgs),
-                                       ctypes.byref(ws)) == 0
-    return splits.value, wgs.value, ws.value
+    return _hip.decode_schedule(batch, heads, heads_kv, head_dim, max_seqlen, DTYPES[dtype], page_size)
 
 
 def test_plan():
