@@ -28,6 +28,8 @@
 //    workgroup then has to wait for its partials to reach device scope and for an atomic before it
 //    frees its slot, which costs more than the second launch.)
 
+#include <type_traits>
+
 #include "decode_sched.hpp"
 #include "gfx950.hpp"
 #include "launch.hpp"
@@ -535,25 +537,28 @@ decode_split_kernel(const DecodeArgs a) {
   }
 }
 
-// Merge pass: one workgroup per head group (kHeads query heads of one KV head).
+// Merge pass: one workgroup per kHeads query heads of one KV head (all of the query heads of the split
+// kernel's work head, or some of them).
 template <typename Tag, int D, int kHeads, bool kBalanced>
 __global__ void __launch_bounds__(kThreads) decode_merge_kernel(const DecodeArgs a) {
   __shared__ __attribute__((aligned(16))) float lds[MergeShape<kHeads, D>::kFloats];
+  const int merges = a.group / kHeads;  // per KV head
   int w = blockIdx.x;
-  const int hchunk = w % a.head_chunks;
-  w /= a.head_chunks;
+  const int first_head = w % merges * kHeads;  // of the KV head's group
+  w /= merges;
   const int hkv = w % a.heads_kv;
   const int b = w / a.heads_kv;
-  const int h0 = hkv * a.group + hchunk * kHeads;
+  const int h0 = hkv * a.group + first_head;
   if constexpr (kBalanced) {
-    // The split kernel's work head: a span of KV heads with this chunk of each one's query heads
-    // (vector kernel) or with all of them (matrix-core kernel).
+    // The split kernel's work head: a span of KV heads with one chunk of each one's query heads (vector
+    // kernel) or with all of them (matrix-core kernel).
     const int span = a.mfma ? a.mfma_span : a.kv_span;
     const int chunks = a.mfma ? 1 : a.head_chunks;
-    const int wg_heads = a.mfma ? span * a.group : span * kHeads;
+    const int chunk_heads = a.group / chunks;
+    const int wg_heads = span * chunk_heads;
     const int rows = a.heads_kv / span * chunks;
-    const int row = b * rows + hkv / span * chunks + (a.mfma ? 0 : hchunk);
-    const int head = hkv % span * (wg_heads / span) + (a.mfma ? hchunk * kHeads : 0);
+    const int row = b * rows + hkv / span * chunks + first_head / chunk_heads;
+    const int head = hkv % span * chunk_heads + first_head % chunk_heads;
     Partials at{row * int64_t{kRowSlots} * wg_heads + head, 0, 1, wg_heads};
     merge_splits<Tag, D, kHeads, true>(a, b, h0, at, [&] {
       const int2 slots = a.row_slots[row];
@@ -621,10 +626,13 @@ hipError_t launch_heads(const DecodeArgs& args, DType dtype, hipStream_t stream)
     }
   }
   if (err != hipSuccess || args.num_splits == 1) return err;
+  // The merge deals its threads over vectors of whole heads, a power of two of them.
+  constexpr int kMergeHeads = kHeads == 3 ? 1 : kHeads;
+  const dim3 merges(args.batch * (args.heads / kMergeHeads));
   if (args.balanced_wgs) {
-    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kHeads, true>), dim3(groups), dim3(kThreads), 0, stream, args);
+    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kMergeHeads, true>), merges, dim3(kThreads), 0, stream, args);
   } else {
-    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kHeads, false>), dim3(groups), dim3(kThreads), 0, stream, args);
+    hipLaunchKernelGGL((decode_merge_kernel<Tag, D, kMergeHeads, false>), merges, dim3(kThreads), 0, stream, args);
   }
   return hipGetLastError();
 }
@@ -634,6 +642,9 @@ hipError_t launch_dim(const DecodeArgs& args, DType dtype, int k_heads, hipStrea
   switch (k_heads) {
     case 1: return launch_heads<Tag, D, 1>(args, dtype, stream);
     case 2: return launch_heads<Tag, D, 2>(args, dtype, stream);
+    case 3:  // (decode_layout plans it for 16-bit caches only)
+      if constexpr (std::is_same_v<Tag, f32_tag>) return hipErrorInvalidValue;
+      else return launch_heads<Tag, D, 3>(args, dtype, stream);
     case 4: return launch_heads<Tag, D, 4>(args, dtype, stream);
     default: return launch_heads<Tag, D, 8>(args, dtype, stream);
   }
@@ -655,21 +666,28 @@ hipError_t launch_type(const DecodeArgs& args, DType dtype, int head_dim, int k_
 // D = 64, B=8 86.4 vs 93.8, B=4 50.7 vs 56.2, B=1 23.4 vs 24.4, one 8.4K-key sequence 14.9 vs
 // 18.0. With 2 it is mixed (D = 128: B=2 54.3 vs 49.3, B=4 89.3 vs 90.6; D = 64: B=2 33.7 vs
 // 30.4, B=8 85.7 vs 89.5), so groups of 2 stay on the vector kernel.
-// A group of 3 has no vector form of its own (one query head per workgroup, three passes over the
-// cache), so it goes to the matrix cores too, from 16K cache rows: (10, 24, 8, 15868) 277 vs 102 us, (4,
-// 24, 8, 2000) 23 vs 14, (1, 24, 8, 2600) 10.2 for both, (1, 24, 8, 640) 7.7 on the vector kernel, 9.3.
-int decode_mfma_min_group(int64_t cache_rows) {
+int decode_mfma_min_group() {
   const int v = knob(FL_KNOB_DECODE_MFMA_MIN_GROUP);
-  if (v >= 1) return v;
-  return cache_rows >= 16384 ? 3 : 4;
+  return v >= 1 ? v : 4;
 }
+
+// Fewest cache rows for which the vector kernel serves a group of 3 with all three heads per workgroup
+// (in 16-bit types), each row read once, instead of one head per workgroup, three passes over the cache.
+// The matrix-core kernel is no faster there and rounds the probabilities to the input type, which this
+// kernel keeps in fp32. us a call, one head / three / matrix cores, bf16 or fp16: (10, 24, 8, 15868) 273 /
+// 119 / 118, paged with spread lengths 165 / 68 / 69, (1, 24, 8, 8192) 32.7 / 16.8 / 16.8, (16, 24, 8,
+// 4000, D = 64) spread 48.8 / 26.5 / 24.2; smaller (device us, one / three): (1, 24, 8, 640) 8.6 / 10.2,
+// (4, 24, 8, 300) 9.2 / 10.2, (2, 24, 8, 1000, D = 64) 10.0 / 10.5. Two rows in flight per buffer, four:
+// 119 / 130, paged 68 / 84.
+constexpr int64_t kThreeHeadRows = 16384;
 
 DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows) {
   DecodeLayout layout{};
   int k = 1;
   while (k < 8 && group % (2 * k) == 0) k *= 2;
+  if (group == 3 && dtype != DType::f32 && cache_rows >= kThreeHeadRows) k = 3;
   layout.heads_per_wg = k;
-  if (dtype != DType::f32 && group >= decode_mfma_min_group(cache_rows) &&
+  if (dtype != DType::f32 && group >= decode_mfma_min_group() &&
       group <= kMaxDecodeMfmaHeads) {
     // One KV head per workgroup. Two fit a CU (256 registers per lane, 64 KiB of LDS at D = 128),
     // but one per CU streamed faster (B=8, 8 KV heads, 32K keys: 6.03-6.09 TB/s against

@@ -142,10 +142,10 @@ hipError_t launch_prefill_causal_stream(const PrefillArgs& args, DType dtype, in
                                         hipStream_t stream);
 
 // How decode work is laid out. The vector kernel (decode.hip): each workgroup serves heads_per_wg
-// query heads (a power of two dividing the GQA group) of each of kv_span adjacent KV heads. The
-// matrix-core kernel (mfma = 1): one KV head and its whole group per workgroup (kv_span 1,
-// wg_heads = group). heads_per_wg is also the merge pass's chunk of heads either way. A CU holds
-// resident_per_cu split workgroups at once (registers or LDS).
+// query heads (a power of two dividing the GQA group, or a group of 3) of each of kv_span adjacent KV
+// heads. The matrix-core kernel (mfma = 1): one KV head and its whole group per workgroup (kv_span 1,
+// wg_heads = group). heads_per_wg is also the merge pass's chunk of heads either way (one head for 3). A
+// CU holds resident_per_cu split workgroups at once (registers or LDS).
 struct DecodeLayout {
   int heads_per_wg;
   int kv_span;

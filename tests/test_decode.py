@@ -480,3 +480,59 @@ def test_inplace_large_batch_takes_four_kv_heads_per_workgroup():
     out, lse = flash_lab.decode(q, k_cache, v_cache, seq_lens, impl="decode_inplace",
                                 return_lse=True)
     check_decode(out, lse, q, k_cache, v_cache, seq_lens)
+
+
+def check_three_head_rounding(out, q, k_cache, v_cache, seq_lens):
+    """Every output is the exact value rounded once to the input type, plus fp32 error: q and k are small
+    integers, so the dot products are exact; at most seven keys, v in [1, 2), so nothing cancels and the
+    fp32 steps (scale, exp2, sums, division: a few 2^-24 each of values up to 32) stay below 2^-17. With
+    probabilities rounded to the input type the error before the last rounding is up to 2^-9 (bf16)."""
+    half_ulp = 2.0**-8 if out.dtype == torch.bfloat16 else 2.0**-11
+    for b, n in enumerate(seq_lens.tolist()):
+        k, v = (x[b, :n].cpu().double().repeat_interleave(3, dim=1) for x in (k_cache, v_cache))
+        scores = torch.einsum("hd,nhd->hn", q[b, 0].cpu().double(), k) / q.shape[-1] ** 0.5
+        want = torch.einsum("hn,nhd->hd", torch.softmax(scores, dim=-1), v)
+        err = (out[b, 0].cpu().double() - want).abs().max().item()
+        assert err <= half_ulp + 2.0**-17, f"sequence {b}: error {err:.3g}, half an ulp is {half_ulp:.3g}"
+
+
+# Groups of 3 have 32-bit probabilities at every cache size: below kThreeHeadRows cache rows one head per
+# workgroup, from there on three (csrc/decode.hip).
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("dtype", DTYPES[:2], ids=lambda d: str(d).removeprefix("torch."))
+@pytest.mark.parametrize("capacity", [1023, 1024])
+def test_group_of_three_keeps_fp32_probabilities(capacity, dtype, head_dim):
+    print(f"decode group of 3 {capacity} {dtype} {head_dim}", flush=True)
+    batch, heads, heads_kv = 2, 24, 8
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    q = torch.randint(-2, 3, (batch, 1, heads, head_dim), device="cuda", generator=gen).to(dtype)
+    k = torch.randint(-1, 2, (batch, capacity, heads_kv, head_dim), device="cuda", generator=gen).to(dtype)
+    v = (1 + torch.rand(batch, capacity, heads_kv, head_dim, device="cuda", generator=gen) * 0.99).to(dtype)
+    seq_lens = torch.tensor([7, 3], device="cuda", dtype=torch.int32)
+    for kwargs in (dict(), dict(num_splits=4), dict(impl="decode_inplace")):
+        check_three_head_rounding(flash_lab.decode(q, k, v, seq_lens, **kwargs), q, k, v, seq_lens)
+    if capacity % 16 == 0:
+        tables = torch.arange(batch * capacity // 16, device="cuda", dtype=torch.int32).view(batch, -1)
+        pools = (x.reshape(-1, 16, heads_kv, head_dim) for x in (k, v))
+        check_three_head_rounding(flash_lab.decode(q, *pools, seq_lens, block_tables=tables), q, k, v, seq_lens)
+
+
+# The three-head workgroups against the oracle: spans of 4, 2 and 1 KV heads, splits without keys, a
+# transposed cache, and pages.
+@pytest.mark.parametrize("heads_kv,head_dim", [(8, 128), (2, 64), (5, 128)])
+@pytest.mark.parametrize("num_splits", [None, 1, 3, 64])
+def test_group_of_three_matches_reference(num_splits, heads_kv, head_dim):
+    print(f"decode group of 3 {heads_kv} {head_dim} splits={num_splits}", flush=True)
+    batch, capacity, heads = 12, 2064, 3 * heads_kv
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    q = torch.randn(batch, 1, heads, head_dim, device="cuda", dtype=torch.bfloat16, generator=gen)
+    k, v = (torch.randn(batch, heads_kv, capacity, head_dim, device="cuda", dtype=torch.bfloat16, generator=gen)
+            .transpose(1, 2) for _ in range(2))
+    seq_lens = torch.randint(1, capacity + 1, (batch,), device="cuda", generator=gen).to(torch.int32)
+    seq_lens[:2] = torch.tensor([capacity, 1])
+    out, lse = flash_lab.decode(q, k, v, seq_lens, num_splits=num_splits, return_lse=True)
+    check_decode(out, lse, q, k, v, seq_lens)
+    tables = torch.arange(batch * capacity // 16, device="cuda", dtype=torch.int32).view(batch, -1)
+    pools = [x.reshape(-1, 16, heads_kv, head_dim) for x in (k, v)]
+    out, lse = flash_lab.decode(q, *pools, seq_lens, num_splits=num_splits, block_tables=tables, return_lse=True)
+    check_decode(out, lse, q, k, v, seq_lens)

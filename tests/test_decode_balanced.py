@@ -131,8 +131,8 @@ def test_split_counts():
     assert plan(8, 32, 8, 128, 16000, dtype=2)[:2] == (4, 0)
     assert plan(4, 8, 8, 128, 3000)[:2] == (8, 0)
     assert plan(1, 32, 32, 128, 32768)[:2] == (16, 0)  # long: as planned
-    # Groups of 3: matrix cores (one KV head per workgroup: 32 splits), and in fp32, where three workgroups
-    # read the same keys, splits of 180 keys or more.
+    # Groups of 3: three heads per workgroup (32 splits), and in fp32, where three workgroups read the same
+    # keys, splits of 180 keys or more.
     assert plan(1, 24, 8, 128, 8192)[:2] == (32, 0)
     assert plan(4, 24, 8, 128, 4000, dtype=2)[:2] == (16, 0)
     # A paged call keeps a split's block numbers within LDS.
