@@ -182,9 +182,9 @@ BalancedLayout balanced_layout(const fl_decode_params* p, const fl::DecodeLayout
   BalancedLayout r{};
   const int forced = layout.mfma ? fl::knob(FL_KNOB_DECODE_MFMA_SPAN) : -1;
   for (r.span = layout.mfma ? kMfmaSpan : layout.kv_span; r.span > 1; r.span /= 2) {
-    if (p->heads_kv % r.span != 0 || (layout.mfma && r.span != kMfmaSpan) || forced == 1) continue;
+    if (p->heads_kv % r.span != 0 || (layout.mfma && r.span != kMfmaSpan)) continue;
     const double keys = double(p->batch) * (p->heads_kv / r.span) * chunks * p->max_seqlen;
-    if (forced == r.span || keys >= double(keys_per_wg) * wgs) break;
+    if (forced >= 1 ? forced == r.span : keys >= double(keys_per_wg) * wgs) break;
   }
   r.unit_shift = 5;
   r.min_units = 4;

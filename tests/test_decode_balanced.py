@@ -139,6 +139,15 @@ def test_split_counts():
     assert plan(1, 16, 8, 128, 131072, page_size=1)[0] == 128
 
 
+@pytest.mark.parametrize("span", [1, 2, 3, 4])
+def test_forced_spans(span, knobs):
+    # 4 KV heads per workgroup, or, at any other value of the knob, one: 48 rows of 16 heads or 192 of 4.
+    knobs("decode_mfma_span", span)
+    rows = 48 if span == 4 else 192
+    want = (256 + rows * 9) * (24 * 32 // rows) * 130 * 4 + rows * 8
+    assert plan(24, 32, 8, 128, 8192, page_size=16) == (0, 256, want)
+
+
 def test_balanced_call_is_checked_before_any_launch():
     p = _hip.DecodeParams()
     p.q = p.k_cache = p.v_cache = p.o = p.lse = p.seq_lens = 256
