@@ -645,8 +645,10 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
   // would take off it cost less than the pass (about 3.9 us, against 11.5 us per 1,000 keys): (B, H,
   // H_kv, S) (16, 32, 8, 320) 10.3 us with one split, 11.9 with two, (2, 8, 8, 90) 3.8 and 6.3, (4, 32,
   // 8, 640) 13.2 and 9.6 with eight.
+  // (Neither this nor scheduled_splits where the knob asks for fl_decode_plan's count at another residency.)
+  const bool plan_only = fl::knob(FL_KNOB_DECODE_WG_PER_CU) >= 1;
   const double fill = double(p->batch) * p->heads_kv / (cu_count > 0 ? cu_count : 256);
-  if (p->max_seqlen < 640 && p->max_seqlen * (fill < 1.0 ? 1.0 - fill : 0.0) < 340.0) {
+  if (!plan_only && p->max_seqlen < 640 && p->max_seqlen * (fill < 1.0 ? 1.0 - fill : 0.0) < 340.0) {
     *num_splits = 1;
     *workspace_bytes = 0;
     return FL_OK;
@@ -654,8 +656,7 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
   const int cus = cu_count > 0 ? cu_count : 256;
   if (!worth_balancing(p, layout, *num_splits, cus)) {
     // (A paged plan also keeps each split's block numbers within LDS: never fewer splits then.)
-    const int n = fl::knob(FL_KNOB_DECODE_WG_PER_CU) >= 1 ? *num_splits
-                                                          : scheduled_splits(p, layout, cus, *num_splits);
+    const int n = plan_only ? *num_splits : scheduled_splits(p, layout, cus, *num_splits);
     if (p->block_tables == nullptr || pages_per_split(p->max_seqlen, n, p->page_size) <= fl::kMaxSplitPages)
       *num_splits = n;
     *workspace_bytes = *num_splits > 1 ? static_cast<size_t>(p->batch) * p->heads * *num_splits *

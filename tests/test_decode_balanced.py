@@ -148,6 +148,13 @@ def test_forced_spans(span, knobs):
     assert plan(24, 32, 8, 128, 8192, page_size=16) == (0, 256, want)
 
 
+@pytest.mark.parametrize("shape", [(1, 8, 8, 128, 300), (16, 32, 8, 128, 320), (2, 8, 8, 64, 90), (4, 32, 8, 128, 4000)],
+                         ids=str)
+def test_workgroups_per_cu_knob_gives_the_plans_count(shape, knobs):
+    knobs("decode_wg_per_cu", 4)
+    assert plan(*shape)[:2] == (_hip.decode_plan(*shape, torch.bfloat16)[0], 0)
+
+
 def test_balanced_call_is_checked_before_any_launch():
     p = _hip.DecodeParams()
     p.q = p.k_cache = p.v_cache = p.o = p.lse = p.seq_lens = 256
