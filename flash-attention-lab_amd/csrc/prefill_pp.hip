@@ -850,7 +850,7 @@ int prefill_pp_block_rows(int head_dim) {
 // fill the CUs gain nothing ((1, 32, 8, 2048, 2048, 128) 49, 60 with two splits), nor do short ones
 // ((1, 32, 8, 512, 1024, 128) 17, 28 with two).
 int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count) {
-  if (knob(FL_KNOB_PREFILL_PP_MIN_WG) >= 0 || knob(FL_KNOB_PREFILL_CAUSAL_STREAM) >= 0) return 1;
+  if (knob(FL_KNOB_PREFILL_PP_MIN_WG) >= 0 || knob(FL_KNOB_PREFILL_CAUSAL_STREAM) == 1) return 1;
   const int cus = cu_count > 0 ? cu_count : 256;
   const int block_rows = prefill_pp_block_rows(head_dim);
   const int64_t q_blocks = (args.rows + block_rows - 1) / block_rows;

@@ -215,13 +215,17 @@ int fl_mfma_tile_test(const void* a, const void* b, float* c, int32_t k, int32_t
  *   FL_KNOB_PREFILL_PP_MIN_WG      [0, 2^30]: fewest ping-pong workgroups
  *                                  for which prefill runs the ping-pong
  *                                  kernel (default 256 non-causal, 128
- *                                  causal; 0 = always, 2^30 = never).
+ *                                  causal; 0 = always, 2^30 = never). Any
+ *                                  value also keeps the keys unsplit where
+ *                                  the caller asks for no split count.
  *   FL_KNOB_DECODE_MFMA_MIN_GROUP  [1, 2^20]: smallest GQA group the
  *                                  matrix-core decode kernel takes (default
  *                                  4 at head_dim 128 and 64; above 32 =
  *                                  never).
  *   FL_KNOB_DECODE_WG_PER_CU       [1, 64]: resident split workgroups per CU
- *                                  that fl_decode_plan assumes.
+ *                                  that fl_decode_plan assumes; its count
+ *                                  is then fl_decode_schedule's too, and a
+ *                                  balanced call has that many workgroups.
  *   FL_KNOB_DECODE_MFMA_SPAN       [1, 4]: KV heads per workgroup of the
  *                                  matrix-core decode kernel, 1 or 4 (4 only
  *                                  where H_kv is a multiple of 4; other
@@ -231,7 +235,9 @@ int fl_mfma_tile_test(const void* a, const void* b, float* c, int32_t k, int32_t
  *                                  causal pair of query blocks: 0 = two
  *                                  blocks one after the other (the default),
  *                                  1 = one stream of key tiles (measured
- *                                  slower; kept for comparison).
+ *                                  slower; kept for comparison; keys stay
+ *                                  unsplit where the caller asks for no
+ *                                  split count).
  */
 enum fl_knob {
   FL_KNOB_PREFILL_PP_MIN_WG = 0,

@@ -45,6 +45,18 @@ def test_plan():
         assert plan((1, 300, 8492, 32, 8, 128), requested)[0] == 1
 
 
+def test_knobs_that_pin_a_kernel_keep_the_keys_unsplit(knobs):
+    shape = (1, 300, 8492, 32, 8, 128)
+    want = plan(shape)
+    knobs("prefill_causal_stream", 0)  # the default's own value changes nothing
+    assert plan(shape) == want and want[1] > 1
+    knobs("prefill_causal_stream", 1)
+    assert plan(shape) == (0, 1, 0)
+    knobs("prefill_causal_stream", None)
+    knobs("prefill_pp_min_wg", 256)
+    assert plan(shape) == (0, 1, 0)
+
+
 def test_workspace_is_checked_before_any_launch():
     p = params((1, 300, 8492, 32, 8, 128))
     buf = torch.empty(1024, dtype=torch.int64)
