@@ -420,7 +420,14 @@ decode_split_kernel(const DecodeArgs a) {
         vr[u] = load16_stream(v_row(key));
       }
     };
-    auto use_batch = [&](int base, const u32x4 (&kr)[kUnroll], const u32x4 (&vr)[kUnroll]) {
+    auto use_batch = [&](int base, const u32x4 (&kr)[kUnroll], u32x4 (&vr)[kUnroll]) {
+      // A masked key's probability is 0, which an infinite value in the row it is clamped to would make
+      // NaN. Segments end within a batch at any 32nd key; splits only at the sequence's end.
+      if (kBalanced && base + kKeysPerIter > k_end) {
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u)
+          if (base + u * kGroups + group >= k_end) vr[u] = u32x4{0, 0, 0, 0};
+      }
 #pragma unroll
       for (int g = 0; g < kHeads; ++g) {
         float s[kUnroll];

@@ -269,3 +269,45 @@ def test_planned_balanced_decode_replays_on_new_lengths():
             blocks = tables[b, : -(-n // 16)].long()
             kc, vc = (t[blocks].flatten(0, 1)[None, :n] for t in (k, v))
             check_decode(out[b : b + 1], lse[b : b + 1], q[b : b + 1], kc, vc, lens[b : b + 1])
+
+
+# Infinities and NaN in one sequence's cache: what a fixed split count gives for it, and no effect on the
+# others. fp32 (eight query heads) and groups of 1 and 3 run on the vector kernel. An infinite value is at
+# every place of a 32-key unit in turn, among them the last keys of workgroups' segments.
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads_kv,group,dtype", [(2, 1, torch.bfloat16), (1, 3, torch.bfloat16),
+                                                  (1, 8, torch.float32), (1, 8, torch.float16)], ids=str)
+def test_balanced_decode_with_infinities_and_nan(heads_kv, group, dtype):
+    batch, longest = 3, 3000
+    q, k, v, lens = inputs((batch, heads_kv * group, heads_kv, longest, 64, [2990, 700, 3000]), dtype)
+    q = q * 0.1  # no probability underflows
+    workgroups = 45 * heads_kv  # five units each: a segment ends within a batch of 64 or 128 keys
+    assert schedule([2990, 700, 3000], heads_kv, workgroups, 32, 4, 2)[0] == 5
+    want, want_lse = balanced(q, k, v, lens, workgroups)
+    vector = dtype == torch.float32 or group < 4
+    print(f"balanced non-finite {heads_kv} {group} {dtype}", flush=True)
+    infinite = v.clone()
+    places = 2528 + 33 * torch.arange(14, device="cuda")  # from its 79th unit on, each at another place in it
+    places = places[places < 2990 - 1]
+    infinite[0, places, 0, 3] = float("inf")
+    infinite[0, 127:2528:32, 0, 5] = -float("inf")  # last keys of units
+    for num_splits in (None, 1, 7):
+        if num_splits is None:
+            out, lse = balanced(q, k, infinite, lens, workgroups)
+            assert torch.equal(out[1:], want[1:]) and torch.equal(lse, want_lse)
+        else:
+            out, lse = flash_lab.decode(q, k, infinite, lens, num_splits=num_splits, return_lse=True)
+        assert torch.isposinf(out[0, 0, :group, 3]).all() and torch.isneginf(out[0, 0, :group, 5]).all()
+        rest = out.clone()
+        rest[0, 0, :group, [3, 5]] = 0
+        assert torch.isfinite(rest).all()
+    for bad in (float("nan"), float("inf")):
+        broken = k.clone()
+        broken[0, 1234, 0] = bad
+        out, lse = balanced(q, broken, v, lens, workgroups)
+        assert torch.equal(out[1:], want[1:]) and torch.equal(lse[1:], want_lse[1:])
+        if vector:
+            fixed, fixed_lse = flash_lab.decode(q, broken, v, lens, num_splits=7, return_lse=True)
+            assert torch.equal(out[0, 0, :group], fixed[0, 0, :group])
+            assert torch.equal(lse[0, :group], fixed_lse[0, :group])
+            assert torch.equal(out[0, 0, group:], want[0, 0, group:])
