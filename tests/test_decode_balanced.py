@@ -271,6 +271,76 @@ def test_planned_balanced_decode_replays_on_new_lengths():
             check_decode(out[b : b + 1], lse[b : b + 1], q[b : b + 1], kc, vc, lens[b : b + 1])
 
 
+# One long sequence among short ones on one KV head, its row cut into more partials than the merge pass
+# takes at a time (128): (batch, longest, workgroups, partials that the long row has at least). The last
+# one's rows are not padded to whole chunks.
+LONG_ROWS = [(2, 20000, 300, 129), (2, 36000, 300, 257), (64, 32000, 229, 129)]
+
+
+def long_row_lens(batch, longest):
+    lens = [1 + 7 * i % 32 for i in range(batch)]
+    lens[batch // 2 - 1] = longest
+    return lens
+
+
+@pytest.mark.parametrize("ramp_units", [2, 4])  # vector and matrix-core kernel
+def test_long_rows_have_more_partials_than_one_merge_step(ramp_units):
+    for batch, longest, workgroups, least in LONG_ROWS:
+        lens = long_row_lens(batch, longest)
+        chunk, starts, sizes = schedule(lens, 1, workgroups, 32, 4, ramp_units)
+        row = batch // 2 - 1
+        assert (starts[row] + -(-longest // 32) - 1) // chunk - starts[row] // chunk + 1 >= least
+        assert (starts[row] % chunk != 0) == (batch == 64)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,dtype", [(8, torch.bfloat16), (8, torch.float32), (3, torch.bfloat16),
+                                         (2, torch.float16), (1, torch.float32)], ids=str)
+@pytest.mark.parametrize("case", LONG_ROWS, ids=str)
+def test_rows_of_many_partials_match_reference(case, heads, dtype):
+    batch, longest, workgroups, _ = case
+    print(f"balanced long row {case} heads={heads} {dtype}", flush=True)
+    q, k, v, lens = inputs((batch, heads, 1, longest, 64, long_row_lens(batch, longest)), dtype)
+    out, lse = balanced(q, k, v, lens, workgroups)
+    check_decode(out, lse, q, k, v, lens)
+    if dtype == torch.float32:
+        assert normwise_rel(out.cpu(), reference.decode(q.cpu(), k.cpu(), v.cpu(), lens.cpu())) <= 1e-5
+    again = balanced(q, k, v, lens, workgroups)
+    assert torch.equal(again[0], out) and torch.equal(again[1], lse)
+
+
+# Layouts beside the contiguous [B, S, H_kv, D] one: transposed caches, query heads a stride apart, pages
+# of 1 and 7 rows. 8 rows of 992 keys on 8 workgroups of the matrix-core kernel: with pages of one row
+# every segment's block numbers nearly fill their 1,024 places in LDS.
+LAYOUT_CASES = [
+    (4, 8, 2, 992, 128, [992, 992, 992, 992], 8),
+    (9, 16, 4, 2002, 64, "random", 256),
+    (6, 4, 4, 1500, 64, [1500, 0, 1, 33, 999, 1499], 100),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("case", LAYOUT_CASES, ids=lambda c: f"B{c[0]}-H{c[1]}-Hkv{c[2]}-S{c[3]}-D{c[4]}")
+def test_balanced_decode_on_other_layouts(case, dtype):
+    *shape, workgroups = case
+    print(f"balanced layouts {case} {dtype}", flush=True)
+    q, k, v, lens = inputs(tuple(shape), dtype)
+    q = q.repeat_interleave(2, dim=2)[:, :, ::2]
+    kt, vt = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (k, v))
+    out, lse = balanced(q, kt, vt, lens, workgroups)
+    full = lens > 0
+    check_decode(out[full], lse[full], q[full], k[full], v[full], lens[full])
+    assert torch.all(out[~full] == 0) and torch.isneginf(lse[~full]).all()
+    for page in (1, 7):
+        (k_pool, tables), (v_pool, _) = paged(k, page), paged(v, page)
+        print(f"pages of {page}", flush=True)
+        got = balanced(q, k_pool, v_pool, lens, workgroups, tables)
+        if tables.shape[1] * page == k.shape[1]:  # the same capacity: the same keys per workgroup
+            assert torch.equal(got[0], out) and torch.equal(got[1], lse)
+        check_decode(got[0][full], got[1][full], q[full], k[full], v[full], lens[full])
+
+
 # Infinities and NaN in one sequence's cache: what a fixed split count gives for it, and no effect on the
 # others. fp32 (eight query heads) and groups of 1 and 3 run on the vector kernel. An infinite value is at
 # every place of a 32-key unit in turn, among them the last keys of workgroups' segments.

@@ -138,3 +138,36 @@ def test_planned_splits_match_reference_and_replay(shape):
         torch.cuda.synchronize()
         assert torch.equal(got, out) and torch.equal(got_lse, lse)
         flash_lab.attention(q, k, v, causal=True)
+
+
+# Infinities and NaN in the keys and values of one KV head: what the unsplit forms and torch give (an
+# infinite value is the output's, a NaN score makes the row NaN), wherever in the splits' shares and in the
+# halves of a tile they are, and no effect on the other heads. (1, 150, 300, 8, 2): half tiles where not split.
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("num_splits", [1, 2, 3, 9])
+def test_infinities_and_nan(num_splits, head_dim, knobs):
+    knobs("prefill_pp_min_wg", 1 << 30)
+    q = torch.randn(1, 150, 8, head_dim, device="cuda", dtype=torch.bfloat16) * 0.1  # no probability underflows
+    k, v = (torch.randn(1, 300, 2, head_dim, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+
+    def call(k, v):
+        if num_splits == 1:
+            return flash_lab.attention(q, k, v, return_lse=True)
+        return split_prefill(q, k, v, False, head_dim**-0.5, num_splits)
+
+    want, want_lse = call(k, v)
+    for key in (0, 31, 40, 63, 64, 191, 256, 299):
+        print(f"non-finite prefill splits={num_splits} D={head_dim} key={key}", flush=True)
+        infinite = v.clone()
+        infinite[0, key, 0, 3], infinite[0, key, 0, 5] = float("inf"), -float("inf")
+        out, lse = call(k, infinite)
+        assert torch.isposinf(out[:, :, :4, 3]).all() and torch.isneginf(out[:, :, :4, 5]).all()
+        out[:, :, :4, [3, 5]] = want[:, :, :4, [3, 5]]
+        assert torch.equal(out, want) and torch.equal(lse, want_lse)
+        for bad in (float("nan"), float("inf")):
+            broken = k.clone()
+            broken[0, key, 0] = bad
+            out, lse = call(broken, v)
+            assert torch.isnan(out[:, :, :4]).all() and not torch.isfinite(lse[:, :4]).any()
+            assert torch.equal(out[:, :, 4:], want[:, :, 4:]) and torch.equal(lse[:, 4:], want_lse[:, 4:])
