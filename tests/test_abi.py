@@ -295,3 +295,18 @@ def test_noalloc_decode_rejects_workspaces_beyond_its_scratch_array():
     p.heads_kv = 7  # shape errors come first, as in fl_decode
     assert _hip.LIB.fl_decode_noalloc(ctypes.byref(p), None) == 1
     assert b"multiple of KV heads" in _hip.LIB.fl_last_error()
+
+
+def test_torch_ops_take_the_functions_in_the_order_they_are_passed():
+    # fl_torch_bind takes untyped addresses by position: its parameters are TORCH_BOUND's names in order, and
+    # each one lands in the member of its own name.
+    source = (HEADER.parent.parent / "flash-attention-lab_amd" / "csrc" / "torch_ops.cpp").read_text()
+    signature = re.search(r"void fl_torch_bind\((.*?)\)", source, flags=re.S).group(1)
+    names = re.findall(r"void\* (\w+)", signature)
+    assert tuple(f"fl_{name}" for name in names) == _hip.TORCH_BOUND
+    body = source[source.index("void fl_torch_bind") :]
+    assert re.findall(r"lib\.(\w+) = reinterpret_cast<decltype\(lib\.(\w+)\)>\((\w+)\)", body) == [
+        (name, name, name) for name in names
+    ]
+    members = re.search(r"struct Library \{(.*?)\};", source, flags=re.S).group(1)
+    assert re.findall(r"decltype\(&(\w+)\) (\w+);", members) == [(f"fl_{name}", name) for name in names]
