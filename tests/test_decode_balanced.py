@@ -139,6 +139,12 @@ def test_split_counts():
     assert plan(1, 16, 8, 128, 131072, page_size=1)[0] == 128
 
 
+@pytest.mark.parametrize("shape", [(2, 32, 8, 128, 352), (8, 16, 2, 128, 300), (13, 64, 8, 128, 176)], ids=str)
+def test_short_fp32_caches_of_512_byte_rows_are_split_as_planned(shape):
+    assert plan(*shape, dtype=2)[:2] == (_hip.decode_plan(*shape, torch.float32)[0], 0)
+    assert plan(*shape, dtype=2)[0] > 1 and plan(*shape)[0] == 1  # bf16: one split
+
+
 @pytest.mark.parametrize("span", [1, 2, 3, 4])
 def test_forced_spans(span, knobs):
     # 4 KV heads per workgroup, or, at any other value of the knob, one: 48 rows of 16 heads or 192 of 4.
