@@ -213,14 +213,15 @@ size_t balanced_partials(const fl_decode_params* p, const BalancedLayout& layout
 // 32, 8, 2600) 11.9 / 11.0; several query heads, (8, 16, 8, 32000) bf16 163 / 153, (1, 32, 8, 8320) fp32
 // 23 / 19, (4, 32, 8, 4000) fp32 30 / 27; one, (4, 8, 8, 3000) 14.3 / 13.8. Where several workgroups
 // read the same keys (a group of 3 in fp32), splits of some 200 keys keep those reads close together:
-// (14, 24, 8, 1600, D = 64) 49 / 32, (4, 24, 8, 4000) 69 / 41.
+// (14, 24, 8, 1600, D = 64) 49 / 32, (4, 24, 8, 4000) 69 / 41; on at most 12 workgroups per CU: (10, 24, 8,
+// 10848, D = 64) 124 us with 8 splits, 140 with 16.
 int scheduled_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, int cus, int planned) {
   const int64_t chunks = p->heads / p->heads_kv / layout.wg_heads;
   const int64_t work = static_cast<int64_t>(p->batch) * p->heads_kv * chunks;
   int n = largest_splits(work, p->max_seqlen, cus, 64);
   if (layout.mfma) return mfma_span(p, layout, planned) == 1 ? n : planned;
   if (chunks > 1)
-    while (n < fl::kMaxSplits && work * 2 * n <= 16 * static_cast<int64_t>(cus) && p->max_seqlen / (2 * n) >= 180) n *= 2;
+    while (n < fl::kMaxSplits && work * 2 * n <= 12 * static_cast<int64_t>(cus) && p->max_seqlen / (2 * n) >= 180) n *= 2;
   // Not where the power of two leaves a tenth of the CUs without a workgroup: (20, 32, 8, 1500) fp32 with
   // unequal lengths 33 us as planned, 50 with one split.
   if (layout.heads_per_wg > 1 || chunks > 1) return 10 * work * n >= 9 * static_cast<int64_t>(cus) ? n : planned;
@@ -241,6 +242,12 @@ int scheduled_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, 
 bool worth_balancing(const fl_decode_params* p, const fl::DecodeLayout& layout, int num_splits, int cus) {
   const double bytes = 2.0 * p->batch * p->heads_kv * p->max_seqlen * p->head_dim * elem_bytes(p->dtype);
   if (p->batch < 6 || bytes < 1048576.0 * cus) return false;
+  // Groups of one-head workgroups, which read the same keys, drift apart over long segments (paged, fp32,
+  // group of 3, planned / balanced / scheduled_splits, equal lengths, then spread: (10, 24, 8, 10848) 359 /
+  // 401 / 293, 266 / 236 / 186, (7, 24, 8, 5000) 126 / 135 / 97, 99 / 81 / 56, (32, 24, 8, 4096, D = 64) 253 /
+  // 246 / 212, 186 / 131 / 142). With eight heads each the balanced form holds: (16, 64, 4, 8192, D = 64) 110 /
+  // 105 / 107, 81 / 68 / 81.
+  if (layout.heads_per_wg == 1 && layout.wg_heads < p->heads / p->heads_kv) return false;
   return p->block_tables != nullptr || (!layout.mfma && layout.heads_per_wg == 1 && num_splits > 1);
 }
 

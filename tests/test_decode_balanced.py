@@ -145,6 +145,15 @@ def test_short_fp32_caches_of_512_byte_rows_are_split_as_planned(shape):
     assert plan(*shape, dtype=2)[0] > 1 and plan(*shape)[0] == 1  # bf16: one split
 
 
+def test_workgroups_that_share_keys_are_not_balanced():
+    # Groups of 3 in fp32: three workgroups read the same keys, and short splits keep those reads together.
+    assert plan(10, 24, 8, 128, 10848, dtype=2, page_size=16)[:2] == (8, 0)
+    assert plan(24, 24, 8, 128, 2048, dtype=2, page_size=16)[:2] == (4, 0)
+    assert plan(8, 24, 8, 64, 4096, dtype=2, page_size=16)[:2] == (16, 0)
+    assert plan(10, 24, 8, 128, 10848, page_size=16)[0] == 0  # bf16: one workgroup for the three heads
+    assert plan(16, 32, 8, 128, 8192, dtype=2, page_size=16)[0] == 0  # fp32, four heads per workgroup
+
+
 @pytest.mark.parametrize("span", [1, 2, 3, 4])
 def test_forced_spans(span, knobs):
     # 4 KV heads per workgroup, or, at any other value of the knob, one: 48 rows of 16 heads or 192 of 4.
