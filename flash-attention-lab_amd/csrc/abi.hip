@@ -170,7 +170,10 @@ int mfma_span_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, 
 // the widest span that leaves a workgroup 512 keys of its KV heads, 1,024 on the matrix-core kernel),
 // keys per unit and what one more segment costs a workgroup, in units (a segment's start is about
 // 2.5 us, in which a CU streams about 64 KiB). At most kMaxBalancedBatch sequences, a line within
-// 2^22 units, and, paged, segments whose block numbers fit LDS whatever the lengths are.
+// 2^22 units, and, paged, segments whose block numbers fit LDS whatever the lengths are. Few matrix-core
+// rows have many partials each, and take the wide span from 1,536 keys (us, four KV heads / one, equal lengths,
+// then spread): (8, 32, 4, 32768) 103 / 98, 76 / 65, (6, 32, 4, 49152) 118 / 113, 90 / 75; (10, 32, 8, 16384,
+// D = 64) 67 / 70, 41 / 44, (64, 32, 8, 2048) 93 / 97, 61 / 69, (6, 32, 8, 32768) 135 / 140, 86 / 89.
 struct BalancedLayout {
   bool fits;
   int span, unit_shift, min_units, ramp_units;
@@ -183,8 +186,10 @@ BalancedLayout balanced_layout(const fl_decode_params* p, const fl::DecodeLayout
   const int forced = layout.mfma ? fl::knob(FL_KNOB_DECODE_MFMA_SPAN) : -1;
   for (r.span = layout.mfma ? kMfmaSpan : layout.kv_span; r.span > 1; r.span /= 2) {
     if (p->heads_kv % r.span != 0 || (layout.mfma && r.span != kMfmaSpan)) continue;
-    const double keys = double(p->batch) * (p->heads_kv / r.span) * chunks * p->max_seqlen;
-    if (forced >= 1 ? forced == r.span : keys >= double(keys_per_wg) * wgs) break;
+    const int64_t rows = p->batch * (p->heads_kv / r.span) * chunks;
+    const double wg_keys = double(rows) * p->max_seqlen / wgs;
+    const bool wide = wg_keys >= keys_per_wg && (!layout.mfma || rows >= 12 || wg_keys >= 1.5 * keys_per_wg);
+    if (forced >= 1 ? forced == r.span : wide) break;
   }
   r.unit_shift = 5;
   r.min_units = 4;

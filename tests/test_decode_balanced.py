@@ -154,6 +154,17 @@ def test_workgroups_that_share_keys_are_not_balanced():
     assert plan(16, 32, 8, 128, 8192, dtype=2, page_size=16)[0] == 0  # fp32, four heads per workgroup
 
 
+@pytest.mark.parametrize("shape,span", [
+    ((8, 32, 4, 128, 32768), 1), ((6, 32, 4, 128, 49152), 1),  # 8 and 6 rows with four KV heads in each
+    ((64, 32, 8, 128, 2048), 4), ((10, 32, 8, 64, 16384), 4),  # 128 and 20 rows
+], ids=str)
+def test_balanced_spans(shape, span):
+    batch, heads, heads_kv, head_dim = shape[:4]
+    rows = batch * heads_kv // span
+    want = (256 + rows * 9) * (batch * heads // rows) * (head_dim + 2) * 4 + rows * 8
+    assert plan(*shape, page_size=16) == (0, 256, want)
+
+
 @pytest.mark.parametrize("span", [1, 2, 3, 4])
 def test_forced_spans(span, knobs):
     # 4 KV heads per workgroup, or, at any other value of the knob, one: 48 rows of 16 heads or 192 of 4.
