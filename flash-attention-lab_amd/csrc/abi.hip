@@ -420,11 +420,19 @@ void attention_sizes(const fl_attn_params* p, bool split, fl::PrefillArgs& a) {
   // Not, unless the keys are split, where the packed grid is smaller than half the CUs: there the
   // time is that of one workgroup's rows, and separate heads spread them over more CUs ((1, 64, 8),
   // 18 new rows after 1,194 keys, D = 128: 23.0 us separate, 25.0 packed). Nor past pack_position's
-  // range.
+  // range. Nor causal calls whose separate heads are one round of ping-pong blocks, where the packed ones
+  // are too few pairs for that kernel and more than a round for the 4-wave one (us, separate / packed; (B, H,
+  // H_kv, S_q, S_k, D)): (8, 32, 4, 186, 186, 128) 11.9 / 14.3, (15, 16, 2, 224, 644, 128) 25.3 / 29.3, (3, 64,
+  // 8, 250, 594, 64) 15.6 / 18.5; with no more than a round, (6, 32, 8, 145, 336, 128) 14.4 / 12.1.
   const int64_t packed_rows = static_cast<int64_t>(p->seqlen_q) * a.group;
   const int64_t packed_grid = (packed_rows + fl::kPrefillBlockM - 1) / fl::kPrefillBlockM *
                               p->batch * p->heads_kv;
-  a.pack = packed_rows < (int64_t{1} << 30) && (split || packed_grid >= 128) ? a.group : 1;
+  const int pp_rows = fl::prefill_pp_block_rows(p->head_dim);
+  const int64_t heads = static_cast<int64_t>(p->batch) * p->heads;
+  const int64_t packed_pairs = (packed_rows + 2 * pp_rows - 1) / (2 * pp_rows) * p->batch * p->heads_kv;
+  const bool one_round = a.causal && p->seqlen_q <= pp_rows && heads >= 128 && heads <= 256 &&
+                         packed_pairs < 128 && packed_grid > 256;
+  a.pack = packed_rows < (int64_t{1} << 30) && (split || (packed_grid >= 128 && !one_round)) ? a.group : 1;
   a.work_heads = p->heads / a.pack;
   a.rows = p->seqlen_q * a.pack;
   // Division by a constant d < 2^31 of any n < 2^31 as a multiplication: with 2^l >= d,

@@ -69,3 +69,19 @@ def test_causal_block_orders(batch):
     q, k, v = (torch.randn(batch, 490, h, 128, device="cuda", dtype=torch.bfloat16) for h in (4, 2, 2))
     out, lse = flash_lab.attention(q, k, v, causal=True, return_lse=True)
     check_prefill(out, lse, q, k, v, True, rows=torch.arange(0, 490, 7))
+
+
+# Causal calls with one ping-pong block per query head in one round: separate heads where the packed rows
+# would be fewer than 128 pairs of that kernel's blocks and more than 256 of the 4-wave kernel's, packed at 256
+# of these.
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(8, 186, 186, 32, 4, 128), (8, 128, 200, 32, 4, 128), (3, 250, 594, 64, 8, 64)],
+                         ids=str)
+def test_one_round_of_heads(shape):
+    print(f"one round of heads {shape}", flush=True)
+    batch, seqlen_q, seqlen_k, heads, heads_kv, head_dim = shape
+    q = torch.randn(batch, seqlen_q, heads, head_dim, device="cuda", dtype=torch.bfloat16)
+    k, v = (torch.randn(batch, heads_kv, seqlen_k, head_dim, device="cuda", dtype=torch.bfloat16).transpose(1, 2)
+            for _ in range(2))
+    out, lse = flash_lab.attention(q, k, v, causal=True, return_lse=True)
+    check_prefill(out, lse, q, k, v, True)
