@@ -145,6 +145,11 @@ def test_short_fp32_caches_of_512_byte_rows_are_split_as_planned(shape):
     assert plan(*shape, dtype=2)[0] > 1 and plan(*shape)[0] == 1  # bf16: one split
 
 
+@pytest.mark.parametrize("shape", [(1, 24, 8, 128, 144), (18, 32, 8, 128, 128), (2, 64, 8, 128, 48)], ids=str)
+def test_the_shortest_fp32_caches_take_one_split(shape):
+    assert plan(*shape, dtype=2) == (1, 0, 0)
+
+
 def test_workgroups_that_share_keys_are_not_balanced():
     # Groups of 3 in fp32: three workgroups read the same keys, and short splits keep those reads together.
     assert plan(10, 24, 8, 128, 10848, dtype=2, page_size=16)[:2] == (8, 0)
