@@ -754,9 +754,12 @@ hipError_t launch_typed(PrefillArgs args, hipStream_t stream) {
   // rounds' workgroups that pairs fill): (1, 32, 8, 5000, 128) 63% 188 / 233, (8, 16, 16, 2048, 64)
   // 75% 95 / 116, (5, 32, 8, 2048, 128) 83% 181 / 184, (14, 32, 8, 512, 128) 88% 63 / 58, (16, 32, 8,
   // 700, 128) 100% 114 / 104; with many blocks per head a start weighs less: (1, 32, 8, 7000, 128)
-  // 86% 340 / 347, (3, 24, 8, 4627, 64) 89% 218 / 230.
+  // 86% 340 / 347, (3, 24, 8, 4627, 64) 89% 218 / 230. Two short blocks per head at head_dim 128 in up to two
+  // rounds are mostly starts: (25, 16, 16, 482, 128) 78% 65 / 62, (13, 32, 32, 436, 128) 81% 62 / 58; (12, 32, 32,
+  // 500, 128) 75% 57 / 60; in three, (26, 32, 32, 321, 128) 81% 100 / 102.
   const int64_t slots = static_cast<int64_t>((pairs + kCus - 1) / kCus) * kCus;
-  args.paired = int64_t{100} * pairs >= (args.q_blocks >= 32 ? 90 : 85) * slots;
+  const int line = args.q_blocks >= 32 ? 90 : D == 128 && args.q_blocks == 2 && pairs <= 2 * kCus ? 77 : 85;
+  args.paired = int64_t{100} * pairs >= line * slots;
   const int blocks = args.causal && args.paired ? pairs : args.q_blocks * args.batch * args.work_heads;
   hipLaunchKernelGGL((prefill_pp_kernel<Tag, D, false>), dim3(blocks), dim3(64 * kPpWavesOf<D>), 0, stream, args);
   return hipGetLastError();
