@@ -668,11 +668,12 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
   // (Neither this nor scheduled_splits where the knob asks for fl_decode_plan's count at another residency.)
   const bool plan_only = fl::knob(FL_KNOB_DECODE_WG_PER_CU) >= 1;
   const double fill = double(p->batch) * p->heads_kv / (cu_count > 0 ? cu_count : 256);
-  // Rows of 512 bytes (fp32, head_dim 128) take a workgroup two to six times as long, by its query heads (about
-  // 24 us per 1,000 keys with one, 44 with four, 70 with eight): one split / planned, (1, 24, 8, 144) 4.9 / 6.7, (18,
-  // 32, 8, 128) 10.7 / 12.0; (2, 32, 8, 352) 14.7 / 10.2, (8, 16, 2, 300) 23.3 / 13.9, (13, 64, 8, 176) 16.6 / 14.5.
+  // Rows of 512 bytes (fp32, head_dim 128) take a workgroup two to six times as long, more with more query
+  // heads, so the line lies lower, between one split / planned, (1, 24, 8, 144) 4.9 / 6.7, (1, 32, 8, 144) 8.6 / 9.2,
+  // (18, 32, 8, 128) 10.7 / 12.0, and (1, 32, 32, 300) 9.0 / 7.8, (2, 32, 8, 352) 14.7 / 10.2, (8, 16, 2, 300) 23.3 /
+  // 13.9, (13, 64, 8, 176) 16.6 / 14.5.
   const bool long_rows = p->head_dim * elem_bytes(p->dtype) > 256;
-  const double keys = long_rows ? 3900.0 / (18.0 + 6.5 * layout.heads_per_wg) : 340.0;
+  const double keys = long_rows ? 3900.0 / (16.0 + 2.8 * layout.heads_per_wg) : 340.0;
   if (!plan_only && p->max_seqlen < 640 && p->max_seqlen * (fill < 1.0 ? 1.0 - fill : 0.0) < keys) {
     *num_splits = 1;
     *workspace_bytes = 0;

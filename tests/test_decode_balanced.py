@@ -145,7 +145,7 @@ def test_short_fp32_caches_of_512_byte_rows_are_split_as_planned(shape):
     assert plan(*shape, dtype=2)[0] > 1 and plan(*shape)[0] == 1  # bf16: one split
 
 
-@pytest.mark.parametrize("shape", [(1, 24, 8, 128, 144), (18, 32, 8, 128, 128), (2, 64, 8, 128, 48)], ids=str)
+@pytest.mark.parametrize("shape", [(1, 24, 8, 128, 144), (1, 32, 8, 128, 144), (18, 32, 8, 128, 128), (2, 64, 8, 128, 48)], ids=str)
 def test_the_shortest_fp32_caches_take_one_split(shape):
     assert plan(*shape, dtype=2) == (1, 0, 0)
 
