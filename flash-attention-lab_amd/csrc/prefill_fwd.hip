@@ -411,17 +411,18 @@ hipError_t launch_parts(PrefillArgs args, hipStream_t stream) {
 
 // Half tiles per wave (kParts = 2) where 128-row blocks leave CUs idle or nearly so, of more than one tile:
 // up to 192 of them at head_dim 64; at 128, where a step moves twice the bytes, while a CU gets one block of
-// 64 rows (132: a few CUs with two cost less than the longer step); up to 256 for long causal calls, whose last
-// blocks run alone. Device us, whole / half, bf16: (1, 32, 8, 512, 128) causal (128 blocks) 14.0 / 10.9, (1, 32,
+// 64 rows (132: a few CUs with two cost less than the longer step; 160 for causal calls, half of whose blocks
+// are light); up to 256 for long causal calls, whose last blocks run alone. Device us, whole / half, bf16: (1, 32, 8, 512, 128) causal (128 blocks) 14.0 / 10.9, (1, 32,
 // 8, 256, 128) (64) 9.8 / 7.7, (1, 16, 16, 1000, 64) (128) 17.1 / 11.6, (5, 16, 2, 197, 128) full (130) 9.9 / 8.4,
-// (1, 32, 8, 1024, 128) causal (256) 24.4 / 21.1, (2, 16, 16, 676, 64) full (192) 13.3 / 12.8; not (2, 8, 8, 1133,
+// (1, 32, 8, 1024, 128) causal (256) 24.4 / 21.1, (2, 16, 16, 676, 64) full (192) 13.3 / 12.8, (3, 16, 2, 294,
+// 128) causal (144) 10.1 / 8.1; not (2, 8, 8, 1133,
 // 128) full (144) 25.2 / 26.6, (2, 16, 16, 656, 128) full (192) 17.8 / 19.3, (8, 8, 8, 307, 128) causal (192)
 // 10.5 / 11.3, (3, 32, 8, 300, 128) causal (240) 12.2 / 12.7, (7, 32, 8, 176, 128) full (336) 13.6 / 16.6, (1, 32,
 // 8, 64, 128) 5.2 / 5.5.
 template <typename Tag, int D>
 hipError_t launch_typed(const PrefillArgs& args, hipStream_t stream) {
   const int64_t blocks = static_cast<int64_t>((args.rows + kBlockM - 1) / kBlockM) * args.batch * args.work_heads;
-  const int most = args.causal && args.seqlen_k >= 10 * kBlockN ? 256 : D == 64 ? 192 : 132;
+  const int most = args.causal && args.seqlen_k >= 10 * kBlockN ? 256 : D == 64 ? 192 : args.causal ? 160 : 132;
   if (blocks <= most && args.seqlen_k > kBlockN) return launch_parts<Tag, D, 2>(args, stream);
   return launch_parts<Tag, D, 1>(args, stream);
 }
