@@ -225,8 +225,14 @@ int scheduled_splits(const fl_decode_params* p, const fl::DecodeLayout& layout, 
   const int64_t work = static_cast<int64_t>(p->batch) * p->heads_kv * chunks;
   int n = largest_splits(work, p->max_seqlen, cus, 64);
   if (layout.mfma) return mfma_span(p, layout, planned) == 1 ? n : planned;
-  if (chunks > 1)
+  if (chunks > 1) {
     while (n < fl::kMaxSplits && work * 2 * n <= 12 * static_cast<int64_t>(cus) && p->max_seqlen / (2 * n) >= 180) n *= 2;
+    // Two or four splits of few or small rows don't pay for the merge pass: planned / 2, fp32, (6, 24, 8, 576, D =
+    // 64) 11.2 / 13.2, (10, 24, 8, 400) 15.9 / 18.6, not (5, 24, 8, 528) 16.8 / 14.1; planned / 4, bf16, (6, 24, 8, 800,
+    // D = 64) 9.7 / 10.8, not fp32, (4, 24, 8, 800, D = 64) 11.9 / 9.3.
+    const int64_t bytes = p->max_seqlen * int64_t{p->head_dim} * elem_bytes(p->dtype);
+    if (n <= 4 && bytes < (n == 2 ? 220000 : 200000)) return planned;
+  }
   // Not where the power of two leaves a tenth of the CUs without a workgroup: (20, 32, 8, 1500) fp32 with
   // unequal lengths 33 us as planned, 50 with one split.
   if (layout.heads_per_wg > 1 || chunks > 1) return 10 * work * n >= 9 * static_cast<int64_t>(cus) ? n : planned;
@@ -309,7 +315,7 @@ int decode_call(const fl_decode_params* p, int balanced_wgs, float* workspace, s
 
   const int group = p->heads / p->heads_kv;
   const fl::DType dt = decode_dtype(p->dtype);
-  const fl::DecodeLayout layout = fl::decode_layout(dt, p->head_dim, p->heads_kv, group, cache_rows(p));
+  const fl::DecodeLayout layout = fl::decode_layout(dt, p->head_dim, p->heads_kv, group, cache_rows(p), p->max_seqlen);
   const int head_chunks = group / layout.heads_per_wg;
   const int num_splits = balanced_wgs > 0 ? 0 : p->num_splits;
   const int64_t blocks = static_cast<int64_t>(p->batch) * p->heads_kv * head_chunks * num_splits;
@@ -609,7 +615,7 @@ int fl_decode_plan(const fl_decode_params* p, int32_t requested_splits, int32_t 
     return fail(FL_ERR_INVALID, "null output pointer");
   const int group = p->heads / p->heads_kv;
   const fl::DecodeLayout layout =
-      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, group, cache_rows(p));
+      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, group, cache_rows(p), p->max_seqlen);
   int n = 1;
   if (allow_splits && requested_splits > 0) {
     n = requested_splits;
@@ -660,7 +666,7 @@ int fl_decode_schedule(const fl_decode_params* p, int32_t cu_count, int32_t* num
   if (int rc = fl_decode_plan(p, 0, 1, cu_count, num_splits, workspace_bytes)) return rc;
   *workgroups = 0;
   const fl::DecodeLayout layout =
-      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, p->heads / p->heads_kv, cache_rows(p));
+      fl::decode_layout(decode_dtype(p->dtype), p->head_dim, p->heads_kv, p->heads / p->heads_kv, cache_rows(p), p->max_seqlen);
   // Short caches: one workgroup per KV head and no merge pass, while the keys that more workgroups
   // would take off it cost less than the pass (about 3.9 us, against 11.5 us per 1,000 keys): (B, H,
   // H_kv, S) (16, 32, 8, 320) 10.3 us with one split, 11.9 with two, (2, 8, 8, 90) 3.8 and 6.3, (4, 32,

@@ -23,7 +23,8 @@
 //  * At the end the row groups are merged by a fixed butterfly inside each wave, then the four
 //    waves in order through LDS. With one split the workgroup writes o and lse; otherwise it
 //    writes its unnormalized partial output and (max, sum), and decode_merge_kernel combines the
-//    splits in a fixed order. No atomics: results are bitwise reproducible for a given split count.
+//    splits in a fixed order. No atomics: results are bitwise reproducible for a given split count, and
+//    a balanced call's for the same lengths of all sequences and workgroups.
 //    (Merging in the split kernel's last workgroup per head group was measured slower: every
 //    workgroup then has to wait for its partials to reach device scope and for an atomic before it
 //    frees its slot, which costs more than the second launch.)
@@ -683,16 +684,19 @@ int decode_mfma_min_group() {
 // The matrix-core kernel is no faster there and rounds the probabilities to the input type, which this
 // kernel keeps in fp32. us a call, one head / three / matrix cores, bf16 or fp16: (10, 24, 8, 15868) 273 /
 // 119 / 118, paged with spread lengths 165 / 68 / 69, (1, 24, 8, 8192) 32.7 / 16.8 / 16.8, (16, 24, 8,
-// 4000, D = 64) spread 48.8 / 26.5 / 24.2; smaller (device us, one / three): (1, 24, 8, 640) 8.6 / 10.2,
-// (4, 24, 8, 300) 9.2 / 10.2, (2, 24, 8, 1000, D = 64) 10.0 / 10.5. Two rows in flight per buffer, four:
-// 119 / 130, paged 68 / 84.
-constexpr int64_t kThreeHeadRows = 16384;
+// 4000, D = 64) spread 48.8 / 26.5 / 24.2. Smaller (device us, one / three), at head_dim 128: (8, 24, 8, 304)
+// 8.2 / 9.7, (16, 24, 8, 208) 8.2 / 8.3, (32, 24, 8, 208) 13.5 / 8.9, (4, 24, 8, 528) 11.0 / 9.2; at 64: (4, 24,
+// 8, 528) 5.4 / 8.9, (8, 24, 8, 400) 6.8 / 8.2, (4, 24, 8, 1008) 9.2 / 9.1, (32, 24, 8, 208) 8.1 / 7.0, (8, 24, 8,
+// 800) 10.5 / 10.0. Two rows in flight per buffer, four: 119 / 130, paged 68 / 84.
+int64_t three_head_rows(int head_dim, int max_seqlen) {
+  return head_dim == 64 ? 49152 : max_seqlen >= 512 ? 16384 : 32768;
+}
 
-DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows) {
+DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows, int max_seqlen) {
   DecodeLayout layout{};
   int k = 1;
   while (k < 8 && group % (2 * k) == 0) k *= 2;
-  if (group == 3 && dtype != DType::f32 && cache_rows >= kThreeHeadRows) k = 3;
+  if (group == 3 && dtype != DType::f32 && cache_rows >= three_head_rows(head_dim, max_seqlen)) k = 3;
   layout.heads_per_wg = k;
   if (dtype != DType::f32 && group >= decode_mfma_min_group() &&
       group <= kMaxDecodeMfmaHeads) {

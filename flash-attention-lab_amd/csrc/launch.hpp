@@ -133,11 +133,11 @@ int prefill_splits(const PrefillArgs& args, int head_dim, int cu_count);
 int64_t prefill_partial_floats(const PrefillArgs& args, int head_dim, int num_splits, int64_t* ml_offset);
 // The ping-pong kernel on args.num_splits shares of each block's key tiles, and the merge pass.
 hipError_t launch_prefill_split(const PrefillArgs& args, DType dtype, int head_dim, hipStream_t stream);
+// Query rows per workgroup of the ping-pong kernel at this head_dim.
+int prefill_pp_block_rows(int head_dim);
 // The same kernel for causal calls with a pair of query blocks per workgroup run as one stream of
 // key tiles (prefill_causal.hip); launch_prefill_pingpong routes causal calls to it when the
 // FL_KNOB_PREFILL_CAUSAL_STREAM knob is 1.
-// Query rows per workgroup of the ping-pong kernel at this head_dim.
-int prefill_pp_block_rows(int head_dim);
 hipError_t launch_prefill_causal_stream(const PrefillArgs& args, DType dtype, int head_dim,
                                         hipStream_t stream);
 
@@ -153,8 +153,8 @@ struct DecodeLayout {
   int mfma;
   int wg_heads;  // query heads per KV head in one split workgroup
 };
-// cache_rows: K (or V) rows of all sequences and KV heads.
-DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows);
+// cache_rows: K (or V) rows of all sequences and KV heads; max_seqlen: of one.
+DecodeLayout decode_layout(DType dtype, int head_dim, int heads_kv, int group, int64_t cache_rows, int max_seqlen);
 hipError_t launch_decode(const DecodeArgs& args, DType dtype, int head_dim, hipStream_t stream);
 // The matrix-core split kernel alone (launch_decode runs it and the merge pass when args.mfma).
 hipError_t launch_decode_mfma_split(const DecodeArgs& args, DType dtype, int head_dim,

@@ -496,11 +496,11 @@ def check_three_head_rounding(out, q, k_cache, v_cache, seq_lens):
         assert err <= half_ulp + 2.0**-17, f"sequence {b}: error {err:.3g}, half an ulp is {half_ulp:.3g}"
 
 
-# Groups of 3 have 32-bit probabilities at every cache size: below kThreeHeadRows cache rows one head per
+# Groups of 3 have 32-bit probabilities at every cache size: below three_head_rows cache rows one head per
 # workgroup, from there on three (csrc/decode.hip).
 @pytest.mark.parametrize("head_dim", [64, 128])
 @pytest.mark.parametrize("dtype", DTYPES[:2], ids=lambda d: str(d).removeprefix("torch."))
-@pytest.mark.parametrize("capacity", [1023, 1024])
+@pytest.mark.parametrize("capacity", [1023, 1024, 3071, 3072])
 def test_group_of_three_keeps_fp32_probabilities(capacity, dtype, head_dim):
     print(f"decode group of 3 {capacity} {dtype} {head_dim}", flush=True)
     batch, heads, heads_kv = 2, 24, 8

@@ -135,6 +135,11 @@ def test_split_counts():
     # keys, splits of 180 keys or more.
     assert plan(1, 24, 8, 128, 8192)[:2] == (32, 0)
     assert plan(4, 24, 8, 128, 4000, dtype=2)[:2] == (16, 0)
+    # ... and one head per workgroup for smaller caches.
+    assert plan(4, 24, 8, 64, 528)[0] == 1 and plan(8, 24, 8, 128, 304)[0] == 1
+    # Two of them, or four of small rows, are left as planned.
+    assert plan(6, 24, 8, 64, 576)[0] == 1 and plan(6, 24, 8, 64, 800)[0] == 1
+    assert plan(10, 24, 8, 128, 400, dtype=2)[0] == 1 and plan(6, 24, 8, 128, 800, dtype=2)[0] == 4
     # A paged call keeps a split's block numbers within LDS.
     assert plan(1, 16, 8, 128, 131072, page_size=1)[0] == 128
 
