@@ -34,12 +34,13 @@
 //    split's block numbers are staged in LDS (or, for splits touching more than kMaxSplitPages
 //    blocks, read from the table in global memory), clamped to the pool, and every lane computes
 //    the address of the row it loads. The keys and their order are the contiguous cache's, so the
-//    results are bitwise the same.
+//    results are bitwise the same for the same split count, or the same lengths, capacity and workgroups of
+//    a balanced call. (Where no count is asked for, the two layouts can be planned differently.)
 //  * At the end the four waves are merged in order through LDS (one KV head; with four, each wave's
 //    state is its own head's and is written as it is), and the workgroup writes o and lse
 //    (one split) or its unnormalized partial output and (reference point, sum), which decode.hip's
 //    merge pass combines as it would (max, sum). No atomics: results are bitwise reproducible for a
-//    given split count.
+//    given split count, and a balanced call's for the same lengths of all sequences and workgroups.
 #include "decode_sched.hpp"
 #include "gfx950.hpp"
 #include "launch.hpp"

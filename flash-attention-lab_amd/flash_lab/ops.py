@@ -225,7 +225,9 @@ def decode(
 
     The cache is [B, S_max, H_kv, D], or [num_blocks, page_size, H_kv, D] with block_tables.
     seq_lens values are not checked on the host (that would force a device sync).
-    num_splits=None lets the library choose how many workgroups share one sequence's keys.
+    num_splits=None lets the library choose how many workgroups share one sequence's keys; a large
+    paged batch then shares all sequences' keys evenly, so a sequence's last bits can depend on the
+    other lengths of the batch and on the cache's layout. A num_splits of one's own pins them.
     """
     q3, shape = check_decode_inputs(q, k_cache, v_cache, seq_lens, block_tables)
     scale = 1.0 / math.sqrt(shape.head_dim) if softmax_scale is None else softmax_scale

@@ -85,8 +85,8 @@ int fl_attention_plan(const fl_attn_params* p, int32_t requested_splits, int32_t
  * fl_attention_fwd with num_splits key splits, resolved by fl_attention_plan, or 0: the count that
  * fl_attention_plan would choose for cu_count. If that count needs a larger workspace than given,
  * nothing is launched and the call returns FL_ERR_WORKSPACE, so that a caller can try without one
- * (most calls need none) and allocate it only when asked to. workspace is 16-byte aligned fp32 device memory of at least the size fl_attention_plan
- * reports for that count (unused, may be NULL, when num_splits == 1). The splits are merged in a
+ * (most calls need none) and allocate it only when asked to. workspace is 16-byte aligned fp32
+ * device memory of at least the size fl_attention_plan reports for that count (unused, may be NULL, when num_splits == 1). The splits are merged in a
  * fixed order: results are bitwise reproducible for a given split count.
  */
 int fl_attention_fwd_split(const fl_attn_params* p, int32_t num_splits, int32_t cu_count,
